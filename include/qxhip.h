@@ -116,7 +116,8 @@ qx_status qx_plan_update_tensor(qx_plan *plan, const char *key, const double *z,
  *                 workgroup; 0 (default) = one launch per level (may be set at any time;
  *                 the walk is latency-bound and slower on the plans measured so far)
  *   "kernel"      -1 (default) = heuristic kernel choice; 0 gather, 1 rows, 2-4
- *                 FP tile GEMMs, 5 / 7 matrix-core GEMM (K chunks of 16 / 32), 6 reduce,
+ *                 FP tile GEMMs, 5 / 7 matrix-core GEMM on any layout (result lanes along
+ *                 C's fastest leg / along the other operand's), 6 reduce,
  *                 8 rocBLAS strided-batched GEMM (steps whose operands are plain
  *                 column-major matrices), 9 skinny contraction (K >= 2^12, at most 32
  *                 output values per batch element, N <= 2), 10 rocBLAS on gathered

@@ -10,6 +10,7 @@
 // every bitstring-dependent tensor, guarantees it for batched steps).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 
@@ -386,193 +387,214 @@ __global__ __launch_bounds__(256) void k_mfma_probe(T *out, int iters, T seed) {
 }
 
 // ---------------------------------------------------------------------------
-// Complex GEMM on 16x16x4 matrix cores (FP32 for complex64, FP64 for complex128),
-// same bit-weight tile gathers as k_contract_gemm.  A 64x64 complex C tile per
-// workgroup, 4 waves of 32x32 (2x2 blocks of 16x16).  4M: Re += Ar.Br - Ai.Bi and
-// Im += Ar.Bi + Ai.Br as four real products per block; 3M (Gauss, complex64 only):
-// RR = Ar.Br, II = Ai.Bi, SS = (Ar+Ai).(Br+Bi), Re = RR - II, Im = SS - RR - II.
-// Accumulation in the operand precision.  Operand and result layouts as in Mfma16.
-template <typename T, bool GAUSS, int TK>
-__global__ __launch_bounds__(256) void k_contract_gemm_mfma(const typename Vec<T>::type *__restrict__ A,
-                                                            const typename Vec<T>::type *__restrict__ B,
-                                                            typename Vec<T>::type *__restrict__ C, GemmArgs a) {
+// Complex GEMM on 16x16x4 matrix cores (FP32 for complex64, FP64 for complex128) on
+// operands of any layout: X (M x K), Y (K x N) and C, each index a set of bits with a
+// stride per operand.  A workgroup of four waves (WGM along M) owns a tile of
+// TM = 16 WGM BI rows and TN = 16 (4 / WGM) BJ columns, K stages of TK values.
+//
+// Addresses: a tile's elements are numbered by their bits in the operand's own stride
+// order, low 8 bits the lane, the rest the lane's registers, so loads run along the
+// operand whatever leg comes first; an element's LDS slot is the same bits' sum in
+// [k][m] / [k][n] order (a tile with fewer elements than lanes has zero weights beyond
+// them: those lanes load and store a copy of the same element).  Every offset that is not
+// the lane's own is wave-uniform: stage and unit offsets advance by one table entry (the
+// entry of the lowest set bit of the next index is its stride less those of the bits that
+// turn to zero).  The lowering picks the tile's bits so that each operand's and C's
+// 128-byte lines are read and written whole, and numbers rows and columns in C order
+// (MFMA result lanes run along C's fastest legs; results are stored from registers).
+//
+// Bound: matrix cores where K is long, HBM where K <= 32.  A lone workgroup would wait
+// for its own first loads, so the next stage -- at a unit's end the next unit's first --
+// is fetched into registers during the products.  Units are numbered in C order and each
+// XCD runs one contiguous range of them, its workgroups side by side (a workgroup's own
+// units are a grid stride apart): panels, and lines of C that two units share (a hyper
+// leg among its lowest), meet in one L2 at one time.  Consecutive units per workgroup
+// were 10-27% slower on the K <= 8 steps.
+//
+// 4M: Re += Xr.Yr - Xi.Yi, Im += Xr.Yi + Xi.Yr; 3M (Gauss, complex64 only): RR = Xr.Yr,
+// II = Xi.Yi, SS = (Xr+Xi).(Yr+Yi), Re = RR - II, Im = SS - RR - II.  Accumulation in
+// the operand precision.  Operand and result layouts as in Mfma16.
+template <typename T, bool GAUSS, int WGM, int BI, int BJ, int TK>
+__global__ __launch_bounds__(256, 3) void k_contract_gemm_mfma(const typename Vec<T>::type *__restrict__ X,
+                                                            const typename Vec<T>::type *__restrict__ Y,
+                                                            typename Vec<T>::type *__restrict__ C, MfmaArgs a) {
   using V = typename Vec<T>::type;
   using M = Mfma16<T>;
-  using f32x4 = typename M::v4;
-  constexpr int TM = 64, TN = 64;
-  constexpr int PA = TM + 1, PB = TN + 1, PC = TN + 1;
-  constexpr int LDS_AB = TK * (PA + PB), LDS_C = TM * PC;
-  constexpr int LDS = LDS_AB > LDS_C ? LDS_AB : LDS_C;
-  constexpr int EA = TM * TK / 256, EB = TN * TK / 256;
-  __shared__ V lds[LDS];
-  __shared__ int64_t t_am[TM], t_cm[TM], t_bn[TN], t_cn[TN], t_ak[TK], t_bk[TK];
-  V *sA = lds;
-  V *sB = lds + TK * PA;
+  using v4 = typename M::v4;
+  constexpr int TM = 16 * WGM * BI, TN = 16 * (4 / WGM) * BJ;
+  constexpr int PA = mfma_pitch(TM, sizeof(V)), PB = mfma_pitch(TN, sizeof(V));
+  constexpr int EA = TM * TK > 256 ? TM * TK / 256 : 1, EB = TN * TK > 256 ? TN * TK / 256 : 1;
+  __shared__ V sA[TK * PA];
+  __shared__ V sB[TK * PB];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int lm = 6, ln = 6, lk = TK == 16 ? 4 : 5;
-  const int rows = a.nbm < lm ? (1 << a.nbm) : TM;
-  const int cols = a.nbn < ln ? (1 << a.nbn) : TN;
-  const int kk = a.nbk < lk ? (1 << a.nbk) : TK;
-  const int64_t tiles_m = a.nbm > lm ? (int64_t(1) << (a.nbm - lm)) : 1;
-  const int64_t tiles_n = a.nbn > ln ? (int64_t(1) << (a.nbn - ln)) : 1;
-  const int64_t chunks_all = a.nbk > lk ? (int64_t(1) << (a.nbk - lk)) : 1;
-  const int64_t chunks = chunks_all / a.ksplit;
-  const int64_t ntiles = tiles_m * tiles_n * (int64_t(1) << a.nbh) * a.ksplit;
-  for (int i = tid; i < TM; i += 256) {
-    int64_t oa = 0, oc = 0;
-    for (int b = 0; b < lm && b < a.nbm; ++b)
-      if ((i >> b) & 1) oa += a.ma[b], oc += a.mc[b];
-    t_am[i] = oa;
-    t_cm[i] = oc;
+  const int wm = wave % WGM, wn = wave / WGM;
+  const int li = lane & 15, lq = lane >> 4;
+  if (a.partial) {   // rows, columns or k values missing from the tile stay zero
+    for (int i = tid; i < TK * PA; i += 256) sA[i] = V{0, 0};
+    for (int i = tid; i < TK * PB; i += 256) sB[i] = V{0, 0};
   }
-  for (int j = tid; j < TN; j += 256) {
-    int64_t ob = 0, oc = 0;
-    for (int b = 0; b < ln && b < a.nbn; ++b)
-      if ((j >> b) & 1) ob += a.nb[b], oc += a.nc[b];
-    t_bn[j] = ob;
-    t_cn[j] = oc;
+  // the lane's part of its elements' offsets, slots and result address
+  int64_t lx = 0, ly = 0, lc = 0;
+  int slx = 0, sly = 0;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const bool on = (tid >> b) & 1;
+    if (on) lx += a.xw[b], slx += a.xs[b], ly += a.yw[b], sly += a.ys[b];
   }
-  for (int l = tid; l < TK; l += 256) {
-    int64_t oa = 0, ob = 0;
-    for (int b = 0; b < lk && b < a.nbk; ++b)
-      if ((l >> b) & 1) oa += a.ka[b], ob += a.kb[b];
-    t_ak[l] = oa;
-    t_bk[l] = ob;
+  const int pm = wm * BI * 16 + M::row(lq, 0), pn = wn * BJ * 16 + li;   // the lane's first row and column
+#pragma unroll
+  for (int b = 0; b < 7; ++b) {
+    if ((pm >> b) & 1) lc += a.cm[b];
+    if ((pn >> b) & 1) lc += a.cn[b];
   }
-  __syncthreads();
-  int64_t offa[EA], offb[EB];
-  int slota[EA], slotb[EB];
-  bool oka[EA], okb[EB];
+  const bool okc = (pm & ~a.mmask) == 0 && (pn & ~a.nmask) == 0;
+  int64_t rox[EA], roy[EB];
+  int rsx[EA], rsy[EB];
 #pragma unroll
   for (int j = 0; j < EA; ++j) {
-    int e = tid + 256 * j, i, l;
-    if (a.a_kfast) i = e / TK, l = e % TK;
-    else l = e / TM, i = e % TM;
-    oka[j] = i < rows && l < kk;
-    offa[j] = oka[j] ? t_am[i] + t_ak[l] : 0;
-    slota[j] = l * PA + i;
+    rox[j] = 0, rsx[j] = 0;
+#pragma unroll
+    for (int b = 0; (1 << b) < EA; ++b)
+      if ((j >> b) & 1) rox[j] += a.xw[8 + b], rsx[j] += a.xs[8 + b];
   }
 #pragma unroll
   for (int j = 0; j < EB; ++j) {
-    int e = tid + 256 * j, jj, l;
-    if (a.b_kfast) jj = e / TK, l = e % TK;
-    else l = e / TN, jj = e % TN;
-    okb[j] = jj < cols && l < kk;
-    offb[j] = okb[j] ? t_bn[jj] + t_bk[l] : 0;
-    slotb[j] = l * PB + jj;
+    roy[j] = 0, rsy[j] = 0;
+#pragma unroll
+    for (int b = 0; (1 << b) < EB; ++b)
+      if ((j >> b) & 1) roy[j] += a.yw[8 + b], rsy[j] += a.ys[8 + b];
   }
-  const int64_t nblk = gridDim.x;
-  int64_t bid = blockIdx.x;
-  if (nblk % 8 == 0) bid = (bid % 8) * (nblk / 8) + bid / 8;
-  const int64_t per = (ntiles + nblk - 1) / nblk;
-  const int64_t t_begin = bid * per;
-  const int64_t t_end = t_begin + per < ntiles ? t_begin + per : ntiles;
-  const int64_t items = t_begin < t_end ? (t_end - t_begin) * chunks : 0;
-  auto tile_offsets = [&](int64_t unit, int64_t &oa, int64_t &ob, int64_t &oc) {
-    const int64_t split = unit % a.ksplit;
-    const int64_t tile = unit / a.ksplit;
-    int64_t nt = tile % tiles_n;
-    int64_t rest = tile / tiles_n;
-    int64_t mt = rest % tiles_m;
-    int64_t h = rest / tiles_m;
-    oa = 0, ob = 0, oc = 0;
-    for (int b = 0; b < a.nbh; ++b)
-      if ((h >> b) & 1) oa += a.ha[b], ob += a.hb[b], oc += a.hc[b];
-    for (int b = lm; b < a.nbm; ++b)
-      if (((mt << lm) >> b) & 1) oa += a.ma[b], oc += a.mc[b];
-    for (int b = ln; b < a.nbn; ++b)
-      if (((nt << ln) >> b) & 1) ob += a.nb[b], oc += a.nc[b];
-    oc += split * a.c_elems;
-  };
+  // units of this workgroup: a grid stride apart within its XCD's contiguous run
+  const uint32_t nwg = gridDim.x;
+  const int tb = a.trip_at, nu = 1 << a.trip_bits;
+  const int64_t u = nwg >= 8 ? (((int64_t)(blockIdx.x % 8) * (nwg / 8)) << a.trip_bits) + blockIdx.x / 8 : blockIdx.x;
+  int64_t ox = 0, oy = 0, oc = 0;
+  for (int b = 0; b < a.nub; ++b)   // the first unit: its trip bits are zero
+    if ((u >> b) & 1) ox += a.ux[b], oy += a.uy[b], oc += a.uc[b];
+  const int nst = 1 << a.nsb;
   V ra[EA], rb[EB];
-  auto fetch = [&](int64_t item) {
-    int64_t unit = t_begin + item / chunks, oa, ob, oc;
-    int64_t kc = (unit % a.ksplit) * chunks + item % chunks;
-    tile_offsets(unit, oa, ob, oc);
-    for (int b = lk; b < a.nbk; ++b)
-      if (((kc << lk) >> b) & 1) oa += a.ka[b], ob += a.kb[b];
+  auto fetch = [&](int64_t fx, int64_t fy) {
+    const V *xp = X + (fx + lx);
+    const V *yp = Y + (fy + ly);
 #pragma unroll
-    for (int j = 0; j < EA; ++j) ra[j] = oka[j] ? A[oa + offa[j]] : V{0, 0};
+    for (int j = 0; j < EA; ++j)
+      ra[j] = xp[rox[j]];
 #pragma unroll
-    for (int j = 0; j < EB; ++j) rb[j] = okb[j] ? B[ob + offb[j]] : V{0, 0};
+    for (int j = 0; j < EB; ++j)
+      rb[j] = yp[roy[j]];
   };
-  // wave (wm, wn) owns rows 32*wm.., cols 32*wn..; block (bi, bj) of 16x16
-  const int wm = wave & 1, wn = wave >> 1;
-  const int li = lane & 15, lq = lane >> 4;
-  f32x4 acc_rr[2][2], acc_ii[2][2], acc_x[2][2];
-  if (items > 0) fetch(0);
-  for (int64_t it = 0; it < items; ++it) {
-    const int64_t kc = it % chunks;
-    if (kc == 0) {
+  v4 acc0[BI][BJ], acc1[BI][BJ], acc2[BI][BJ];   // 4M: Re, Im; 3M: RR, II, SS
+  // the tile's products of four k values
+  auto products = [&](int kc) {
+            V fa[BI], fb[BJ];
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
+            for (int i = 0; i < BI; ++i) fa[i] = sA[(kc + lq) * PA + 16 * (BI * wm + i) + li];
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj) {
-          acc_rr[bi][bj] = f32x4{0, 0, 0, 0};
-          acc_ii[bi][bj] = f32x4{0, 0, 0, 0};
-          acc_x[bi][bj] = f32x4{0, 0, 0, 0};
-        }
-    }
-    __syncthreads();
+            for (int j = 0; j < BJ; ++j) fb[j] = sB[(kc + lq) * PB + 16 * (BJ * wn + j) + li];
+            if (GAUSS) {
+              T fs[BI], gs[BJ];
 #pragma unroll
-    for (int j = 0; j < EA; ++j) {
-      V v = ra[j];
-      if (a.conj_a) v.y = -v.y;
-      sA[slota[j]] = v;
-    }
+              for (int i = 0; i < BI; ++i) fs[i] = fa[i].x + fa[i].y;
 #pragma unroll
-    for (int j = 0; j < EB; ++j) {
-      V v = rb[j];
-      if (a.conj_b) v.y = -v.y;
-      sB[slotb[j]] = v;
-    }
-    __syncthreads();
-    if (it + 1 < items) fetch(it + 1);
+              for (int j = 0; j < BJ; ++j) gs[j] = fb[j].x + fb[j].y;
 #pragma unroll
-    for (int k0 = 0; k0 < TK; k0 += 4) {
-      V fa[2], fb[2];
+              for (int i = 0; i < BI; ++i)
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi) fa[bi] = sA[(k0 + lq) * PA + 32 * wm + 16 * bi + li];
+                for (int j = 0; j < BJ; ++j) {
+                  acc0[i][j] = M::mma(fa[i].x, fb[j].x, acc0[i][j]);
+                  acc1[i][j] = M::mma(fa[i].y, fb[j].y, acc1[i][j]);
+                  acc2[i][j] = M::mma(fs[i], gs[j], acc2[i][j]);
+                }
+            } else {
 #pragma unroll
-      for (int bj = 0; bj < 2; ++bj) fb[bj] = sB[(k0 + lq) * PB + 32 * wn + 16 * bj + li];
+              for (int i = 0; i < BI; ++i) {
+                const T nai = -fa[i].y;
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
+                for (int j = 0; j < BJ; ++j) {
+                  acc0[i][j] = M::mma(fa[i].x, fb[j].x, acc0[i][j]);
+                  acc1[i][j] = M::mma(fa[i].x, fb[j].y, acc1[i][j]);
+                }
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj) {
-          acc_rr[bi][bj] = M::mma(fa[bi].x, fb[bj].x, acc_rr[bi][bj]);
-          acc_ii[bi][bj] = M::mma(fa[bi].y, fb[bj].y, acc_ii[bi][bj]);
-          if (GAUSS) {
-            acc_x[bi][bj] = M::mma(fa[bi].x + fa[bi].y, fb[bj].x + fb[bj].y, acc_x[bi][bj]);
-          } else {
-            acc_x[bi][bj] = M::mma(fa[bi].x, fb[bj].y, acc_x[bi][bj]);
-            acc_x[bi][bj] = M::mma(fa[bi].y, fb[bj].x, acc_x[bi][bj]);
-          }
-        }
-    }
-    if (kc == chunks - 1) {
-      int64_t oa, ob, oc;
-      tile_offsets(t_begin + it / chunks, oa, ob, oc);
+                for (int j = 0; j < BJ; ++j) {
+                  acc0[i][j] = M::mma(nai, fb[j].y, acc0[i][j]);
+                  acc1[i][j] = M::mma(fa[i].y, fb[j].x, acc1[i][j]);
+                }
+              }
+            }
+  };
+  int64_t fx = ox, fy = oy;   // offsets of the stage fetched last
+  fetch(fx, fy);
+  for (int t = 0; t < nu; ++t) {
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+        acc0[i][j] = v4{0, 0, 0, 0}, acc1[i][j] = v4{0, 0, 0, 0}, acc2[i][j] = v4{0, 0, 0, 0};
+    for (int sg = 0; sg < nst; ++sg) {
       __syncthreads();
-      V *sC = lds;
 #pragma unroll
-      for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int i = 32 * wm + 16 * bi + M::row(lq, r), j = 32 * wn + 16 * bj + li;
-            const T rr = acc_rr[bi][bj][r], ii = acc_ii[bi][bj][r], x = acc_x[bi][bj][r];
-            sC[i * PC + j] = GAUSS ? V{rr - ii, x - rr - ii} : V{rr - ii, x};
-          }
-      __syncthreads();
-      V *Cb = C + oc;
-      for (int e = tid; e < TM * TN; e += 256) {
-        int i, j;
-        if (a.c_nfast) i = e / TN, j = e % TN;
-        else j = e / TM, i = e % TM;
-        if (i < rows && j < cols) Cb[t_cm[i] + t_cn[j]] = sC[i * PC + j];
+      for (int j = 0; j < EA; ++j) {
+        V v = ra[j];
+        if (a.conj_x) v.y = -v.y;
+        sA[slx + rsx[j]] = v;
       }
+#pragma unroll
+      for (int j = 0; j < EB; ++j) {
+        V v = rb[j];
+        if (a.conj_y) v.y = -v.y;
+        sB[sly + rsy[j]] = v;
+      }
+      __syncthreads();
+      // the next stage of this unit, or the first of the next unit (one fetch in the code:
+      // with two, or with loads under conditions of their own, the compiler waits for them
+      // where their paths meet, before the products)
+      const bool in_unit = sg + 1 < nst;
+      if (in_unit) {
+        const int z = __ffs(sg + 1) - 1;
+        fx += a.sx[z], fy += a.sy[z];
+      } else if (t + 1 < nu) {
+        const int z = __ffs(t + 1) - 1 + tb;
+        ox += a.ux[z], oy += a.uy[z];
+        fx = ox, fy = oy;
+      }
+      if (in_unit || t + 1 < nu) fetch(fx, fy);
+#pragma unroll
+      for (int kc = 0; kc < TK; kc += 4) products(kc);
     }
+    // results from registers: the lane's part of the address, the rest wave-uniform (formed
+    // here per unit: hoisted out of the unit loop, the sixteen offsets overflow the scalar
+    // registers)
+    int64_t wr[7], wc[7];
+#pragma unroll
+    for (int b = 0; b < 7; ++b) {
+      wr[b] = a.cm[b], wc[b] = a.cn[b];
+      asm volatile("" : "+s"(wr[b]), "+s"(wc[b]));
+    }
+    V *dst = C + (oc + lc);
+#pragma unroll
+    for (int i = 0; i < BI; ++i)
+#pragma unroll
+      for (int j = 0; j < BJ; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int rm = 16 * i + M::row(0, e), rn = 16 * j;   // row and column beyond the lane's first
+          int64_t o = 0;
+#pragma unroll
+          for (int b = 0; b < 7; ++b) {
+            if ((rm >> b) & 1) o += wr[b];
+            if ((rn >> b) & 1) o += wc[b];
+          }
+          V v;
+          if (GAUSS) {
+            v.x = acc0[i][j][e] - acc1[i][j][e];
+            v.y = acc2[i][j][e] - acc0[i][j][e] - acc1[i][j][e];
+          } else {
+            v.x = acc0[i][j][e];
+            v.y = acc1[i][j][e];
+          }
+          if (okc && (rm & ~a.mmask) == 0 && (rn & ~a.nmask) == 0) dst[o] = v;
+        }
+    if (t + 1 < nu) oc += a.uc[__ffs(t + 1) - 1 + tb];
   }
 }
 
@@ -1159,29 +1181,88 @@ void launch_contract_rows(int prec, const void *A, const void *B, void *C, const
 
 namespace {
 
+template <typename T, bool GAUSS>
+void mfma_launch(const void *X, const void *Y, void *C, const MfmaArgs &a, int g, hipStream_t s) {
+  using V = typename Vec<T>::type;
+  // Steps of one stage stream C: unused LDS holds the resident workgroups down to about
+  // 96 KiB of results per CU, 3 MiB per XCD, so that lines of C which several units write
+  // parts of are whole when they leave its 4 MiB L2.  On the 7x7 workload's M 16, N 2^17,
+  // K 4, 512-fold step: complex128 6.3 -> 4.0 ms, complex64 3.2 -> 2.8 ms.
+  size_t pad = 0;
+  if (a.nsb == 0) {
+    const int tm = kMfmaTiles[a.cfg][0], tn = kMfmaTiles[a.cfg][1], es = (int)sizeof(V);
+    const int wgs = std::max(2, (96 << 10) / (tm * tn * es));
+    const int used = a.kk * (mfma_pitch(tm, es) + mfma_pitch(tn, es)) * es;
+    pad = (size_t)std::max(0, (160 << 10) / wgs - used - 1024);
+  }
+#define QX_MFMA(WGM, BI, BJ)                                                                                      \
+  if (a.kk == 16)                                                                                                 \
+    hipLaunchKernelGGL((k_contract_gemm_mfma<T, GAUSS, WGM, BI, BJ, 16>), dim3(g), dim3(256), pad, s, (const V *)X, \
+                       (const V *)Y, (V *)C, a);                                                                  \
+  else if (a.kk == 8)                                                                                             \
+    hipLaunchKernelGGL((k_contract_gemm_mfma<T, GAUSS, WGM, BI, BJ, 8>), dim3(g), dim3(256), pad, s, (const V *)X,  \
+                       (const V *)Y, (V *)C, a);                                                                  \
+  else                                                                                                            \
+    hipLaunchKernelGGL((k_contract_gemm_mfma<T, GAUSS, WGM, BI, BJ, 4>), dim3(g), dim3(256), pad, s, (const V *)X,  \
+                       (const V *)Y, (V *)C, a)
+  switch (a.cfg) {   // rows x columns of kMfmaTiles
+    case 0: QX_MFMA(2, 2, 2); break;
+    case 1: QX_MFMA(2, 1, 2); break;
+    case 2: QX_MFMA(2, 2, 1); break;
+    case 3: QX_MFMA(1, 1, 2); break;
+    case 4: QX_MFMA(4, 2, 1); break;
+    default: throw Error(QX_ERR_STATE, "internal: matrix-core tile");
+  }
+#undef QX_MFMA
+}
+
 }  // namespace
+
+// One unit per workgroup (units then start in C order as others end); K = 64 (four
+// stages) takes two, whose second first loads run during the first's products (7x7,
+// M 64, N 2048, 1024-fold, complex128: 1.30 -> 1.21 ms; longer K hides its first loads by
+// itself, shorter K lost 3-25% with two or more).
+void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &a, void *stream) {
+  hipStream_t s = (hipStream_t)stream;
+  const void *X = a.swap ? B : A, *Y = a.swap ? A : B;
+  void *dst = a.ksplit > 1 ? ws : C;
+  const int q = a.nsb == 2 && a.nub > 12 ? 1 : 0;
+  if (a.nub - q > 30) throw Error(QX_ERR_STATE, "internal: matrix-core GEMM grid");
+  const int g = 1 << (a.nub - q);
+  MfmaArgs b = a;   // strides -> increments: of the stages, and of the unit bits a trip counter walks
+  auto increments = [](int64_t *w, int n) {
+    int64_t below = 0;
+    for (int i = 0; i < n; ++i) {
+      const int64_t d = w[i] - below;
+      below += w[i];
+      w[i] = d;
+    }
+  };
+  b.trip_bits = q;
+  b.trip_at = a.nub - q - (g >= 8 ? 3 : 0);   // below the XCD's bits
+  increments(b.sx, b.nsb), increments(b.sy, b.nsb);
+  for (int64_t *w : {b.ux, b.uy, b.uc}) increments(w + b.trip_at, q);
+  if (prec == QX_C128) mfma_launch<double, false>(X, Y, dst, b, g, s);
+  else if (prec == QX_C64_3M) mfma_launch<float, true>(X, Y, dst, b, g, s);
+  else mfma_launch<float, false>(X, Y, dst, b, g, s);
+  check_launch("contract_gemm_mfma");
+  if (a.ksplit > 1) {
+    const int gs = grid_for(a.c_elems, 256);
+    if (prec == QX_C128)
+      hipLaunchKernelGGL(k_sum_splits<double>, dim3(gs), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, a.c_elems,
+                         a.ksplit);
+    else
+      hipLaunchKernelGGL(k_sum_splits<float>, dim3(gs), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, a.c_elems,
+                         a.ksplit);
+    check_launch("sum_splits");
+  }
+}
 
 void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void *ws, const GemmArgs &args,
                           void *stream) {
   hipStream_t s = (hipStream_t)stream;
   void *dst = args.ksplit > 1 ? ws : C;
-  if (args.tile >= 3) {   // matrix cores, 64x64 tiles, K chunks of 16 (tile 3) or 32 (tile 4)
-    int64_t tiles = (args.nbm > 6 ? (int64_t(1) << (args.nbm - 6)) : 1) *
-                    (args.nbn > 6 ? (int64_t(1) << (args.nbn - 6)) : 1) * (int64_t(1) << args.nbh) * args.ksplit;
-    int g = (int)(tiles < 1024 ? tiles : 1024);
-#define QX_MFMA_GEMM(TT, V2, GA, TKK)                                                                   \
-  hipLaunchKernelGGL((k_contract_gemm_mfma<TT, GA, TKK>), dim3(g), dim3(256), 0, s, (const V2 *)A, \
-                     (const V2 *)B, (V2 *)dst, args)
-    const bool k32 = args.tile == 4;
-    if (prec == QX_C128) {
-      if (k32) QX_MFMA_GEMM(double, double2, false, 32); else QX_MFMA_GEMM(double, double2, false, 16);
-    } else if (prec == QX_C64_3M) {
-      if (k32) QX_MFMA_GEMM(float, float2, true, 32); else QX_MFMA_GEMM(float, float2, true, 16);
-    } else {
-      if (k32) QX_MFMA_GEMM(float, float2, false, 32); else QX_MFMA_GEMM(float, float2, false, 16);
-    }
-#undef QX_MFMA_GEMM
-  } else switch (args.tile) {
+  switch (args.tile) {
     case 0: gemm_launch<128, 16, 16>(prec, A, B, dst, args, s); break;
     case 1: gemm_launch<128, 32, 16>(prec, A, B, dst, args, s); break;
     default: gemm_launch<64, 64, 16>(prec, A, B, dst, args, s); break;

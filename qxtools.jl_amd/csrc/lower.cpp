@@ -167,7 +167,7 @@ static void check_bounds(const Program &p, const Lowered &L, const std::vector<i
 }
 
 // Kernel configurations a power-of-two step can run with.
-enum Choice { kBits = 0, kRows = 1, kGemm0 = 2, kGemm1 = 3, kGemm2 = 4, kMfma = 5, kReduce = 6, kMfma32 = 7,
+enum Choice { kBits = 0, kRows = 1, kGemm0 = 2, kGemm1 = 3, kGemm2 = 4, kMfma = 5, kReduce = 6, kMfmaT = 7,
               kBlas = 8, kSkinny = 9, kTtgt = 10, kPlain = 11, kPlain3 = 12, kNumChoices = 13 };
 
 // K split of the hand-written plain GEMM: enough work units to give every CU two
@@ -291,6 +291,122 @@ bool plain_gemm(const Step &st, BlasArgs &b) {
   b.opx = opx, b.opy = opy, b.ldx = ldx, b.ldy = ldy, b.k = K, b.sc = hc;
   const int64_t lim = int64_t(1) << 31;   // rocblas_int sizes and leading dimensions
   return b.r < lim && b.s < lim && b.k < lim && b.ldx < lim && b.ldy < lim && b.ldc < lim && b.batch < lim;
+}
+// Arguments of the matrix-core GEMM on operands of any layout.  The operand that holds
+// the lowest of C's M and N bits becomes Y (C's columns, which the result lanes walk;
+// `other`: the other one), the tile is 64 x 64 or, where a side has fewer values, the
+// narrower shape that wastes least.  Tile bits: first those below a 128-byte line of X, Y
+// and C (lowest first, so each line is read and written by one workgroup), then each
+// operand's next smallest strides.
+bool mfma_args(const StepBits &sb, int precision, bool other, int64_t c_elems, MfmaArgs &g) {
+  const int line_bits = precision == QX_C128 ? 3 : 4;
+  struct Bit {
+    int64_t x, y, c;
+    char cls;       // X only (M), Y only (N), both and contracted (K), all (H)
+    bool in_tile;
+  };
+  int64_t low_m = INT64_MAX, low_n = INT64_MAX;
+  for (auto &c : sb.mb) low_m = std::min(low_m, c.wc);
+  for (auto &c : sb.nbits) low_n = std::min(low_n, c.wc);
+  g.other = other;
+  g.swap = (low_m < low_n) != other;
+  std::vector<Bit> bits;
+  for (auto &c : sb.cbits) {
+    const int64_t x = g.swap ? c.wb : c.wa, y = g.swap ? c.wa : c.wb;
+    bits.push_back({x, y, c.wc, x && y ? 'H' : x ? 'M' : 'N', false});
+  }
+  for (auto &k : sb.kbits)
+    bits.push_back({g.swap ? k.second : k.first, g.swap ? k.first : k.second, 0, 'K', false});
+  auto count = [&](char cls) { return (int)std::count_if(bits.begin(), bits.end(), [&](const Bit &b) { return b.cls == cls; }); };
+  const int nm = count('M'), nn = count('N'), nk = count('K');
+  // tile shape
+  if (nm >= 6 && nn >= 6) g.cfg = 0;
+  else if (nm <= 4 && nm <= nn) g.cfg = 3;
+  else if (nn <= 4) g.cfg = 4;
+  else g.cfg = nm <= nn ? 1 : 2;
+  int cap[3] = {ilog2(kMfmaTiles[g.cfg][0]), ilog2(kMfmaTiles[g.cfg][1]), kMfmaStageBits};
+  int used[3] = {0, 0, 0};
+  auto slot = [](char cls) { return cls == 'M' ? 0 : cls == 'N' ? 1 : cls == 'K' ? 2 : -1; };
+  auto take = [&](Bit &b) {
+    const int s = slot(b.cls);
+    if (s < 0 || b.in_tile || used[s] == cap[s]) return;
+    b.in_tile = true;
+    ++used[s];
+  };
+  for (int l = 0; l < line_bits; ++l)
+    for (int o = 0; o < 3; ++o)
+      for (Bit &b : bits)
+        if ((o == 0 ? b.x : o == 1 ? b.y : b.c) == int64_t(1) << l) take(b);
+  auto fill = [&](char cls, auto key) {
+    std::vector<Bit *> v;
+    for (Bit &b : bits)
+      if (b.cls == cls) v.push_back(&b);
+    std::stable_sort(v.begin(), v.end(), [&](Bit *p, Bit *q) { return key(*p) < key(*q); });
+    for (Bit *b : v) take(*b);
+  };
+  fill('M', [](const Bit &b) { return b.x; });
+  fill('N', [](const Bit &b) { return b.y; });
+  fill('K', [](const Bit &b) { return std::min(b.x, b.y); });
+  g.kk = std::max(4, 1 << used[2]);
+  g.partial = used[0] < cap[0] || used[1] < cap[1] || used[2] < 2;
+  // row and column index bits in C order: for FP32 the lanes hold row bits 2-3 of a
+  // 16-row block and the registers bits 0-1, for FP64 the other way round
+  static const int rows32[7] = {2, 3, 0, 1, 4, 5, 6};
+  const int pa = mfma_pitch(kMfmaTiles[g.cfg][0], precision == QX_C128 ? 16 : 8);
+  const int pb = mfma_pitch(kMfmaTiles[g.cfg][1], precision == QX_C128 ? 16 : 8);
+  struct Elem {
+    int64_t w;
+    int32_t slot;
+  };
+  std::vector<Elem> ex, ey;
+  std::vector<Bit *> tile, rest;
+  for (Bit &b : bits) (b.in_tile ? tile : rest).push_back(&b);
+  std::stable_sort(tile.begin(), tile.end(), [](Bit *p, Bit *q) { return p->c < q->c; });
+  int im = 0, in = 0, ik = 0;
+  for (Bit *b : tile) {
+    if (b->cls == 'M') {
+      const int p = precision == QX_C128 ? im : rows32[im];
+      ++im;
+      g.cm[p] = b->c;
+      g.mmask |= 1 << p;
+      ex.push_back({b->x, 1 << p});
+    } else if (b->cls == 'N') {
+      g.cn[in] = b->c;
+      g.nmask |= 1 << in;
+      ey.push_back({b->y, 1 << in});
+      ++in;
+    } else {
+      ex.push_back({b->x, pa << ik});
+      ey.push_back({b->y, pb << ik});
+      ++ik;
+    }
+  }
+  auto by_w = [](const Elem &p, const Elem &q) { return p.w < q.w; };
+  std::stable_sort(ex.begin(), ex.end(), by_w);
+  std::stable_sort(ey.begin(), ey.end(), by_w);
+  for (auto &e : ex) g.xw[g.nxb] = e.w, g.xs[g.nxb] = e.slot, ++g.nxb;
+  for (auto &e : ey) g.yw[g.nyb] = e.w, g.ys[g.nyb] = e.slot, ++g.nyb;
+  // units in C order; K: stages in X order, the largest strides split over workgroups
+  // where the tiles alone are fewer than 1024 (at least 8 stages per split)
+  std::vector<Bit *> kb;
+  for (Bit *b : rest)
+    if (b->cls == 'K') kb.push_back(b);
+  std::stable_sort(rest.begin(), rest.end(), [](Bit *p, Bit *q) { return p->c < q->c; });
+  std::stable_sort(kb.begin(), kb.end(), [](Bit *p, Bit *q) { return p->x < q->x; });
+  for (Bit *b : rest)
+    if (b->cls != 'K') g.ux[g.nub] = b->x, g.uy[g.nub] = b->y, g.uc[g.nub] = b->c, ++g.nub;
+  g.nsb = (int)kb.size();
+  g.c_elems = c_elems;
+  int split = 0;
+  while (g.nub + split < 10 && g.nsb - split > 3) ++split;
+  g.nsb -= split;
+  for (int i = 0; i < g.nsb; ++i) g.sx[i] = kb[i]->x, g.sy[i] = kb[i]->y;
+  for (int i = 0; i < split; ++i) {
+    if (g.nub >= kMaxBits) return false;
+    g.ux[g.nub] = kb[g.nsb + i]->x, g.uy[g.nub] = kb[g.nsb + i]->y, g.uc[g.nub] = c_elems << i, ++g.nub;
+  }
+  g.ksplit = 1 << split;
+  return g.nub <= 36;
 }
 }  // namespace
 
@@ -446,11 +562,21 @@ bool configure_kernel(Step &st, int precision, int choice) {
       }
       break;
     }
+    case kMfma:
+    case kMfmaT: {
+      st.kern = Kern::Gemm;
+      st.gemm = GemmArgs{};
+      st.gemm.tile = 3;
+      st.mfma = MfmaArgs{};
+      if (!mfma_args(sb, precision, choice == kMfmaT, st.c_elems, st.mfma)) return false;
+      st.mfma.conj_x = st.mfma.swap ? st.radix.conj_b : st.radix.conj_a;
+      st.mfma.conj_y = st.mfma.swap ? st.radix.conj_a : st.radix.conj_b;
+      st.ws_elems = st.mfma.ksplit > 1 ? st.mfma.ksplit * st.c_elems : 0;
+      return true;
+    }
     case kGemm0:
     case kGemm1:
-    case kGemm2:
-    case kMfma:
-    case kMfma32: {
+    case kGemm2: {
       st.kern = Kern::Gemm;
       GemmArgs &g = st.gemm;
       g = GemmArgs{};
@@ -468,8 +594,8 @@ bool configure_kernel(Step &st, int precision, int choice) {
       for (int i = 0; i < nm; ++i) g.ma[i] = mb[i].wa, g.mc[i] = mb[i].wc;
       for (int i = 0; i < nn; ++i) g.nb[i] = nbits[i].wb, g.nc[i] = nbits[i].wc;
       for (int i = 0; i < nk; ++i) g.ka[i] = kbits[i].first, g.kb[i] = kbits[i].second;
-      g.tile = choice == kMfma32 ? 4 : choice - kGemm0;
-      const int lm = g.tile >= 2 ? 6 : 7, ln = g.tile == 0 ? 4 : g.tile == 1 ? 5 : 6, lk = g.tile == 4 ? 5 : 4;
+      g.tile = choice - kGemm0;
+      const int lm = g.tile == 2 ? 6 : 7, ln = g.tile == 0 ? 4 : g.tile == 1 ? 5 : 6, lk = 4;
       auto min_w = [](const int64_t *w, int n) {
         int64_t m = INT64_MAX;
         for (int i = 0; i < n; ++i) m = std::min(m, w[i]);
@@ -495,26 +621,52 @@ bool configure_kernel(Step &st, int precision, int choice) {
   return true;
 }
 
+// Whether the matrix-core GEMM on any layout is the default of a step with at least 8
+// rows and columns and 2^18 multiply-adds.  complex64: always (6x6 workload, 256 strings,
+// H 4096, M 64, N 128, K 512: 1.28 ms, vector tiles 2.65; M 16, N 65536, K 8: 22 us,
+// gather kernel 117).  complex128: from 2^25 multiply-adds (7x7, H 128, M 256, N 16384,
+// K 256: 17.1 ms, vector tiles 33.5; H 512, M 16, N 131072, K 4: 4.0 ms, gather kernel
+// 10.6) or 16 batch elements (H 128, M 16, N 256, K 32: 12 us, gather kernel 54); the
+// few tiles of a smaller single product run as fast on the vector pipe, whose FP64 rate
+// is the same.
+bool mfma_default(const StepBits &sb, const Step &st, int precision) {
+  const double macs = (double)st.H * st.M * st.N * st.K;
+  if (std::min(sb.nm, sb.nn) < 3 || macs < double(1 << 18)) return false;
+  return precision != QX_C128 || sb.hb.size() >= 4 || macs >= double(1 << 25);
+}
+
 // The heuristic choice:
-//  * Rows   : >= 2^12 rows (H and M), K <= 16, N <= 64, C's fastest bit a row bit
+//  * Plain  : steps of >= 2^30 flops whose operands are plain matrices: the hand-written
+//             plain matrix-core GEMM (k_plain_gemm) where K > 256 (its larger complex64
+//             tiles pay with K: 5x5, M 4096, N 128, K 8192: 0.30 ms against 0.34); up to
+//             there the any-layout GEMM below (7x7, M 4096, N 512, K 64: 2.8 ms against
+//             3.3, complex128 4.7 against 5.3; 6x6, M 1024, N 128, K 128: 2.7 against
+//             2.9).  With QX_C64_BF16X3, plain steps with M, N, K >= 1024 as its split
+//             bf16 product
+//  * Rows   : >= 2^12 rows (H and M), K <= 16, N <= 64, C's fastest bit a row bit;
+//             where the any-layout GEMM is on offer only K <= 4 on >= 2^18 rows, which
+//             stream (6x6, 2^19 rows, N 64, K 4: 56 us against 97; 2^14 rows: 38 against
+//             11, too few lanes)
+//  * Mfma   : mfma_default
 //  * Gemm   : K >= 8, N >= 8, M >= 32 (bits of each class counted without H); complex64
 //             with N, M >= 64 on FP32 matrix cores
 //  * small C (<= 2^14) with K >= 256: lanes along K (Reduce) when a K bit is A's
 //    unit stride, else the gather kernel with K split over workgroups
 //  * Bits   : everything else with power-of-two dims
 //  * Radix  : any other dims
-//  * Plain  : steps of >= 2^30 flops whose operands are plain matrices: the
-//             hand-written matrix-core GEMM (k_plain_gemm); with QX_C64_BF16X3, plain
-//             steps with M, N, K >= 1024 as its split bf16 product
 //  * Blas   : the vendor BLAS, a tuned candidate only
 int default_choice(const Step &st, int precision) {
   const StepBits sb = step_bits(st);
   BlasArgs ba;
   if (precision == QX_C64_BF16X3 && plain_gemm(st, ba) && ba.r >= 1024 && ba.s >= 1024 && ba.k >= 1024)
     return kPlain;   // the split bf16 product
-  if (8.0 * st.H * st.M * st.N * st.K >= double(int64_t(1) << 30) && plain_gemm(st, ba)) return kPlain;
-  if (sb.nr >= 12 && sb.nk <= 4 && sb.nk + sb.nn >= 1 && !sb.cbits.empty() && sb.cbits[0].wa != 0 && rows_ok(sb))
+  const bool mfma = mfma_default(sb, st, precision);
+  if (8.0 * st.H * st.M * st.N * st.K >= double(int64_t(1) << 30) && plain_gemm(st, ba) && (!mfma || ba.k > 256))
+    return kPlain;
+  if (sb.nr >= 12 && sb.nk <= 4 && sb.nk + sb.nn >= 1 && !sb.cbits.empty() && sb.cbits[0].wa != 0 && rows_ok(sb) &&
+      (!mfma || (sb.nk <= 2 && sb.nr >= 18)))
     return kRows;
+  if (mfma) return kMfma;
   if (sb.nk >= 3 && sb.nn >= 3 && sb.nm >= 5) {
     if (precision != QX_C128 && sb.nn >= 6 && sb.nm >= 6) return kMfma;
     return sb.nn <= 4 ? kGemm0 : sb.nn == 5 ? kGemm1 : kGemm2;
@@ -606,8 +758,9 @@ std::vector<Step> kernel_candidates(const Step &st, int precision) {
   if (st.kern == Kern::Radix || st.kern == Kern::Outer) return out;
   const StepBits sb = step_bits(st);
   std::vector<int> alts;
-  if (sb.nk >= 2 && sb.nn >= 2 && sb.nm >= 4) alts.insert(alts.end(), {kGemm0, kGemm1, kGemm2, kMfma});
-  if (sb.nk >= 5 && sb.nn >= 4 && sb.nm >= 4) alts.push_back(kMfma32);
+  if (st.kern == Kern::Gemm || (sb.nk >= 2 && sb.nn >= 2 && sb.nm >= 4))
+    alts.insert(alts.end(), {kGemm0, kGemm1, kGemm2});
+  if (sb.nn >= 2 && sb.nm >= 2) alts.insert(alts.end(), {kMfma, kMfmaT});
   if (sb.nr >= 8 && rows_ok(sb)) alts.push_back(kRows);
   if (st.c_elems <= (int64_t(1) << 16) && sb.nk >= 6) alts.push_back(kReduce);
   if (sb.nk >= 12 && sb.nm + sb.nn <= 5 && sb.nn <= 1) alts.push_back(kSkinny);

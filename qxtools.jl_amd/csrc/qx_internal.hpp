@@ -224,6 +224,38 @@ struct GemmArgs {
   int64_t c_elems = 0;                        // dense C size: stride between K-split partials
 };
 
+// The matrix-core GEMM on operands of any layout (k_contract_gemm_mfma): X (M x K) and
+// Y (K x N) are A and B, or B and A (swap).  Tile bits: the rows and columns of a tile
+// and the k values of a stage, as the bits of an element's number in X's (Y's) own stride
+// order -- the low 8 the lane, the rest its registers -- each with its stride and its LDS
+// slot increment.  Unit bits (tiles, batch elements, K splits) in C order, stage bits in X
+// order.  cm / cn: C strides of the tile's row and column index bits.
+constexpr int kMfmaTiles[5][2] = {{64, 64}, {32, 64}, {64, 32}, {16, 128}, {128, 16}};   // rows, columns
+constexpr int kMfmaStageBits = 4;   // log2 of a stage's k values
+constexpr int kMfmaTileBits = 11;   // bits of a 128 x 16 stage
+// Elements between consecutive k of a tile in LDS: complex64 rows 136 bytes apart modulo
+// the banks (the two rows a read covers share none but two), complex128 rows 16 bytes
+// (a read covers one row; stores along k still spread).
+constexpr int mfma_pitch(int width, int elem_bytes) {
+  return elem_bytes == 16 ? width + 1 : width % 32 ? width + 1 : width + 17;
+}
+struct MfmaArgs {
+  int cfg = 0, swap = 0, other = 0;   // other: result lanes not along C's fastest leg
+  int partial = 0;                      // the tile has fewer rows, columns or k values
+  int conj_x = 0, conj_y = 0;
+  int nxb = 0, nyb = 0, kk = 0;         // tile bits of X and Y; k values of a stage
+  int nsb = 0, nub = 0, ksplit = 1;     // stage bits, unit bits (K splits the highest)
+  int trip_bits = 0, trip_at = 0;       // units of a workgroup: the values of these unit bits (set at launch)
+  int mmask = 0, nmask = 0;             // row / column index bits in use
+  int32_t xs[kMfmaTileBits] = {0}, ys[kMfmaTileBits] = {0};
+  int64_t xw[kMfmaTileBits] = {0}, yw[kMfmaTileBits] = {0};
+  int64_t cm[7] = {0}, cn[7] = {0};
+  int64_t sx[kMaxBits] = {0}, sy[kMaxBits] = {0};
+  int64_t ux[kMaxBits] = {0}, uy[kMaxBits] = {0}, uc[kMaxBits] = {0};
+  int64_t c_elems = 0;                  // dense C size: stride between K-split partials
+};
+static_assert(sizeof(MfmaArgs) <= 4000, "matrix-core GEMM arguments must fit the kernel argument segment");
+
 // One leg of a step in canonical form: dims and element strides in A, B and C.
 struct Leg {
   int64_t dim;
@@ -292,6 +324,7 @@ struct Step {
   bool swapped = false;    // operands exchanged (in_a is the DSL's B): C = B.A, M and N traded
   BitArgs bits;            // Kern::Bits / Kern::Reduce
   GemmArgs gemm;           // Kern::Gemm
+  MfmaArgs mfma;           // Kern::Gemm with gemm.tile 3: the matrix-core GEMM
   RowArgs rows;            // Kern::Rows
   RadixArgs radix;         // Kern::Radix
   BlasArgs blas;           // Kern::Blas
@@ -387,7 +420,7 @@ constexpr int kLdsCycleBytes = 256;
 void chain_swizzle(ChainArgs &a, int elem_bytes);
 
 // Run `st` with kernel configuration `choice` (0 gather, 1 rows, 2-4 FP tile GEMMs,
-// 5 / 7 matrix-core GEMM, 6 reduce, 8 vendor BLAS on plain matrix layouts); false
+// 5 / 7 matrix-core GEMM on any layout, 6 reduce, 8 vendor BLAS on plain matrix layouts); false
 // (and `st` unchanged) if that kernel cannot.
 bool force_kernel(Step &st, int precision, int choice);
 // Alternative kernel configurations of a step (the current one first) for the autotuner.
@@ -397,6 +430,8 @@ void launch_contract_bits(int prec, const void *A, const void *B, void *C, void 
 // With args.ksplit > 1, `ws` receives ksplit partials of C which are then summed
 // into C.
 void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void *ws, const GemmArgs &args,
+                          void *stream);
+void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &args,
                           void *stream);
 void launch_contract_rows(int prec, const void *A, const void *B, void *C, const RowArgs &args,
                           void *stream);

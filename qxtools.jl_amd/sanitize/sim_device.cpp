@@ -375,6 +375,31 @@ void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void 
   });
 }
 
+void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &g, void *stream) {
+  const size_t es = esize(prec);
+  if (g.cfg < 0 || g.cfg >= 5 || g.nxb > kMfmaTileBits || g.nyb > kMfmaTileBits || g.nsb > kMaxBits || g.nub > kMaxBits)
+    violation("matrix-core GEMM arguments out of range");
+  // LDS slots of the tile's elements, rows and columns of its results
+  const int tm = kMfmaTiles[g.cfg][0], tn = kMfmaTiles[g.cfg][1], tk = g.kk;
+  int mx = 0, my = 0;
+  for (int i = 0; i < g.nxb; ++i) mx += g.xs[i];
+  for (int i = 0; i < g.nyb; ++i) my += g.ys[i];
+  if (mx >= tk * mfma_pitch(tm, (int)es) || my >= tk * mfma_pitch(tn, (int)es) || g.mmask >= tm || g.nmask >= tn ||
+      (g.kk != 4 && g.kk != 8 && g.kk != 16))
+    violation("matrix-core GEMM tile outside its LDS");
+  const long double cu = sum_n(g.cm, 7) + sum_n(g.cn, 7) + sum_n(g.uc, g.nub) + 1;
+  const long double rx = (sum_n(g.xw, g.nxb) + sum_n(g.sx, g.nsb) + sum_n(g.ux, g.nub) + 1) * es;
+  const long double ry = (sum_n(g.yw, g.nyb) + sum_n(g.sy, g.nsb) + sum_n(g.uy, g.nub) + 1) * es;
+  const void *X = g.swap ? B : A, *Y = g.swap ? A : B;
+  if (cu > (long double)g.c_elems * g.ksplit) violation("matrix-core GEMM results outside C");
+  launch(stream, [=]() {
+    need(X, rx, "matrix-core GEMM X");
+    need(Y, ry, "matrix-core GEMM Y");
+    need(C, (long double)g.c_elems * es, "matrix-core GEMM C");
+    need(ws, g.ksplit > 1 ? (long double)g.c_elems * g.ksplit * es : 0, "matrix-core GEMM K-split partials");
+  });
+}
+
 void launch_contract_rows(int prec, const void *A, const void *B, void *C, const RowArgs &r, void *stream) {
   const size_t es = esize(prec);
   const long double ra = (sum_n(r.ra, r.nbr) + max_n(r.ka, r.nk) + 1) * es;
