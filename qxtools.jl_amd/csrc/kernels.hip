@@ -614,34 +614,67 @@ __global__ void k_sum_splits(typename Vec<T>::type *__restrict__ C, const typena
   }
 }
 
-// One wave per C element, the K range split over lanes, shuffle reduction.
+// One wave per C element and K range, lanes along K (the larger operand's smallest
+// strides first), shuffle reduction.  Bound by HBM reads: four terms per lane are loaded
+// before they are used, and the offsets of the next four come from one table entry per
+// operand (the entry of the lowest set bit of the trip counter: its stride less those of
+// the bits that turn to zero), instead of a walk over all K bits per term.  6x6, N 256,
+// K 131072, complex64: see launch_contract_reduce.
+constexpr int kReduceTerms = 4;   // per lane and trip: K bits 6 and 7
+
 template <typename T>
 __global__ __launch_bounds__(256) void k_contract_reduce(const typename Vec<T>::type *__restrict__ A,
                                                          const typename Vec<T>::type *__restrict__ B,
                                                          typename Vec<T>::type *__restrict__ C,
                                                          int64_t c_elems, BitArgs a) {
   using V = typename Vec<T>::type;
+  __shared__ int64_t inc[2][kMaxBits];
+  for (int b = 8 + threadIdx.x; b < a.nbk; b += 256) {
+    int64_t ia = a.ka[b], ib = a.kb[b];
+    for (int j = 8; j < b; ++j) ia -= a.ka[j], ib -= a.kb[j];
+    inc[0][b - 8] = ia;
+    inc[1][b - 8] = ib;
+  }
+  __syncthreads();
   const int lane = threadIdx.x & 63;
   const int64_t nk = int64_t(1) << a.nbk;
-  const int64_t kper = nk / a.ksplit;         // K range of one wave
-  // per-lane offsets of the low 6 k bits
-  int64_t la = 0, lb = 0;
+  const int64_t kper = nk / a.ksplit;         // K range of one wave, a power of two >= 64
+  // per-lane offsets of the low 6 k bits; per term those of the next two
+  int64_t la = 0, lb = 0, ta[kReduceTerms], tb[kReduceTerms];
   for (int b = 0; b < 6 && b < a.nbk; ++b)
     if ((lane >> b) & 1) la += a.ka[b], lb += a.kb[b];
+#pragma unroll
+  for (int t = 0; t < kReduceTerms; ++t) {
+    ta[t] = (t & 1 ? a.ka[6] : 0) + (t & 2 ? a.ka[7] : 0);
+    tb[t] = (t & 1 ? a.kb[6] : 0) + (t & 2 ? a.kb[7] : 0);
+  }
+  const int64_t trips = kper / (64 * kReduceTerms);
   const int64_t waves = (int64_t)gridDim.x * 4;
   const int64_t units = c_elems * a.ksplit;   // (C element, K range); partials land at C[split*c_elems + idx]
   for (int64_t u = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); u < units; u += waves) {
     const int64_t idx = u % c_elems, split = u / c_elems;
-    int64_t oa = 0, ob = 0;
+    int64_t oa = la, ob = lb;
     for (int b = 0; b < a.nbc; ++b)
       if ((idx >> b) & 1) oa += a.wa[b], ob += a.wb[b];
+    const int64_t k0 = split * kper;
+    for (int b = 6; b < a.nbk; ++b)
+      if ((k0 >> b) & 1) oa += a.ka[b], ob += a.kb[b];
     V acc{0, 0};
-    for (int64_t k0 = split * kper; k0 < (split + 1) * kper; k0 += 64) {
-      if (k0 + lane >= nk) break;
-      int64_t ha = 0, hb = 0;
-      for (int b = 6; b < a.nbk; ++b)
-        if ((k0 >> b) & 1) ha += a.ka[b], hb += a.kb[b];
-      cmac<T>(acc, A[oa + ha + la], B[ob + hb + lb], a.conj_a, a.conj_b);
+    if (trips >= 1) {
+      for (int64_t t = 0; t < trips; ++t) {
+        V av[kReduceTerms], bv[kReduceTerms];
+#pragma unroll
+        for (int e = 0; e < kReduceTerms; ++e) av[e] = A[oa + ta[e]], bv[e] = B[ob + tb[e]];
+#pragma unroll
+        for (int e = 0; e < kReduceTerms; ++e) cmac<T>(acc, av[e], bv[e], a.conj_a, a.conj_b);
+        if (t + 1 < trips) {
+          const int z = __ffsll((unsigned long long)(t + 1)) - 1;
+          oa += inc[0][z], ob += inc[1][z];
+        }
+      }
+    } else {   // a range of 64 or 128 (or fewer lanes than 64)
+      for (int64_t k = 0; k < kper && k + lane < nk; k += 64)
+        cmac<T>(acc, A[oa + (k ? a.ka[6] : 0)], B[ob + (k ? a.kb[6] : 0)], a.conj_a, a.conj_b);
     }
     for (int off = 32; off > 0; off >>= 1) {
       acc.x += __shfl_xor(acc.x, off, 64);

@@ -456,6 +456,12 @@ bool configure_kernel(Step &st, int precision, int choice) {
       if (nk < 6) return false;
       st.kern = Kern::Reduce;
       while (st.c_elems * b.ksplit < 8192 && (int64_t(1) << nk) / b.ksplit >= 128) b.ksplit *= 2;
+      // lanes walk the low K bits: give them the larger operand's smallest strides
+      std::vector<std::pair<int64_t, int64_t>> kb(sb.kbits);
+      std::stable_sort(kb.begin(), kb.end(), [&](const auto &p, const auto &q) {
+        return nn > nm ? p.second < q.second : p.first < q.first;
+      });
+      for (int i = 0; i < nk; ++i) b.ka[i] = kb[i].first, b.kb[i] = kb[i].second;
       break;
     }
     case kPlain3:   // complex128 as three real products per complex product
@@ -567,11 +573,12 @@ bool configure_kernel(Step &st, int precision, int choice) {
       st.kern = Kern::Gemm;
       st.gemm = GemmArgs{};
       st.gemm.tile = 3;
-      st.mfma = MfmaArgs{};
-      if (!mfma_args(sb, precision, choice == kMfmaT, st.c_elems, st.mfma)) return false;
-      st.mfma.conj_x = st.mfma.swap ? st.radix.conj_b : st.radix.conj_a;
-      st.mfma.conj_y = st.mfma.swap ? st.radix.conj_a : st.radix.conj_b;
-      st.ws_elems = st.mfma.ksplit > 1 ? st.mfma.ksplit * st.c_elems : 0;
+      auto m = std::make_shared<MfmaArgs>();
+      if (!mfma_args(sb, precision, choice == kMfmaT, st.c_elems, *m)) return false;
+      m->conj_x = m->swap ? st.radix.conj_b : st.radix.conj_a;
+      m->conj_y = m->swap ? st.radix.conj_a : st.radix.conj_b;
+      st.ws_elems = m->ksplit > 1 ? m->ksplit * st.c_elems : 0;
+      st.mfma = std::move(m);
       return true;
     }
     case kGemm0:
@@ -621,8 +628,15 @@ bool configure_kernel(Step &st, int precision, int choice) {
   return true;
 }
 
-// Whether the matrix-core GEMM on any layout is the default of a step with at least 8
-// rows and columns and 2^18 multiply-adds.  complex64: always (6x6 workload, 256 strings,
+// With 4 rows and columns or more the any-layout matrix-core GEMM is faster than the gather
+// kernel from about 2^15 multiply-adds (complex128, in one call's graph: H 2, M 512, N 16,
+// K 2: 7.0 us, 9.7; H 1024, M 4, N 64, K 4: 11, 16; H 8, M 8, N 16384, K 8: 14, 28).
+bool mfma_over_bits(const StepBits &sb, const Step &st) {
+  return std::min(sb.nm, sb.nn) >= 2 && (double)st.H * st.M * st.N * st.K >= double(1 << 15);
+}
+
+// Whether it is preferred to the row kernel and the vector tiles too: a step with at least
+// 8 rows and columns and 2^18 multiply-adds.  complex64: always (6x6 workload, 256 strings,
 // H 4096, M 64, N 128, K 512: 1.28 ms, vector tiles 2.65; M 16, N 65536, K 8: 22 us,
 // gather kernel 117).  complex128: from 2^25 multiply-adds (7x7, H 128, M 256, N 16384,
 // K 256: 17.1 ms, vector tiles 33.5; H 512, M 16, N 131072, K 4: 4.0 ms, gather kernel
@@ -650,8 +664,11 @@ bool mfma_default(const StepBits &sb, const Step &st, int precision) {
 //  * Mfma   : mfma_default
 //  * Gemm   : K >= 8, N >= 8, M >= 32 (bits of each class counted without H); complex64
 //             with N, M >= 64 on FP32 matrix cores
-//  * small C (<= 2^14) with K >= 256: lanes along K (Reduce) when a K bit is A's
-//    unit stride, else the gather kernel with K split over workgroups
+//  * Skinny : K >= 4096 into at most 32 values per batch element, 2^18 multiply-adds or
+//             more (7x7, H 32, M 16, N 2, K 2^21, complex128: 3.5 ms at 5.5 TB/s, one wave
+//             per element 13.5; 5x5, H 256, K 4096: 24 us, gather kernel 319)
+//  * small C (<= 2^14) with K >= 256: lanes along K (Reduce) when a K bit is the larger
+//    operand's unit stride, else the gather kernel with K split over workgroups
 //  * Bits   : everything else with power-of-two dims
 //  * Radix  : any other dims
 //  * Blas   : the vendor BLAS, a tuned candidate only
@@ -671,14 +688,17 @@ int default_choice(const Step &st, int precision) {
     if (precision != QX_C128 && sb.nn >= 6 && sb.nm >= 6) return kMfma;
     return sb.nn <= 4 ? kGemm0 : sb.nn == 5 ? kGemm1 : kGemm2;
   }
+  if (sb.nk >= 12 && sb.nm + sb.nn <= 5 && sb.nn <= 1 && (double)st.H * st.M * st.N * st.K >= double(1 << 18))
+    return kSkinny;
   if (st.c_elems <= (int64_t(1) << 14) && sb.nk >= 8) {
+    const bool by_b = sb.nn > sb.nm;
     int64_t kmin = INT64_MAX, cmin = INT64_MAX;
-    for (auto &kb : sb.kbits) kmin = std::min(kmin, kb.first);
+    for (auto &kb : sb.kbits) kmin = std::min(kmin, by_b ? kb.second : kb.first);
     for (auto &c : sb.cbits)
-      if (c.wa) cmin = std::min(cmin, c.wa);
+      if (by_b ? c.wb : c.wa) cmin = std::min(cmin, by_b ? c.wb : c.wa);
     return kmin < cmin ? kReduce : kBits;
   }
-  return kBits;
+  return mfma_over_bits(sb, st) ? kMfma : kBits;
 }
 
 void set_kernel_args(Step &st, int precision) {
@@ -706,6 +726,25 @@ static Step swap_operands(const Step &st) {
   std::swap(v.bits.conj_a, v.bits.conj_b);
   v.swapped = !st.swapped;
   return v;
+}
+
+// A forward step whose N side is long and M side narrow runs the row kernel over B's
+// legs (C = B.A) where that streams better: 2^17 rows or more and 2 or 4 columns (7x7,
+// H 64, M 4, N 2^19, K 2, complex128: 0.58 ms, gather kernel 1.17); with 8 columns and
+// K <= 4, or 16 and K <= 2, on 2^18 rows when C's fastest bit is a row's, so that lanes
+// store side by side (H 2, M 16, N 2^22, K 2, complex64: 0.25 ms, any-layout GEMM 0.30;
+// with a column bit fastest the GEMM is the faster: H 1, M 8, N 2^20: 31 us against 50).
+static void prefer_rows_swapped(Step &st, int precision) {
+  const bool gemm = st.kern == Kern::Gemm && st.gemm.tile == 3;
+  if (st.level >= 0 || st.swapped || !(gemm || st.kern == Kern::Bits) || st.bits.ksplit > 1) return;
+  if (st.M < 2 || st.M > 16 || st.K > 16 || st.H * st.N < (int64_t(1) << 17)) return;
+  Step w = swap_operands(st);
+  const StepBits sw = step_bits(w);
+  if (!rows_ok(sw) || sw.nk > 4 || sw.nn < 1 || sw.nm < 8 || sw.cbits.empty()) return;
+  const bool narrow = sw.nn <= 2 && sw.nr >= 17;
+  const bool wide = sw.nr >= 18 && sw.cbits[0].wa != 0 && ((sw.nn <= 3 && sw.nk <= 2) || (sw.nn <= 4 && sw.nk <= 1));
+  if (narrow || wide)
+    if (force_kernel(w, precision, kRows)) st = std::move(w);
 }
 
 bool force_kernel(Step &st, int precision, int choice) {
@@ -760,7 +799,7 @@ std::vector<Step> kernel_candidates(const Step &st, int precision) {
   std::vector<int> alts;
   if (st.kern == Kern::Gemm || (sb.nk >= 2 && sb.nn >= 2 && sb.nm >= 4))
     alts.insert(alts.end(), {kGemm0, kGemm1, kGemm2});
-  if (sb.nn >= 2 && sb.nm >= 2) alts.insert(alts.end(), {kMfma, kMfmaT});
+  if ((sb.nn >= 2 && sb.nm >= 2) || (sb.nk >= 8 && std::max(sb.nm, sb.nn) >= 5)) alts.insert(alts.end(), {kMfma, kMfmaT});
   if (sb.nr >= 8 && rows_ok(sb)) alts.push_back(kRows);
   if (st.c_elems <= (int64_t(1) << 16) && sb.nk >= 6) alts.push_back(kReduce);
   if (sb.nk >= 12 && sb.nm + sb.nn <= 5 && sb.nn <= 1) alts.push_back(kSkinny);
@@ -1881,6 +1920,7 @@ Lowered lower(const Program &p, int64_t batch, bool keep_all, int precision, uin
     }
   }
   if (chains || keep_all) level_small_steps(p, L);
+  for (Step &st : L.steps) prefer_rows_swapped(st, precision);
 
   // result elements per bitstring
   L.result_elems = 1;

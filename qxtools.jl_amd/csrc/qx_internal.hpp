@@ -4,6 +4,7 @@
 
 #include <cstdint>
 #include <map>
+#include <memory>
 #include <stdexcept>
 #include <string>
 #include <vector>
@@ -324,7 +325,7 @@ struct Step {
   bool swapped = false;    // operands exchanged (in_a is the DSL's B): C = B.A, M and N traded
   BitArgs bits;            // Kern::Bits / Kern::Reduce
   GemmArgs gemm;           // Kern::Gemm
-  MfmaArgs mfma;           // Kern::Gemm with gemm.tile 3: the matrix-core GEMM
+  std::shared_ptr<const MfmaArgs> mfma;   // Kern::Gemm with gemm.tile 3: the matrix-core GEMM
   RowArgs rows;            // Kern::Rows
   RadixArgs radix;         // Kern::Radix
   BlasArgs blas;           // Kern::Blas

@@ -416,7 +416,7 @@ void launch_step(qx_plan *P, const qx::Lowered &L, const qx::Step &st, void *A, 
     }
     case qx::Kern::Radix: qx::launch_contract_radix(P->prec, A, B, C, st.c_elems, st.radix, stream); break;
     case qx::Kern::Gemm:
-      if (st.gemm.tile == 3) qx::launch_contract_mfma(P->prec, A, B, C, P->ws.p, st.mfma, stream);
+      if (st.gemm.tile == 3) qx::launch_contract_mfma(P->prec, A, B, C, P->ws.p, *st.mfma, stream);
       else qx::launch_contract_gemm(P->prec, A, B, C, P->ws.p, st.gemm, stream);
       break;
     case qx::Kern::Reduce: qx::launch_contract_reduce(P->prec, A, B, C, P->ws.p, st.c_elems, st.bits, stream); break;
@@ -1144,7 +1144,7 @@ std::string kern_variant(const qx::Step &st) {
       return "k_contract_rows<" + std::to_string(st.rows.nk) + "," + std::to_string(nc) + ">";
     }
     case qx::Kern::Gemm:
-      if (st.gemm.tile == 3) return st.mfma.other ? "k_contract_gemm_mfma<yx>" : "k_contract_gemm_mfma";
+      if (st.gemm.tile == 3) return st.mfma->other ? "k_contract_gemm_mfma<yx>" : "k_contract_gemm_mfma";
       return st.gemm.tile == 0 ? "k_contract_gemm<128,16,16>" : st.gemm.tile == 1 ? "k_contract_gemm<128,32,16>"
                                                                                    : "k_contract_gemm<64,64,16>";
     case qx::Kern::Reduce:
