@@ -2508,132 +2508,162 @@ __global__ __launch_bounds__(kChainThreads) void k_contract_chain(const typename
 }
 
 // ---------------------------------------------------------------------------
-// Small-step batch: workgroup i contracts C elements [c0, c1) of the step of
-// descriptor i (lanes along C, the K loop in registers; a range shorter than the
-// workgroup splits each element's K range over 256 / (c1 - c0) lanes, summed in
-// LDS).  The steps of one launch are independent.
+// Small steps: items of one wave each (SmallDesc).  Bound by latency alone: a level's
+// arithmetic is a few multiply-adds per lane, its time the descriptor, the operand loads
+// and the launch.  So the descriptor of a wave's next item is loaded (one word per lane)
+// while it works on the current one, across levels too, and read by lane index; offsets
+// are a lane part and wave-uniform parts; up to eight terms' operands are in flight at
+// once; K lanes are summed by shuffles, so no item needs a barrier.
 
-// Sum over k = k0, k0 + dk, ... < nk of A[oa + offset_a(k)] * B[ob + offset_b(k)] for a
-// small-step descriptor, in that order: the operands of 8 terms are loaded before
-// they are used, so that their loads are in flight together.
-template <typename T>
-__device__ __forceinline__ typename Vec<T>::type small_dot(const SmallDesc &s, const typename Vec<T>::type *A,
-                                                           const typename Vec<T>::type *B, int64_t oa, int64_t ob,
-                                                           int k0, int dk, int nk) {
+// Terms f = 0 .. F-1 of an item, U at a time: element f >> t, K term f & (2^t - 1).
+// `prefetch` runs once the first terms' loads are issued: loads return in order, so one
+// issued ahead of them would hold them up.
+template <typename T, int U, typename Prefetch>
+__device__ __forceinline__ void small_terms(int32_t d0, int32_t d1, const typename Vec<T>::type *A,
+                                            const typename Vec<T>::type *B, void *C, int32_t oa, int32_t ob, int32_t oc,
+                                            int32_t pack, bool store, Prefetch &&prefetch) {
   using V = typename Vec<T>::type;
-  constexpr int U = 8;
-  V acc{0, 0};
-  int k = k0;
-  for (; k + (U - 1) * dk < nk; k += U * dk) {
-    V av[U], bv[U];
+  constexpr int LU = U == 8 ? 3 : U == 4 ? 2 : U == 2 ? 1 : 0;
+  const int lt = pack & 15, nt = 1 << ((pack >> 12) & 31), nf = nt << ((pack >> 8) & 15);
+  const int conj_a = (pack >> 20) & 1, conj_b = (pack >> 21) & 1;
+  auto word = [&](int i) { return __builtin_amdgcn_readlane(i < 64 ? d0 : d1, i & 63); };
+  // offsets of the U terms of a trip from the first of its increments
+  int32_t ua[U], ub[U];
+  {
+    int32_t wa[3] = {0, 0, 0}, wb[3] = {0, 0, 0}, sa = 0, sb = 0;
+#pragma unroll
+    for (int b = 0; b < LU; ++b) {
+      wa[b] = word(26 + b) + sa, wb[b] = word(45 + b) + sb;
+      sa += wa[b], sb += wb[b];
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int kk = k + u * dk;
-      int64_t xa = oa, xb = ob;
-      for (int b = 0; b < s.nbk; ++b)
-        if ((kk >> b) & 1) xa += s.ka[b], xb += s.kb[b];
-      av[u] = A[xa];
-      bv[u] = B[xb];
+      ua[u] = (u & 1 ? wa[0] : 0) + (u & 2 ? wa[1] : 0) + (u & 4 ? wa[2] : 0);
+      ub[u] = (u & 1 ? wb[0] : 0) + (u & 2 ? wb[1] : 0) + (u & 4 ? wb[2] : 0);
+    }
+  }
+  V acc{0, 0};
+  int e = 0;
+  for (int f0 = 0; f0 < nf; f0 += U) {
+    V av[U], bv[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) av[u] = A[oa + ua[u]], bv[u] = B[ob + ub[u]];
+    if (f0 == 0) prefetch();
+    if (f0 + U < nf) {   // the next trip's first term: one increment, plus what this trip's low bits hold
+      const int z = __ffs(f0 + U) - 1;
+      oa += __builtin_amdgcn_readlane(d0, 26 + z) + ua[U - 1];
+      ob += __builtin_amdgcn_readlane(d0, 45 + z) + ub[U - 1];
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) cmac<T>(acc, av[u], bv[u], s.conj_a, s.conj_b);
-  }
-  for (; k < nk; k += dk) {
-    int64_t xa = oa, xb = ob;
-    for (int b = 0; b < s.nbk; ++b)
-      if ((k >> b) & 1) xa += s.ka[b], xb += s.kb[b];
-    cmac<T>(acc, A[xa], B[xb], s.conj_a, s.conj_b);
-  }
-  return acc;
-}
-
-// One chunk of a small step (descriptor `s`) by the workgroup's kSmallThreads lanes.
-template <typename T>
-__device__ __forceinline__ void small_item(const SmallDesc &s, typename Vec<T>::type *part) {
-  using V = typename Vec<T>::type;
-  const V *A = (const V *)s.A;
-  const V *B = (const V *)s.B;
-  V *C = (V *)s.C;
-  const int nk = 1 << s.nbk;
-  const int len = s.c1 - s.c0;   // a power of two
-  if (len < kSmallThreads && nk > 1) {   // lanes split K: 2^lt lanes per element of the chunk
-    const int lt = 8 - (__ffs(len) - 1);   // kSmallThreads = 2^8
-    const int c = s.c0 + (threadIdx.x >> lt), sub = threadIdx.x & ((1 << lt) - 1);
-    int64_t oa = 0, ob = 0;
-    for (int b = 0; b < s.nbc; ++b)
-      if ((c >> b) & 1) oa += s.wa[b], ob += s.wb[b];
-    V acc = small_dot<T>(s, A, B, oa, ob, sub, 1 << lt, nk);
-    part[threadIdx.x] = acc;
-    __syncthreads();
-    if (sub == 0) {
-      V sum = part[threadIdx.x];
-      for (int j = 1; j < (1 << lt); ++j) {
-        sum.x += part[threadIdx.x + j].x;
-        sum.y += part[threadIdx.x + j].y;
+    for (int u = 0; u < U; ++u) {
+      cmac<T>(acc, av[u], bv[u], conj_a, conj_b);
+      if (((f0 + u + 1) & (nt - 1)) == 0) {   // element e is complete
+        for (int k = 1; k < (1 << lt); k <<= 1) {
+          acc.x += __shfl_xor(acc.x, k, 64);
+          acc.y += __shfl_xor(acc.y, k, 64);
+        }
+        const int32_t o = oc + (e & 1 ? word(64) : 0) + (e & 2 ? word(65) : 0) + (e & 4 ? word(66) : 0);
+        if (store) {
+          if (!((pack >> 22) & 1)) {
+            ((V *)C)[o] = acc;
+          } else if ((pack >> 23) & 1) {   // add into an FP64 gradient
+            double2 *dst = (double2 *)C + o;
+            dst->x += (double)acc.x;
+            dst->y += (double)acc.y;
+          } else {                         // add into a cotangent buffer
+            V *dst = (V *)C + o;
+            dst->x += acc.x;
+            dst->y += acc.y;
+          }
+        }
+        acc = V{0, 0};
+        ++e;
       }
-      C[c] = sum;
     }
-    __syncthreads();   // `part` is free again
-    return;
-  }
-  for (int c = s.c0 + threadIdx.x; c < s.c1; c += blockDim.x) {
-    int64_t oa = 0, ob = 0;
-    for (int b = 0; b < s.nbc; ++b)
-      if ((c >> b) & 1) oa += s.wa[b], ob += s.wb[b];
-    C[c] = small_dot<T>(s, A, B, oa, ob, 0, 1, nk);
   }
 }
 
-template <typename T>
-__global__ __launch_bounds__(kSmallThreads) void k_small_batch(const SmallDesc *__restrict__ d) {
-  __shared__ typename Vec<T>::type part[kSmallThreads];
-  small_item<T>(d[blockIdx.x], part);
+template <typename T, typename Prefetch>
+__device__ __forceinline__ void small_item(int32_t d0, int32_t d1, const SmallVars &vars, Prefetch &&prefetch) {
+  using V = typename Vec<T>::type;
+  const int lane = threadIdx.x & 63;
+  auto word = [&](int i) { return __builtin_amdgcn_readlane(i < 64 ? d0 : d1, i & 63); };
+  auto pointer = [&](int i) { return (uint64_t)(uint32_t)word(i) | (uint64_t)(uint32_t)word(i + 1) << 32; };
+  const int32_t pack = word(6);
+  const V *A = (const V *)pointer(0);
+  const V *B = (const V *)pointer(2);
+  for (int q = 0; q < ((pack >> 24) & 15); ++q)
+    A += (int64_t)vars.v[(word(67) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 5 + q);
+  for (int q = 0; q < ((pack >> 28) & 15); ++q)
+    B += (int64_t)vars.v[(word(68) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 9 + q);
+  int32_t oa = 0, ob = 0, oc = 0;
+#pragma unroll
+  for (int b = 0; b < kSmallLaneBits; ++b) {
+    const int32_t on = -((lane >> b) & 1);
+    oa += on & word(8 + b), ob += on & word(14 + b), oc += on & word(20 + b);
+  }
+  const int lt = pack & 15;
+  const bool store = lane < (1 << ((pack >> 4) & 15)) && (lane & ((1 << lt) - 1)) == 0;
+  void *C = (void *)pointer(4);
+  switch (((pack >> 8) & 15) + ((pack >> 12) & 31)) {
+    case 0: small_terms<T, 1>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
+    case 1: small_terms<T, 2>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
+    case 2: small_terms<T, 4>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
+    default: small_terms<T, 8>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
+  }
 }
 
-// Every dependency level of a section's small steps in one launch by one workgroup:
-// the levels' chunks in order, a workgroup barrier between levels (so a level reads
-// what the previous ones wrote).  For sections whose small steps are tiny in total:
-// the levels' launch gaps cost more than their arithmetic.  One workgroup keeps every
-// producer and consumer on one CU; workgroups on several XCDs would need an L2
-// write-back and invalidate at each level to see each other's results, which costs
-// more than a launch.
+// Levels [0, nlevels) of items in order, the waves of the grid taking a level's items in
+// turn, a workgroup barrier between levels (one workgroup: producers and consumers share
+// a CU; workgroups on several XCDs would need an L2 write-back and invalidate per level,
+// dearer than a launch).
 template <typename T>
-__global__ __launch_bounds__(kSmallThreads) void k_small_walk(const SmallDesc *__restrict__ d,
-                                                              const int *__restrict__ level_off, int nlevels) {
-  __shared__ typename Vec<T>::type part[kSmallThreads];
+__device__ __forceinline__ void small_levels(const SmallDesc *__restrict__ d, const int *__restrict__ off, int n,
+                                             int nlevels, const SmallVars &vars) {
+  const int lane = threadIdx.x & 63;
+  const int waves = (int)(gridDim.x * (blockDim.x >> 6));
+  const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)));
+  int32_t d0 = 0, d1 = 0;
+  auto load = [&](int i) {
+    const int32_t *w = d[i].w;
+    d0 = w[lane];
+    d1 = w[64 + (lane & 31)];
+  };
+  auto bound = [&](int L) { return off ? off[L] : L ? n : 0; };
+  int lo = bound(0), hi = bound(1);
+  load(lo + wave < hi ? lo + wave : lo);
   for (int L = 0; L < nlevels; ++L) {
-    const int i1 = level_off[L + 1];
-    for (int i = level_off[L]; i < i1; ++i) small_item<T>(d[i], part);
-    __syncthreads();
+    // this wave's first item of the next level (its own last item again where it has none)
+    const int nlo = hi, nhi = L + 1 < nlevels ? bound(L + 2) : hi;
+    const int next = nlo + wave < nhi ? nlo + wave : lo;
+    int i = lo + wave;
+    if (i >= hi) {
+      load(next);
+    } else {
+      for (; i < hi; i += waves) {
+        const int32_t c0 = d0, c1 = d1;
+        small_item<T>(c0, c1, vars, [&]() { load(i + waves < hi ? i + waves : next); });
+      }
+    }
+    lo = nlo, hi = nhi;
+    if (L + 1 < nlevels) __syncthreads();
   }
 }
 
-// Batched scatter-add: workgroup i adds descriptor i's dense temp into its FP64
-// destination through the destination's strides.  Destinations of one launch are
-// disjoint.
-template <typename TS>
-__global__ __launch_bounds__(256) void k_add_batch(const AddDesc *__restrict__ d) {
-  using VS = typename Vec<TS>::type;
-  const AddDesc &a = d[blockIdx.x];
-  const VS *src = (const VS *)a.src;
-  for (int64_t e = threadIdx.x; e < a.n; e += blockDim.x) {
-    int64_t r = e, o = 0;
-    for (int j = 0; j < a.nd; ++j) {
-      const int64_t q = r % a.dim[j];
-      r /= a.dim[j];
-      o += q * a.st[j];
-    }
-    const VS v = src[e];
-    if (a.dst_f64) {
-      double2 *dst = (double2 *)a.dst;
-      dst[o].x += (double)v.x;
-      dst[o].y += (double)v.y;
-    } else {
-      VS *dst = (VS *)a.dst;
-      dst[o].x += v.x;
-      dst[o].y += v.y;
-    }
-  }
+// One level (off null: the n items) over the grid, or a run of levels in one workgroup.
+template <typename T>
+__global__ __launch_bounds__(kSmallRunThreads) void k_small_batch(const SmallDesc *__restrict__ d,
+                                                                  const int *__restrict__ off, int n, int nlevels,
+                                                                  SmallVars vars) {
+  small_levels<T>(d, off, n, nlevels, vars);
+}
+
+// Every level of a section in one workgroup (plan option small_walk).
+template <typename T>
+__global__ __launch_bounds__(kSmallRunThreads) void k_small_walk(const SmallDesc *__restrict__ d,
+                                                                 const int *__restrict__ off, int n, int nlevels,
+                                                                 SmallVars vars) {
+  small_levels<T>(d, off, n, nlevels, vars);
 }
 
 // ---------------------------------------------------------------------------
@@ -3043,34 +3073,29 @@ void launch_plain_gemm(int prec, const void *X, const void *Y, void *C, void *ws
   }
 }
 
-void launch_small_batch(int prec, const SmallDesc *d_desc, int n, void *stream) {
+void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVars &vars, void *stream) {
   if (n <= 0) return;
   hipStream_t s = (hipStream_t)stream;
+  const int per = kSmallThreads / 64, g = (n + per - 1) / per;
   if (prec == QX_C128)
-    hipLaunchKernelGGL(k_small_batch<double>, dim3(n), dim3(kSmallThreads), 0, s, d_desc);
+    hipLaunchKernelGGL(k_small_batch<double>, dim3(g), dim3(kSmallThreads), 0, s, d_desc, (const int *)nullptr, n, 1, vars);
   else
-    hipLaunchKernelGGL(k_small_batch<float>, dim3(n), dim3(kSmallThreads), 0, s, d_desc);
+    hipLaunchKernelGGL(k_small_batch<float>, dim3(g), dim3(kSmallThreads), 0, s, d_desc, (const int *)nullptr, n, 1, vars);
   check_launch("small_batch");
 }
 
-void launch_small_walk(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, void *stream) {
+void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
+                      bool walk, void *stream) {
   if (nlevels <= 0) return;
   hipStream_t s = (hipStream_t)stream;
-  if (prec == QX_C128)
-    hipLaunchKernelGGL(k_small_walk<double>, dim3(1), dim3(kSmallThreads), 0, s, d_desc, d_level_off, nlevels);
-  else
-    hipLaunchKernelGGL(k_small_walk<float>, dim3(1), dim3(kSmallThreads), 0, s, d_desc, d_level_off, nlevels);
-  check_launch("small_walk");
-}
-
-void launch_add_batch(int prec, const AddDesc *d_desc, int n, void *stream) {
-  if (n <= 0) return;
-  hipStream_t s = (hipStream_t)stream;
-  if (prec == QX_C128)
-    hipLaunchKernelGGL(k_add_batch<double>, dim3(n), dim3(256), 0, s, d_desc);
-  else
-    hipLaunchKernelGGL(k_add_batch<float>, dim3(n), dim3(256), 0, s, d_desc);
-  check_launch("add_batch");
+#define QX_RUN(K) hipLaunchKernelGGL(K, dim3(1), dim3(kSmallRunThreads), 0, s, d_desc, d_level_off, 0, nlevels, vars)
+  if (prec == QX_C128) {
+    if (walk) QX_RUN(k_small_walk<double>); else QX_RUN(k_small_batch<double>);
+  } else {
+    if (walk) QX_RUN(k_small_walk<float>); else QX_RUN(k_small_batch<float>);
+  }
+#undef QX_RUN
+  check_launch("small_run");
 }
 
 }  // namespace qx

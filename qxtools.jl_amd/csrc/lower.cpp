@@ -1419,7 +1419,8 @@ std::vector<int> form_outer_runs(const Program &p, Lowered &L) {
   for (auto &run : runs) {
     // runs that end in a small step stay: the small steps of a section run batched by
     // dependency level, many per launch
-    if (run.size() < 2 || small_step(L.steps[run.back()], false)) continue;
+    // (not section 1's: one launch for the run there, once per slice)
+    if (run.size() < 2 || (L.steps[run.back()].section != 1 && small_step(L.steps[run.back()], false))) continue;
     Step f;
     if (!outer_step(L, run, f)) continue;
     for (size_t j = 0; j + 1 < run.size(); ++j) {
@@ -1558,39 +1559,86 @@ void chain_swizzle(ChainArgs &a, int elem_bytes) {
 
 namespace {
 
-// Whether a step may run inside a small-step batch (one workgroup per step):
-// slice-free, power-of-two legs with at most kSmallMaxBits C and K bits each, at most
-// 2^18 MACs, and operand offsets that fit 32 bits.  C and K are each at most 4096,
+// Whether a step may run inside a small-step batch: power-of-two legs with at most
+// kSmallMaxBits C and K bits each, at most 2^18 MACs, and operand offsets that fit 32 bits.  C and K are each at most 4096,
 // except with `wide` (the pullback, whose gradient steps sum long bitstring-batch
 // ranges into a few elements): then up to 2^16 MACs with any split.  (The forward
 // keeps the limit: its larger steps run faster as multi-workgroup launches.)
 bool small_step(const Step &st, bool wide = false) {
-  if (st.section == 1 || st.kern == Kern::Chain || st.kern == Kern::Radix || st.kern == Kern::Outer) return false;
+  if (st.kern == Kern::Chain || st.kern == Kern::Radix || st.kern == Kern::Outer) return false;
   const int64_t macs = st.c_elems * st.K;
   if (macs > (int64_t(1) << 18)) return false;
   if ((st.c_elems > 4096 || st.K > 4096) && (!wide || macs > (int64_t(1) << 16))) return false;
   int nbc = 0, nbk = 0;
-  int64_t wmax = 0;
+  int64_t wa = 0, wb = 0;
   for (auto &g : st.cl) {
     if (!pow2(g.dim)) return false;
     nbc += ilog2(g.dim);
-    wmax = std::max({wmax, g.sa * (g.dim - 1), g.sb * (g.dim - 1)});
+    wa += g.sa * (g.dim - 1), wb += g.sb * (g.dim - 1);
   }
   for (auto &g : st.kl) {
     if (!pow2(g.dim)) return false;
     nbk += ilog2(g.dim);
-    wmax = std::max({wmax, g.sa * (g.dim - 1), g.sb * (g.dim - 1)});
+    wa += g.sa * (g.dim - 1), wb += g.sb * (g.dim - 1);
   }
-  return nbc <= kSmallMaxBits && nbk <= kSmallMaxBits && wmax < (int64_t(1) << 30);
+  return nbc <= kSmallMaxBits && nbk <= kSmallMaxBits && std::max(wa, wb) < (int64_t(1) << 30);
 }
 
-// Hoist the small steps of section 0 (once per call) and of section 2 (once per
-// bitstring batch) whose inputs are available at the section's start (data, values
-// of earlier sections, bitstring tensors, or other such steps) to the front of
-// their section, grouped by dependency level (a level's steps are independent of
-// each other).  Steps reading slice-dependent views are left alone (their
-// addresses change per slice).  The order stays topological; liveness is computed
-// on the new order afterwards.
+// Items of a small step (waves that work on it).
+int small_items(const Step &st) {
+  int nbc = 0, nbk = 0;
+  for (auto &g : st.cl) nbc += ilog2(g.dim);
+  for (auto &g : st.kl) nbk += ilog2(g.dim);
+  return 1 << (nbc - small_len_bits(nbc, nbk));
+}
+
+// Whether an operand's slice-dependent offset fits an item's descriptor.
+bool small_terms_ok(const Value &v) {
+  if (v.var_terms.size() > (size_t)kSmallTerms) return false;
+  for (auto &t : v.var_terms)
+    if (t.first >= kSmallVars || t.second >= (int64_t(1) << 30)) return false;
+  return true;
+}
+
+// Steps alone on their level join the batched small steps only as part of a run of
+// levels: with at most kSmallRunItems items, next to another such level of the section
+// (a launch of its own is no faster with their items than with their own kernel).
+template <typename Steps, typename Get>
+void settle_lone(Steps &steps, Get step) {
+  struct Group {
+    size_t first, last;
+    int section, items;
+    bool small;
+  };
+  std::vector<Group> groups;
+  for (size_t i = 0; i < steps.size(); ++i) {
+    const int lv = steps[i].level;
+    const bool cont = i > 0 && lv >= 0 && steps[i - 1].level == lv;
+    if (!cont) groups.push_back({i, i, step(steps[i]).section, 0, lv >= 0});
+    groups.back().last = i;
+    if (lv >= 0) groups.back().items += small_items(step(steps[i]));
+  }
+  auto joins = [&](size_t g) { return groups[g].small && groups[g].items <= kSmallRunItems; };
+  std::vector<char> keep(groups.size(), 0);
+  for (size_t g = 0; g < groups.size(); ++g) {
+    if (!groups[g].small || groups[g].first != groups[g].last) continue;
+    const bool prev = g > 0 && groups[g - 1].section == groups[g].section && joins(g - 1);
+    const bool next = g + 1 < groups.size() && groups[g + 1].section == groups[g].section && joins(g + 1);
+    keep[g] = joins(g) && (prev || next);
+  }
+  for (size_t g = 0; g < groups.size(); ++g)
+    if (groups[g].small && groups[g].first == groups[g].last) {
+      steps[groups[g].first].lone = true;
+      if (!keep[g]) steps[groups[g].first].level = -1;
+    }
+}
+
+// Hoist the small steps of each section whose inputs are available at the section's start
+// (data, values of earlier sections, bitstring tensors, or other such steps) to the front
+// of their section, grouped by dependency level (a level's steps are independent of each
+// other); slice-dependent offsets are added on the device from the slice's variables.  A
+// small step that waits for a large one keeps its place, a level of its own.  The order
+// stays topological; liveness is computed on the new order afterwards.
 void level_small_steps(const Program &p, Lowered &L) {
   const size_t nn = p.nodes.size();
   std::vector<int> root(nn, -1), prod(nn, -1);
@@ -1599,48 +1647,69 @@ void level_small_steps(const Program &p, Lowered &L) {
     root[i] = (n.op == Op::View || n.op == Op::Save) ? root[n.ia] : (int)i;
   }
   for (size_t s = 0; s < L.steps.size(); ++s) prod[L.steps[s].node] = (int)s;
-  std::vector<int> level(L.steps.size(), -1);
-  int maxlev = -1;
-  for (size_t s = 0; s < L.steps.size(); ++s) {
-    const Step &st = L.steps[s];
-    if (!small_step(st)) continue;
-    if (!L.values[st.in_a].var_terms.empty() || !L.values[st.in_b].var_terms.empty()) continue;
-    int lv = 0;
-    bool ok = true;
-    for (int in : {st.in_a, st.in_b}) {
-      const int r = root[in];
-      if (r < 0) continue;
-      const int ps = prod[r];
-      if (ps < 0) continue;                               // data or bitstring output
-      if (L.steps[ps].section != st.section) continue;   // an earlier section's value
-      if (level[ps] < 0) {
-        ok = false;
-        break;
-      }
-      lv = std::max(lv, level[ps] + 1);
-    }
-    if (!ok) continue;
-    level[s] = lv;
-    maxlev = std::max(maxlev, lv);
-  }
-  if (maxlev < 0) return;
-  // levels are numbered per section; section 2's are offset past section 0's
-  const int off2 = maxlev + 1;
-  std::vector<int> count(2 * (maxlev + 1), 0);
+  std::vector<char> small(L.steps.size(), 0);
   for (size_t s = 0; s < L.steps.size(); ++s)
-    if (level[s] >= 0) count[level[s] + (L.steps[s].section == 2 ? off2 : 0)]++;
+    small[s] = small_step(L.steps[s]) && small_terms_ok(L.values[L.steps[s].in_a]) &&
+               small_terms_ok(L.values[L.steps[s].in_b]);
+  // level of each step that `may` run at its section's front; -1: not
+  auto levels = [&](auto may) {
+    std::vector<int> level(L.steps.size(), -1);
+    for (size_t s = 0; s < L.steps.size(); ++s) {
+      const Step &st = L.steps[s];
+      if (!may(s)) continue;
+      int lv = 0;
+      bool ok = true;
+      for (int in : {st.in_a, st.in_b}) {
+        const int r = root[in];
+        if (r < 0) continue;
+        const int ps = prod[r];
+        if (ps < 0) continue;                               // data or bitstring output
+        if (L.steps[ps].section != st.section) continue;   // an earlier section's value
+        if (level[ps] < 0) {
+          ok = false;
+          break;
+        }
+        lv = std::max(lv, level[ps] + 1);
+      }
+      if (ok) level[s] = lv;
+    }
+    return level;
+  };
+  {   // the launches of a pass were slice-dependent steps launched one by one
+    const std::vector<int> level = levels([&](size_t s) {
+      const Step &st = L.steps[s];
+      return small[s] && st.section != 1 && L.values[st.in_a].var_terms.empty() && L.values[st.in_b].var_terms.empty();
+    });
+    for (int sec = 0; sec < 3; ++sec) {
+      std::set<int> seen;
+      int64_t n = 0;
+      for (size_t s = 0; s < L.steps.size(); ++s)
+        if (L.steps[s].section == sec && (level[s] < 0 || seen.insert(level[s]).second)) ++n;
+      L.est_launches[sec] = n;
+    }
+  }
+  const std::vector<int> level = levels([&](size_t s) { return small[s] != 0; });
+  int key = 0;
   std::vector<Step> out;
   for (int sec : {0, 1, 2}) {
-    for (int lv = 0; lv <= maxlev; ++lv)
+    const int maxlev = level.empty() ? -1 : *std::max_element(level.begin(), level.end());
+    for (int lv = 0; lv <= maxlev; ++lv) {
+      bool any = false;
       for (size_t s = 0; s < L.steps.size(); ++s)
         if (L.steps[s].section == sec && level[s] == lv) {
-          const int key = lv + (sec == 2 ? off2 : 0);
           out.push_back(L.steps[s]);
-          out.back().level = count[key] > 1 ? key : -1;   // a lone step keeps its own kernel
+          out.back().level = key;
+          any = true;
         }
+      key += any;
+    }
     for (size_t s = 0; s < L.steps.size(); ++s)
-      if (L.steps[s].section == sec && level[s] < 0) out.push_back(L.steps[s]);
+      if (L.steps[s].section == sec && level[s] < 0) {
+        out.push_back(L.steps[s]);
+        out.back().level = small[s] ? key++ : -1;
+      }
   }
+  settle_lone(out, [](const Step &st) -> const Step & { return st; });
   L.steps = std::move(out);
 }
 
@@ -2181,9 +2250,8 @@ VjpLowered lower_vjp(const Program &p, int64_t batch, int precision, uint64_t fu
     std::vector<size_t> order(bv.size());
     for (size_t i = 0; i < order.size(); ++i) order[i] = i;
     std::stable_sort(order.begin(), order.end(), [&](size_t a, size_t b) { return lev[a] < lev[b]; });
-    std::vector<BwdStep> sorted;
-    std::map<int, int64_t> level_temp;
-    std::map<int, int> level_count;
+    std::vector<BwdStep> sorted, others;
+    int prev_lev = -1;
     std::set<std::pair<int, int>> level_cot;   // (level, cotangent buffer) added into by the level
     for (size_t i : order) {
       BwdStep b = std::move(bv[i]);
@@ -2194,19 +2262,17 @@ VjpLowered lower_vjp(const Program &p, int64_t batch, int precision, uint64_t fu
                               ((b.dest == Buf::Grad && key_uses[b.dest_key] == 1) ||
                                (b.dest == Buf::Cot && !level_cot.count({level_base + lev[i], b.dest_root})))));
       if (ok && !b.direct && b.dest == Buf::Cot) level_cot.insert({level_base + lev[i], b.dest_root});
-      if (ok) {
-        b.level = level_base + lev[i];
-        level_count[b.level]++;
-        if (!b.direct) {
-          b.temp_off = level_temp[b.level];
-          level_temp[b.level] += (b.add_elems + 31) / 32 * 32;
-          V.temp_elems = std::max(V.temp_elems, level_temp[b.level]);
-        }
+      if (ok) b.level = level_base + lev[i];
+      // a level's batched steps first, then its others (all independent of each other)
+      if (lev[i] != prev_lev) {
+        for (auto &o : others) sorted.push_back(std::move(o));
+        others.clear();
       }
-      sorted.push_back(std::move(b));
+      prev_lev = lev[i];
+      (ok ? sorted : others).push_back(std::move(b));
     }
-    for (auto &b : sorted)   // a lone step keeps its own launch
-      if (b.level >= 0 && level_count[b.level] < 2) b.level = -1, b.temp_off = 0;
+    for (auto &o : others) sorted.push_back(std::move(o));
+    settle_lone(sorted, [](const BwdStep &b) -> const Step & { return b.step; });
     bv = std::move(sorted);
     level_base += maxlev + 1;
   }

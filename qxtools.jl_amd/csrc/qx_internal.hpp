@@ -112,31 +112,44 @@ struct RadixArgs {
   int conj_a = 0, conj_b = 0;
 };
 
-// Small slice-free steps (gate-block building) run many per launch: one workgroup
-// per step, its bit weights read from a device table of these descriptors.
+// Small steps (gate-block building, and what is left of a tree near its leaves) run many
+// per launch as items of one wave: an item is 2^len consecutive C elements of a step, at
+// most 2^kSmallItemBits multiply-adds where the element count allows it.  Low C bits and,
+// where an item has fewer elements than lanes, low K bits are lane bits (K lanes lowest);
+// the other C bits (E) and K bits (T) are walked by a trip counter, T fastest.  All of an
+// item's offsets come from its descriptor, which the wave holds in two registers (word
+// l in lane l, word 64 + l in lane l of the second):
+//   0-5   A, B, C of the item        6  bit fields (small_pack)
+//   8-25  per lane bit: A, B and C offsets (elements)
+//   26-63 per trip bit: A and B increments (stride less those of the bits that turn zero)
+//   64-66 C offset of each E bit     67-76 slice terms: variables (a byte each), strides
 constexpr int kSmallMaxBits = 18;
-constexpr int kSmallChunk = 1024;   // most C elements per workgroup of a small-step batch
-constexpr int kSmallThreads = 256;  // lanes per workgroup of a small-step batch
+constexpr int kSmallItemBits = 9;
+constexpr int kSmallLaneBits = 6, kSmallTripBits = 19, kSmallEBits = 3, kSmallTerms = 4;
+constexpr int kSmallWords = 96;
+constexpr int kSmallVars = 32;      // slice variables a small step may depend on
+constexpr int kSmallThreads = 256;  // lanes per workgroup of a level's launch
+constexpr int kSmallRunThreads = 1024;   // lanes of the one workgroup of a run of levels
+// A level of at most this many items joins a run of levels that one workgroup of 16 waves
+// walks in one launch: three rounds of 16 items and a barrier cost less than a launch.
+constexpr int kSmallRunItems = 48;
 struct SmallDesc {
-  const void *A = nullptr, *B = nullptr;
-  void *C = nullptr;
-  int32_t nbc = 0, nbk = 0, conj_a = 0, conj_b = 0;
-  int32_t c0 = 0, c1 = 0;      // C elements [c0, c1) of this workgroup (a large C is split)
-  int32_t wa[kSmallMaxBits] = {0}, wb[kSmallMaxBits] = {0};   // C bits
-  int32_t ka[kSmallMaxBits] = {0}, kb[kSmallMaxBits] = {0};   // K bits
+  int32_t w[kSmallWords];
 };
-
-// Batched scatter-add of small temps into FP64 gradients or cotangent buffers:
-// dst[map(e)] += src[e], map(e) = sum of digit_j(e) * st[j] over the dims (first
-// fastest).
-struct AddDesc {
-  void *dst = nullptr;
-  const void *src = nullptr;
-  int64_t n = 0;
-  int32_t nd = 0;
-  int32_t dst_f64 = 1;   // destination FP64 (a gradient); else the plan's element type
-  int64_t dim[kSmallMaxBits] = {0}, st[kSmallMaxBits] = {0};
+// Values of the slice variables, passed with each launch.
+struct SmallVars {
+  int32_t v[kSmallVars] = {0};
 };
+inline int32_t small_pack(int lt, int lanes, int e, int t, int conj_a, int conj_b, int add, int f64, int na, int nb) {
+  return (int32_t)((uint32_t)lt | (uint32_t)lanes << 4 | (uint32_t)e << 8 | (uint32_t)t << 12 | (uint32_t)conj_a << 20 |
+                   (uint32_t)conj_b << 21 | (uint32_t)add << 22 | (uint32_t)f64 << 23 | (uint32_t)na << 24 |
+                   (uint32_t)nb << 28);
+}
+// log2 of an item's C elements for a step of nbc C bits and nbk K bits.
+inline int small_len_bits(int nbc, int nbk) {
+  const int l = kSmallItemBits - nbk;
+  return l < 0 ? 0 : l < nbc ? l : nbc;
+}
 
 // A chain of steps that each contract a small operand (a gate block: at most 2^10
 // elements) into one large tensor X, X_j = S_j . X_{j-1}, run as one pass over X:
@@ -321,7 +334,8 @@ struct Step {
   int64_t ws_elems = 0;    // workspace for K-split partials
   Kern kern = Kern::Bits;
   int section = 0;         // 0 shared slice-free, 1 shared per slice, 2 per bitstring batch
-  int level = -1;          // >= 0: small slice-free step run with the others of its level in one launch
+  int level = -1;          // >= 0: small step run with the others of its level in one launch
+  bool lone = false;       // its level holds no other step
   bool swapped = false;    // operands exchanged (in_a is the DSL's B): C = B.A, M and N traded
   BitArgs bits;            // Kern::Bits / Kern::Reduce
   GemmArgs gemm;           // Kern::Gemm
@@ -358,6 +372,9 @@ struct Lowered {
   int64_t ws_elems = 0;             // largest K-split workspace of any step
   int64_t out_elems = 0;            // elements of one output tensor incl. batch
   int64_t result_elems = 1;         // complex values per bitstring
+  // per section: launches of a pass were every slice-dependent or lone step a launch of
+  // its own (the size a call is held to for graph capture); -1: one per step
+  int64_t est_launches[3] = {-1, -1, -1};
 };
 
 // batch_last: lay the batched bitstring leg out slowest in bitstring-dependent
@@ -387,8 +404,9 @@ struct BwdStep {
   int dest_key = -1;          // data key (Grad)
   std::vector<int64_t> add_dims, add_strides;   // temp (dense) -> destination
   int64_t add_elems = 0;
-  int level = -1;             // >= 0: runs batched with the other small steps of its level
-  int64_t temp_off = 0;       // offset (elements) of its temp in the temp buffer
+  int level = -1;             // >= 0: runs batched with the other small steps of its level,
+                              // its add (if any) with it: no temp
+  bool lone = false;          // its level holds no other step
 };
 
 struct VjpLowered {
@@ -458,11 +476,13 @@ void launch_root_cot(int prec, void *dst, int64_t dep, int64_t batch, int64_t nv
 // root cotangent 2 * root value (the loss sum |amp|^2); amplitudes of the batch into `amp`
 void launch_root_cot_norm(int prec, void *dst, const void *val, int64_t dep, int64_t batch, int64_t nvalid,
                           int64_t relems, const int64_t *d_relem_off, double *amp, int64_t row0, void *stream);
-void launch_small_batch(int prec, const SmallDesc *d_desc, int n, void *stream);
-// Levels [0, nlevels) of small-step chunks in one workgroup: level L is the descriptors
-// [d_level_off[L], d_level_off[L + 1]), run after every earlier level.
-void launch_small_walk(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, void *stream);
-void launch_add_batch(int prec, const AddDesc *d_desc, int n, void *stream);
+// n independent items (one level), a wave each.
+void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVars &vars, void *stream);
+// Levels [0, nlevels) of items in one workgroup: level L is the descriptors
+// [d_level_off[L], d_level_off[L + 1]), run after every earlier level.  `walk`: the
+// instance named k_small_walk (a whole section, plan option small_walk).
+void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
+                      bool walk, void *stream);
 // bf16 split of n complex64 values: out holds four planar n-element bf16 arrays
 // (re hi, re lo, im hi, im lo); hi = x rounded to bf16 (nearest, ties to even),
 // lo = (x - hi) rounded likewise.

@@ -127,20 +127,24 @@ struct qx_plan {
     DevBuf desc;
     void *arena = nullptr;                  // arena base the descriptors point into
     std::vector<int> index;                 // per step: descriptor index, or -1
-    std::vector<int> count;                 // per step that starts a level: steps in the level
-    // one-workgroup walk of a section's levels (k_small_walk): per section, the offset
-    // of its level table in `walk` (device ints) and its level count (0: not walked)
+    std::vector<int> count;                 // per step that starts a level: items in the level
+    // level tables (device ints) of the runs of levels that one workgroup walks: per step
+    // that starts a run, its table's offset and its level count (0: a level of its own);
+    // `inside`: a later level of a run
     DevBuf walk;
+    std::vector<int> run_at, run_levels;
+    std::vector<char> inside;
+    // a whole section's levels (plan option small_walk): table offset, levels (0: not)
     int walk_at[3] = {0, 0, 0}, walk_levels[3] = {0, 0, 0};
   };
   std::map<const qx::Lowered *, SmallTable> small;   // per lowering (forward or pullback)
   // batched slice-free backward levels of one pullback lowering
   struct BwdTable {
-    DevBuf desc, adds, zeros;
+    DevBuf desc, walk, zeros;
     int zero0[3] = {0, 0, 0}, nzero[3] = {0, 0, 0};   // per section: its zero-fill ranges
     std::vector<char *> bases;              // arena, cot, temp, grad the tables point into
     std::vector<int> first[3];              // per section and backward step: its level's group, or -1
-    struct Group { int desc0, ndesc, add0, nadd; };
+    struct Group { int desc0, ndesc, run_at, run_levels, inside; };   // runs as in SmallTable
     std::vector<Group> groups;
   };
   std::map<const qx::VjpLowered *, BwdTable> bwd;
@@ -174,7 +178,7 @@ struct qx_plan {
     ampcot.release();
     ws.release();
     for (auto &kv : small) kv.second.desc.release(), kv.second.walk.release();
-    for (auto &kv : bwd) kv.second.desc.release(), kv.second.adds.release();
+    for (auto &kv : bwd) kv.second.desc.release(), kv.second.walk.release(), kv.second.zeros.release();
     for (auto e : events) (void)hipEventDestroy(e);
     for (auto e : tune_events) (void)hipEventDestroy(e);
     drop_graphs();
@@ -212,8 +216,10 @@ const qx::Lowered &ensure_lowered(qx_plan *P, int64_t batch, uint64_t fused = 0)
   if (it != P->lowered.end()) return it->second;
   qx::Lowered L = qx::lower(P->prog, batch, false, P->prec, fused, P->opt_chains != 0, P->opt_batch_last != 0);
   if (P->opt_kernel >= 0)
-    for (auto &st : L.steps)
+    for (auto &st : L.steps) {
+      if (st.lone) st.level = -1;   // a forced kernel runs every step of its own
       if (qx::force_kernel(st, P->prec, (int)P->opt_kernel)) L.ws_elems = std::max(L.ws_elems, st.ws_elems);
+    }
   if (P->opt_chain_variant >= 0)
     for (auto &st : L.steps) force_chain_variant(st, P->opt_chain_variant);
   size_t need = (size_t)L.arena_elems * P->esize();
@@ -425,97 +431,174 @@ void launch_step(qx_plan *P, const qx::Lowered &L, const qx::Step &st, void *A, 
   }
 }
 
-// Append x to a small-step descriptor table, its C split into workgroup ranges of
-// kSmallChunk elements; returns the number of descriptors added.
-int push_small(std::vector<qx::SmallDesc> &d, qx::SmallDesc x) {
-  // chunks of C (powers of two) sized for about 32 multiply-adds per lane of the
-  // workgroup: a chunk of fewer elements than lanes splits K over its lanes
-  const int nc = 1 << x.nbc;
-  const int64_t nk = int64_t(1) << x.nbk;
-  int len = qx::kSmallChunk;
-  while (len > 1 && len * nk > 32 * qx::kSmallThreads) len >>= 1;
-  len = std::min(len, nc);
-  int n = 0;
-  for (int c0 = 0; c0 < nc; c0 += len, ++n) {
-    x.c0 = c0;
-    x.c1 = c0 + len;
+// Append the items of a small step to a descriptor table: C = A.B stored, or added into
+// `C` through the C offsets `cw` of its bits (f64: an FP64 destination).  Returns their
+// number.
+int push_small(std::vector<qx::SmallDesc> &d, const qx::Step &st, const qx::Value *va, const qx::Value *vb,
+               const void *A, const void *B, void *C, size_t es, const std::vector<int64_t> *cw = nullptr,
+               bool f64 = false) {
+  struct Bit {
+    int64_t a, b, c;
+  };
+  std::vector<Bit> cb, kb;
+  for (auto &g : st.cl)
+    for (int64_t m = 1; m < g.dim; m <<= 1)
+      cb.push_back({g.sa * m, g.sb * m, cw ? cw->at(cb.size()) : int64_t(1) << cb.size()});
+  for (auto &g : st.kl)
+    for (int64_t m = 1; m < g.dim; m <<= 1) kb.push_back({g.sa * m, g.sb * m, 0});
+  const int nbc = (int)cb.size(), nbk = (int)kb.size();
+  if (nbc > qx::kSmallMaxBits || nbk > qx::kSmallMaxBits || (cw && (int)cw->size() != nbc))
+    throw qx::Error(QX_ERR_STATE, "internal: small step bits");
+  const int len = qx::small_len_bits(nbc, nbk), lc = std::min(len, qx::kSmallLaneBits);
+  const int lt = std::min(nbk, qx::kSmallLaneBits - lc), e = len - lc, t = nbk - lt;
+  if (e > qx::kSmallEBits || e + t > qx::kSmallTripBits) throw qx::Error(QX_ERR_STATE, "internal: small step item");
+  qx::SmallDesc x{};
+  int na = 0, nb = 0;
+  auto terms = [&](const qx::Value *v, int vars, int strides, int &n) {
+    if (!v) return;
+    for (auto &q : v->var_terms) {
+      if (n == qx::kSmallTerms || q.first >= qx::kSmallVars) throw qx::Error(QX_ERR_STATE, "internal: small step slices");
+      x.w[vars] |= q.first << (8 * n);
+      x.w[strides + n++] = (int32_t)q.second;
+    }
+  };
+  terms(va, 67, 69, na);
+  terms(vb, 68, 73, nb);
+  x.w[6] = qx::small_pack(lt, lc + lt, e, t, st.bits.conj_a, st.bits.conj_b, cw != nullptr, f64, na, nb);
+  for (int i = 0; i < lc + lt; ++i) {
+    const Bit &b = i < lt ? kb[i] : cb[i - lt];
+    x.w[8 + i] = (int32_t)b.a, x.w[14 + i] = (int32_t)b.b, x.w[20 + i] = (int32_t)b.c;
+  }
+  int64_t sa = 0, sb = 0;
+  for (int i = 0; i < e + t; ++i) {   // trip bits: K terms lowest, then elements
+    const Bit &b = i < t ? kb[lt + i] : cb[lc + i - t];
+    x.w[26 + i] = (int32_t)(b.a - sa), x.w[45 + i] = (int32_t)(b.b - sb);
+    sa += b.a, sb += b.b;
+  }
+  for (int i = 0; i < e; ++i) x.w[64 + i] = (int32_t)cb[lc + i].c;
+  const int items = 1 << (nbc - len);
+  for (int n = 0; n < items; ++n) {
+    int64_t oa = 0, ob = 0, oc = 0;
+    for (int i = len; i < nbc; ++i)
+      if ((n >> (i - len)) & 1) oa += cb[i].a, ob += cb[i].b, oc += cb[i].c;
+    auto put = [&](int w, const void *p, int64_t off) {
+      const uint64_t v = (uint64_t)(uintptr_t)p + (uint64_t)off;
+      x.w[w] = (int32_t)(uint32_t)v, x.w[w + 1] = (int32_t)(uint32_t)(v >> 32);
+    };
+    put(0, A, oa * (int64_t)es);
+    put(2, B, ob * (int64_t)es);
+    put(4, C, oc * (int64_t)(cw && f64 ? 16 : es));
     d.push_back(x);
   }
-  return n;
+  return items;
 }
 
-// Build and upload the descriptor table of L's batched small steps (slice-free, so
-// their operand addresses depend only on the arena and data buffers).
+// Runs of levels for one workgroup: consecutive levels of at most kSmallRunItems items
+// each.  `lv`: (first descriptor, items, section) of each level in order, (-1, 0, section)
+// for any other launch in between; the tables go to `tab`.  Returns per level its table's
+// offset and level count (0: launched alone), and whether it lies inside a run.
+struct LevelRun {
+  int at = 0, levels = 0;
+  bool inside = false;
+};
+std::vector<LevelRun> find_runs(const std::vector<std::array<int, 3>> &lv, std::vector<int> &tab) {
+  std::vector<LevelRun> r(lv.size());
+  for (size_t i = 0; i < lv.size();) {
+    size_t j = i;
+    while (j < lv.size() && lv[j][0] >= 0 && lv[j][1] <= qx::kSmallRunItems && lv[j][2] == lv[i][2] &&
+           (j == i || lv[j][0] == lv[j - 1][0] + lv[j - 1][1]))
+      ++j;
+    if (j - i >= 2) {
+      r[i].at = (int)tab.size();
+      r[i].levels = (int)(j - i);
+      for (size_t k = i; k < j; ++k) {
+        tab.push_back(lv[k][0]);
+        r[k].inside = k > i;
+      }
+      tab.push_back(lv[j - 1][0] + lv[j - 1][1]);
+    }
+    i = std::max(j, i + 1);
+  }
+  return r;
+}
+
+qx::SmallVars small_vars(const std::vector<int64_t> &varval) {
+  qx::SmallVars v;
+  for (size_t i = 0; i < varval.size() && i < (size_t)qx::kSmallVars; ++i) v.v[i] = (int32_t)varval[i];
+  return v;
+}
+
+// Build and upload the descriptor table of L's batched small steps (operand addresses at
+// the first slice; an item adds its slice's terms) and the level tables of its runs.
 void prepare_small(qx_plan *P, const qx::Lowered &L, const Bases &bs) {
   qx_plan::SmallTable &T = P->small[&L];
   if (T.arena == bs.arena && !T.index.empty()) return;
   std::vector<qx::SmallDesc> d;
-  T.index.assign(L.steps.size(), -1);
-  T.count.assign(L.steps.size(), 0);
+  const size_t ns = L.steps.size();
+  T.index.assign(ns, -1);
+  T.count.assign(ns, 0);
+  T.run_at.assign(ns, 0);
+  T.run_levels.assign(ns, 0);
+  T.inside.assign(ns, 0);
   const std::vector<int64_t> zero(P->prog.vars.size(), 0);
+  std::vector<std::array<int, 3>> lv;   // levels and other launches, in order
+  std::vector<int> at;                  // their first steps
   int first = -1;
-  for (size_t s = 0; s < L.steps.size(); ++s) {
+  for (size_t s = 0; s < ns; ++s) {
     const qx::Step &st = L.steps[s];
-    if (st.level < 0) continue;
-    if (first < 0 || L.steps[first].level != st.level) first = (int)s;
+    if (st.level < 0) {
+      lv.push_back({-1, 0, st.section});
+      at.push_back((int)s);
+      first = -1;
+      continue;
+    }
+    if (first < 0 || L.steps[first].level != st.level) {
+      first = (int)s;
+      lv.push_back({(int)d.size(), 0, st.section});
+      at.push_back(first);
+    }
     T.index[s] = (int)d.size();
-    qx::SmallDesc x;
-    x.A = value_ptr(P, L.values[st.in_a], zero, bs);
-    x.B = value_ptr(P, L.values[st.in_b], zero, bs);
-    x.C = value_ptr(P, L.values[st.node], zero, bs);
-    x.conj_a = st.bits.conj_a;
-    x.conj_b = st.bits.conj_b;
-    for (auto &g : st.cl)
-      for (int64_t m = 1; m < g.dim; m <<= 1) {
-        if (x.nbc >= qx::kSmallMaxBits) throw qx::Error(QX_ERR_STATE, "internal: small step bits");
-        x.wa[x.nbc] = (int32_t)(g.sa * m);
-        x.wb[x.nbc] = (int32_t)(g.sb * m);
-        ++x.nbc;
-      }
-    for (auto &g : st.kl)
-      for (int64_t m = 1; m < g.dim; m <<= 1) {
-        if (x.nbk >= qx::kSmallMaxBits) throw qx::Error(QX_ERR_STATE, "internal: small step bits");
-        x.ka[x.nbk] = (int32_t)(g.sa * m);
-        x.kb[x.nbk] = (int32_t)(g.sb * m);
-        ++x.nbk;
-      }
-    T.count[first] += push_small(d, x);
+    T.count[first] += push_small(d, st, &L.values[st.in_a], &L.values[st.in_b],
+                                 value_ptr(P, L.values[st.in_a], zero, bs), value_ptr(P, L.values[st.in_b], zero, bs),
+                                 value_ptr(P, L.values[st.node], zero, bs), P->esize());
+    lv.back()[1] = T.count[first];
   }
   if (!d.empty()) {
     T.desc.reserve(d.size() * sizeof(qx::SmallDesc));
     hip_check(hipMemcpy(T.desc.p, d.data(), d.size() * sizeof(qx::SmallDesc), hipMemcpyHostToDevice),
               "copy descriptors");
   }
-  // level tables of the sections whose small steps are few enough for one workgroup:
-  // at most 2^22 multiply-adds and 4096 chunks in all (the levels' descriptors are
-  // contiguous, in level order)
   std::vector<int> walk;
+  const std::vector<LevelRun> runs = find_runs(lv, walk);
+  for (size_t g = 0; g < runs.size(); ++g) {
+    T.run_at[at[g]] = runs[g].at;
+    T.run_levels[at[g]] = runs[g].levels;
+    T.inside[at[g]] = runs[g].inside;
+  }
+  // whole sections (plan option small_walk): levels at its front of at most 2^22
+  // multiply-adds and 2^14 items in all
   for (int sec = 0; sec < 3; ++sec) {
     T.walk_at[sec] = (int)walk.size();
     T.walk_levels[sec] = 0;
     std::vector<int> offs;
     double macs = 0;
-    int chunks = 0;
-    bool other_seen = false;   // a step of the section outside the levels, before a level
-    for (size_t s = 0; s < L.steps.size(); ++s) {
-      if (L.steps[s].section != sec) continue;
-      if (L.steps[s].level < 0) {
-        other_seen = true;
-        continue;
-      }
-      if (T.count[s] == 0) continue;
-      if (other_seen || (!offs.empty() && offs.back() != T.index[s])) {
-        offs.clear();   // levels of a section are contiguous; anything else keeps one launch per level
-        break;
-      }
-      if (offs.empty()) offs.push_back(T.index[s]);
-      for (int i = T.index[s]; i < T.index[s] + T.count[s]; ++i) {
-        macs += double(d[i].c1 - d[i].c0) * double(int64_t(1) << d[i].nbk);
-        ++chunks;
-      }
-      offs.push_back(T.index[s] + T.count[s]);
+    bool front = true;
+    for (size_t g = 0; g < lv.size() && front; ++g) {
+      if (lv[g][2] != sec) continue;
+      if (lv[g][0] < 0) break;
+      if (offs.empty()) offs.push_back(lv[g][0]);
+      front = offs.back() == lv[g][0];
+      if (front) offs.push_back(lv[g][0] + lv[g][1]);
+      macs += double(lv[g][1]) * double(1 << qx::kSmallItemBits);
     }
-    if (offs.size() >= 2 && macs <= double(int64_t(1) << 22) && chunks <= 4096) {
+    // a level after another launch of the section keeps the section's launches apart
+    bool later = false, other = false;
+    for (auto &l : lv)
+      if (l[2] == sec) {
+        later |= other && l[0] >= 0;
+        other |= l[0] < 0;
+      }
+    if (front && !later && offs.size() >= 2 && macs <= double(1 << 22)) {
       walk.insert(walk.end(), offs.begin(), offs.end());
       T.walk_levels[sec] = (int)offs.size() - 1;
     }
@@ -533,7 +616,8 @@ bool walks(const qx_plan *P, const qx_plan::SmallTable &T, int sec) {
   return P->opt_small_walk && T.walk_levels[sec] > 0;
 }
 
-void run_small_walk(qx_plan *P, const qx::Lowered &L, size_t s, int sec, bool timed = true) {
+void run_small_walk(qx_plan *P, const qx::Lowered &L, size_t s, int sec, const std::vector<int64_t> &varval,
+                    bool timed = true) {
   hipStream_t stream = P->ctx->stream;
   const qx_plan::SmallTable &T = P->small.at(&L);
   size_t ev = 0;
@@ -548,13 +632,14 @@ void run_small_walk(qx_plan *P, const qx::Lowered &L, size_t s, int sec, bool ti
     P->event_step.push_back((int)s);
     hip_check(hipEventRecord(P->events[2 * ev], stream), "hipEventRecord");
   }
-  qx::launch_small_walk(P->prec, (const qx::SmallDesc *)T.desc.p, (const int *)T.walk.p + T.walk_at[sec],
-                        T.walk_levels[sec], stream);
+  qx::launch_small_run(P->prec, (const qx::SmallDesc *)T.desc.p, (const int *)T.walk.p + T.walk_at[sec],
+                       T.walk_levels[sec], small_vars(varval), true, stream);
   if (timed) hip_check(hipEventRecord(P->events[2 * ev + 1], stream), "hipEventRecord");
 }
 
-// Launch the level of batched small steps that starts at step s.
-void run_small_level(qx_plan *P, const qx::Lowered &L, size_t s, bool timed = true) {
+// Launch the level of batched small steps, or the run of levels, that starts at step s.
+void run_small_level(qx_plan *P, const qx::Lowered &L, size_t s, const std::vector<int64_t> &varval,
+                     bool timed = true) {
   hipStream_t stream = P->ctx->stream;
   const qx_plan::SmallTable &T = P->small.at(&L);
   size_t ev = 0;
@@ -569,8 +654,11 @@ void run_small_level(qx_plan *P, const qx::Lowered &L, size_t s, bool timed = tr
     P->event_step.push_back((int)s);
     hip_check(hipEventRecord(P->events[2 * ev], stream), "hipEventRecord");
   }
-  const qx::SmallDesc *d = (const qx::SmallDesc *)T.desc.p + T.index[s];
-  qx::launch_small_batch(P->prec, d, T.count[s], stream);
+  if (T.run_levels[s] > 0)
+    qx::launch_small_run(P->prec, (const qx::SmallDesc *)T.desc.p, (const int *)T.walk.p + T.run_at[s],
+                         T.run_levels[s], small_vars(varval), false, stream);
+  else
+    qx::launch_small_batch(P->prec, (const qx::SmallDesc *)T.desc.p + T.index[s], T.count[s], small_vars(varval), stream);
   if (timed) hip_check(hipEventRecord(P->events[2 * ev + 1], stream), "hipEventRecord");
 }
 
@@ -746,9 +834,10 @@ void slice_values(const qx_plan *P, uint64_t fused, int64_t sl, std::vector<int6
   }
 }
 
-// Launches of one section of a lowered program per pass: unbatched steps, plus one
-// per level of batched small steps.
+// Launches of one section of a lowered program per pass, at most (Lowered::est_launches:
+// runs of levels and slice-dependent small steps take fewer).
 int64_t section_launches(const qx::Lowered &L, int sec) {
+  if (L.est_launches[sec] >= 0) return L.est_launches[sec];
   int64_t n = 0;
   std::set<int> levels;
   for (auto &st : L.steps)
@@ -802,13 +891,13 @@ void enqueue_amplitudes(qx_plan *P, const qx::Lowered &L, uint64_t fused, int64_
     bool walked = false;
     for (size_t s = 0; s < L.steps.size(); ++s) {
       if (L.steps[s].section != sec) continue;
-      if (L.steps[s].level >= 0) {   // batched small steps: one launch per level, or one walk
+      if (L.steps[s].level >= 0) {   // batched small steps: one launch per level or run of levels, or one walk
         if (ST.count[s] == 0) continue;
-        if (!walks(P, ST, sec)) {
-          run_small_level(P, L, s, timed);
-        } else if (!walked) {
-          run_small_walk(P, L, s, sec, timed);
+        if (walks(P, ST, sec)) {
+          if (!walked) run_small_walk(P, L, s, sec, varval, timed);
           walked = true;
+        } else if (!ST.inside[s]) {
+          run_small_level(P, L, s, varval, timed);
         }
         continue;
       }
@@ -1256,9 +1345,15 @@ const qx::VjpLowered &ensure_vjp(qx_plan *P, int64_t batch, uint64_t fused) {
     auto force = [&](qx::Step &st) {
       if (qx::force_kernel(st, P->prec, (int)P->opt_kernel)) V.fwd.ws_elems = std::max(V.fwd.ws_elems, st.ws_elems);
     };
-    for (auto &st : V.fwd.steps) force(st);
+    for (auto &st : V.fwd.steps) {
+      if (st.lone) st.level = -1;
+      force(st);
+    }
     for (auto &sec : V.bsteps)
-      for (auto &b : sec) force(b.step);
+      for (auto &b : sec) {
+        if (b.lone) b.level = -1;
+        force(b.step);
+      }
   }
   if (P->opt_chain_variant >= 0)
     for (auto &st : V.fwd.steps) force_chain_variant(st, P->opt_chain_variant);
@@ -1355,13 +1450,13 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
     for (size_t s = 0; s < L.steps.size(); ++s) {
       const qx::Step &st = L.steps[s];
       if (st.section != sec) continue;
-      if (st.level >= 0) {   // batched small steps: one launch per level, or one walk
+      if (st.level >= 0) {   // batched small steps: one launch per level or run of levels, or one walk
         if (ST.count[s] == 0) continue;
-        if (!walks(P, ST, sec)) {
-          run_small_level(P, L, s);
-        } else if (!walked) {
-          run_small_walk(P, L, s, sec);
+        if (walks(P, ST, sec)) {
+          if (!walked) run_small_walk(P, L, s, sec, varval);
           walked = true;
+        } else if (!ST.inside[s]) {
+          run_small_level(P, L, s, varval);
         }
         continue;
       }
@@ -1377,7 +1472,7 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
     const bool xa = b.x == cn.ia;
     A = xa ? value_ptr(P, cv, varval, bs) : value_ptr(P, L.values[cn.ia], varval, bs);
     B = xa ? value_ptr(P, L.values[cn.ib], varval, bs) : value_ptr(P, cv, varval, bs);
-    C = b.direct ? value_ptr(P, V.cot[b.x], varval, bs) : (void *)(bs.temp + b.temp_off * es);
+    C = b.direct ? value_ptr(P, V.cot[b.x], varval, bs) : (void *)bs.temp;
   };
   // descriptor tables of the batched backward levels (sections 0 and 2; their
   // operands have no slice-dependent offsets)
@@ -1386,62 +1481,61 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
     std::vector<char *> bases = {bs.arena, bs.cot, bs.temp, (char *)P->grad.p};
     if (BT.bases != bases) {
       std::vector<qx::SmallDesc> d;
-      std::vector<qx::AddDesc> ad;
+      std::vector<int> walk;
       BT.groups.clear();
       for (int sec = 0; sec < 3; ++sec) {
         const auto &bv = V.bsteps[sec];
         BT.first[sec].assign(bv.size(), -1);
+        std::vector<std::array<int, 3>> lv;   // the section's levels and other launches
+        std::vector<int> group;               // their groups (-1: another launch)
         int cur_level = -1;
         for (size_t i = 0; i < bv.size(); ++i) {
           const qx::BwdStep &b = bv[i];
-          if (b.level < 0) continue;
+          if (b.level < 0) {
+            lv.push_back({-1, 0, sec});
+            group.push_back(-1);
+            cur_level = -1;
+            continue;
+          }
           if (b.level != cur_level) {   // the level's first batched step launches the group
             cur_level = b.level;
-            BT.groups.push_back({(int)d.size(), 0, (int)ad.size(), 0});
+            BT.groups.push_back({(int)d.size(), 0, 0, 0, 0});
             BT.first[sec][i] = (int)BT.groups.size() - 1;
+            lv.push_back({(int)d.size(), 0, sec});
+            group.push_back(BT.first[sec][i]);
           }
           auto &g = BT.groups.back();
-          qx::SmallDesc x;
           void *A, *B, *C;
           bwd_ptrs(b, A, B, C);
-          x.A = A, x.B = B, x.C = C;
-          x.conj_a = b.step.bits.conj_a;
-          x.conj_b = b.step.bits.conj_b;
-          for (auto &l : b.step.cl)
-            for (int64_t m = 1; m < l.dim; m <<= 1)
-              x.wa[x.nbc] = (int32_t)(l.sa * m), x.wb[x.nbc] = (int32_t)(l.sb * m), ++x.nbc;
-          for (auto &l : b.step.kl)
-            for (int64_t m = 1; m < l.dim; m <<= 1)
-              x.ka[x.nbk] = (int32_t)(l.sa * m), x.kb[x.nbk] = (int32_t)(l.sb * m), ++x.nbk;
-          g.ndesc += push_small(d, x);
-          if (!b.direct) {
-            qx::AddDesc a;
-            a.src = C;
+          if (b.direct) {
+            g.ndesc += push_small(d, b.step, nullptr, nullptr, A, B, C, P->esize());
+          } else {   // added into a gradient or cotangent through the view's offsets and strides
             const int64_t xoff = value_offset(L.values[b.x], varval);
-            if (b.dest == qx::Buf::Grad) {
-              a.dst = (char *)P->grad.p + (key_off[b.dest_key] + xoff) * 16;
-            } else {
-              a.dst = bs.cot + (V.cot[b.dest_root].slot + xoff) * es;
-              a.dst_f64 = P->prec == QX_C128;
-            }
-            a.n = b.add_elems;
-            a.nd = (int32_t)b.add_dims.size();
-            for (int j = 0; j < a.nd; ++j) a.dim[j] = b.add_dims[j], a.st[j] = b.add_strides[j];
-            ad.push_back(a);
-            g.nadd++;
+            const bool grad_dst = b.dest == qx::Buf::Grad;
+            void *dst = grad_dst ? (void *)((char *)P->grad.p + (key_off[b.dest_key] + xoff) * 16)
+                                 : (void *)(bs.cot + (V.cot[b.dest_root].slot + xoff) * es);
+            std::vector<int64_t> cw;
+            for (size_t j = 0; j < b.add_dims.size(); ++j)
+              for (int64_t m = 1; m < b.add_dims[j]; m <<= 1) cw.push_back(b.add_strides[j] * m);
+            g.ndesc += push_small(d, b.step, nullptr, nullptr, A, B, dst, P->esize(), &cw, grad_dst || P->prec == QX_C128);
           }
+          lv.back()[1] = g.ndesc;
         }
+        const std::vector<LevelRun> runs = find_runs(lv, walk);
+        for (size_t k = 0; k < runs.size(); ++k)
+          if (group[k] >= 0) {
+            auto &g = BT.groups[group[k]];
+            g.run_at = runs[k].at, g.run_levels = runs[k].levels, g.inside = runs[k].inside;
+          }
       }
       if (!d.empty()) {
         BT.desc.reserve(d.size() * sizeof(qx::SmallDesc));
         hip_check(hipMemcpy(BT.desc.p, d.data(), d.size() * sizeof(qx::SmallDesc), hipMemcpyHostToDevice), "copy");
       }
-      if (!ad.empty()) {
-        BT.adds.reserve(ad.size() * sizeof(qx::AddDesc));
-        hip_check(hipMemcpy(BT.adds.p, ad.data(), ad.size() * sizeof(qx::AddDesc), hipMemcpyHostToDevice), "copy");
+      if (!walk.empty()) {
+        BT.walk.reserve(walk.size() * sizeof(int));
+        hip_check(hipMemcpy(BT.walk.p, walk.data(), walk.size() * sizeof(int), hipMemcpyHostToDevice), "copy");
       }
-      // zero fills of the accumulating cotangents: one launch per section, ranges of
-      // at most 64 KiB per workgroup
       std::vector<int64_t> zr;
       for (int sec = 0; sec < 3; ++sec) {
         BT.zero0[sec] = (int)(zr.size() / 2);
@@ -1466,12 +1560,16 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   auto run_bwd = [&](int sec) {
     for (size_t bi = 0; bi < V.bsteps[sec].size(); ++bi) {
       const qx::BwdStep &b = V.bsteps[sec][bi];
-      if (b.level >= 0) {   // batched level: contractions, then adds into gradients
-        if (BT.first[sec][bi] >= 0) {
-          const auto &g = BT.groups[BT.first[sec][bi]];
-          qx::launch_small_batch(P->prec, (const qx::SmallDesc *)BT.desc.p + g.desc0, g.ndesc, stream);
-          qx::launch_add_batch(P->prec, (const qx::AddDesc *)BT.adds.p + g.add0, g.nadd, stream);
-        }
+      if (b.level >= 0) {   // batched level, or a run of levels: contractions and their adds
+        const int gi = BT.first[sec][bi];
+        if (gi < 0 || BT.groups[gi].inside) continue;
+        const auto &g = BT.groups[gi];
+        const qx::SmallDesc *d = (const qx::SmallDesc *)BT.desc.p;
+        if (g.run_levels > 0)
+          qx::launch_small_run(P->prec, d, (const int *)BT.walk.p + g.run_at, g.run_levels, qx::SmallVars(), false,
+                               stream);
+        else
+          qx::launch_small_batch(P->prec, d + g.desc0, g.ndesc, qx::SmallVars(), stream);
         continue;
       }
       const qx::Node &cn = P->prog.nodes[b.step.node];

@@ -519,46 +519,60 @@ void launch_root_cot_norm(int prec, void *dst, const void *val, int64_t dep, int
   });
 }
 
-void launch_small_batch(int prec, const SmallDesc *d_desc, int n, void *stream) {
+// Reach of one item from its descriptor, as the kernel decodes it.
+void check_small(int prec, const SmallDesc &d, const SmallVars &vars) {
   const size_t es = esize(prec);
+  auto ptr = [&](int i) { return (const char *)((uint64_t)(uint32_t)d.w[i] | (uint64_t)(uint32_t)d.w[i + 1] << 32); };
+  const uint32_t p = (uint32_t)d.w[6];
+  const int lt = p & 15, lanes = (p >> 4) & 15, e = (p >> 8) & 15, t = (p >> 12) & 31;
+  const int na = (p >> 24) & 15, nb = (p >> 28) & 15;
+  if (lanes > kSmallLaneBits || lt > lanes || e > kSmallEBits || e + t > kSmallTripBits || na > kSmallTerms || nb > kSmallTerms)
+    violation("small-step descriptor out of range");
+  long double ra = 1, rb = 1, rc = 1;
+  for (int b = 0; b < kSmallLaneBits; ++b) {
+    if (d.w[8 + b] < 0 || d.w[14 + b] < 0 || d.w[20 + b] < 0) violation("small-step lane offset");
+    if (b >= lanes && (d.w[8 + b] || d.w[14 + b] || d.w[20 + b])) violation("small-step idle lane offset");
+    ra += d.w[8 + b], rb += d.w[14 + b], rc += d.w[20 + b];
+  }
+  int64_t sa = 0, sb = 0;
+  for (int b = 0; b < kSmallTripBits; ++b) {   // increments back to strides
+    const int64_t wa = d.w[26 + b] + sa, wb = d.w[45 + b] + sb;
+    if (b >= e + t) {
+      if (d.w[26 + b] || d.w[45 + b]) violation("small-step idle trip bit");
+      continue;
+    }
+    if (wa < 0 || wb < 0) violation("small-step trip stride");
+    sa += wa, sb += wb;
+  }
+  for (int b = 0; b < kSmallEBits; ++b) {
+    if (b >= e && d.w[64 + b]) violation("small-step idle element bit");
+    rc += d.w[64 + b];
+  }
+  ra += sa, rb += sb;
+  int64_t oa = 0, ob = 0;
+  for (int q = 0; q < na; ++q) oa += (int64_t)vars.v[(d.w[67] >> (8 * q)) & 31] * d.w[69 + q];
+  for (int q = 0; q < nb; ++q) ob += (int64_t)vars.v[(d.w[68] >> (8 * q)) & 31] * d.w[73 + q];
+  need(ptr(0) + oa * (int64_t)es, ra * es, "small-step A");
+  need(ptr(2) + ob * (int64_t)es, rb * es, "small-step B");
+  need(ptr(4), rc * ((p >> 22) & 1 && (p >> 23) & 1 ? 16 : es), "small-step C");
+}
+
+void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVars &vars, void *stream) {
   launch(stream, [=]() {
     need(d_desc, (long double)n * sizeof(SmallDesc), "small-step descriptors");
-    for (int i = 0; i < n; ++i) {
-      const SmallDesc &d = d_desc[i];
-      if (d.nbc > kSmallMaxBits || d.nbk > kSmallMaxBits || d.c0 < 0 || d.c1 <= d.c0 || d.c1 > (1 << d.nbc))
-        violation("small-step descriptor out of range");
-      need(d.A, (sum_n(d.wa, d.nbc) + sum_n(d.ka, d.nbk) + 1) * es, "small-step A");
-      need(d.B, (sum_n(d.wb, d.nbc) + sum_n(d.kb, d.nbk) + 1) * es, "small-step B");
-      need(d.C, (long double)d.c1 * es, "small-step C");
-    }
+    for (int i = 0; i < n; ++i) check_small(prec, d_desc[i], vars);
   });
 }
 
-void launch_small_walk(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, void *stream) {
+void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
+                      bool, void *stream) {
   launch(stream, [=]() {
     need(d_level_off, (long double)(nlevels + 1) * 4, "level table");
     for (int L = 0; L < nlevels; ++L)
-      if (d_level_off[L + 1] < d_level_off[L]) violation("level table not increasing");
-  });
-  if (nlevels > 0)   // the chunks themselves: as a batch of every level's descriptors
-    submit((hipStream_t)stream, [=]() {
-      const int n = d_level_off[nlevels] - d_level_off[0];
-      launch_small_batch(prec, d_desc + d_level_off[0], n, nullptr);
-    });
-}
-
-void launch_add_batch(int prec, const AddDesc *d_desc, int n, void *stream) {
-  const size_t es = esize(prec);
-  launch(stream, [=]() {
-    need(d_desc, (long double)n * sizeof(AddDesc), "add descriptors");
-    for (int i = 0; i < n; ++i) {
-      const AddDesc &d = d_desc[i];
-      if (d.nd < 0 || d.nd > kSmallMaxBits) violation("add descriptor out of range");
-      long double rd = 1;
-      for (int j = 0; j < d.nd; ++j) rd += (long double)(d.dim[j] - 1) * d.st[j];
-      need(d.dst, rd * (d.dst_f64 ? 16 : es), "batched add destination");
-      need(d.src, (long double)d.n * es, "batched add source");
-    }
+      if (d_level_off[L + 1] <= d_level_off[L]) violation("level table not increasing");
+    // the kernel reads descriptors from the table's start by absolute index
+    need(d_desc, (long double)d_level_off[nlevels] * sizeof(SmallDesc), "small-step descriptors");
+    for (int i = d_level_off[0]; i < d_level_off[nlevels]; ++i) check_small(prec, d_desc[i], vars);
   });
 }
 
