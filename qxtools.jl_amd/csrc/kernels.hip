@@ -2508,32 +2508,83 @@ __global__ __launch_bounds__(kChainThreads) void k_contract_chain(const typename
 }
 
 // ---------------------------------------------------------------------------
-// Small steps: items of one wave each (SmallDesc).  Bound by latency alone: a level's
-// arithmetic is a few multiply-adds per lane, its time the descriptor, the operand loads
-// and the launch.  So the descriptor of a wave's next item is loaded (one word per lane)
-// while it works on the current one, across levels too, and read by lane index; offsets
-// are a lane part and wave-uniform parts; up to eight terms' operands are in flight at
-// once; K lanes are summed by shuffles, so no item needs a barrier.
+// Small steps: items of one wave each (SmallDesc).  A level's arithmetic is a few
+// multiply-adds per lane; its time is the issue of an item's instructions (four waves of a
+// SIMD share it, a lone wave takes four cycles per instruction), then the latency of its
+// operands.  So the descriptor of a wave's next item is loaded (one word per lane) while it
+// works on the current one, across levels too, and read by lane index; a term's address is
+// a wave-uniform 64-bit base, formed by the scalar unit, plus a 32-bit lane part that all
+// terms share; an item's element and term counts are template parameters, so all operands
+// (up to eight terms) are loaded by straight-line code; K lanes are summed by lane
+// permutes, so no item needs a barrier.  3x3 depth 16, 39 levels of one run: 91 us with
+// per-lane addresses, branches per term and LDS shuffles, 76 us so; a level of one or two
+// items 0.6 to 0.9 us, one of sixteen 512-product items 2.7, bound by the 16 bytes per lane
+// and operand that every product loads (64 bytes a cycle).
+template <typename T> struct SmallGlobal;
+template <> struct SmallGlobal<double> {
+  typedef double V __attribute__((ext_vector_type(2)));
+  static constexpr int shift = 4;
+};
+template <> struct SmallGlobal<float> {
+  typedef float V __attribute__((ext_vector_type(2)));
+  static constexpr int shift = 3;
+};
+template <typename V>
+__device__ __forceinline__ V small_load(uint64_t base, uint32_t off) {
+  typedef const __attribute__((address_space(1))) char *P;
+  return *(const __attribute__((address_space(1))) V *)((P)base + off);
+}
+template <typename V>
+__device__ __forceinline__ void small_store(uint64_t base, uint32_t off, V v) {
+  typedef __attribute__((address_space(1))) char *P;
+  *(__attribute__((address_space(1))) V *)((P)base + off) = v;
+}
 
-// Terms f = 0 .. F-1 of an item, U at a time: element f >> t, K term f & (2^t - 1).
-// `prefetch` runs once the first terms' loads are issued: loads return in order, so one
-// issued ahead of them would hold them up.
-template <typename T, int U, typename Prefetch>
-__device__ __forceinline__ void small_terms(int32_t d0, int32_t d1, const typename Vec<T>::type *A,
-                                            const typename Vec<T>::type *B, void *C, int32_t oa, int32_t ob, int32_t oc,
-                                            int32_t pack, bool store, Prefetch &&prefetch) {
-  using V = typename Vec<T>::type;
-  constexpr int LU = U == 8 ? 3 : U == 4 ? 2 : U == 2 ? 1 : 0;
-  const int lt = pack & 15, nt = 1 << ((pack >> 12) & 31), nf = nt << ((pack >> 8) & 15);
-  const int conj_a = (pack >> 20) & 1, conj_b = (pack >> 21) & 1;
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float x) {
+  return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xf, 0xf, false));
+}
+template <int CTRL>
+__device__ __forceinline__ double dpp_add(double x) {
+  return x + __hiloint2double(__builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xf, 0xf, false),
+                              __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xf, 0xf, false));
+}
+// Sum over the lanes that differ in the low lt lane bits (each lane gets it): neighbours
+// and pairs within four lanes, then, equal within those, the mirrored half rows and rows.
+template <typename V>
+__device__ __forceinline__ void small_lane_sum(V &v, int lt) {
+  if (lt > 0) v.x = dpp_add<0xB1>(v.x), v.y = dpp_add<0xB1>(v.y);
+  if (lt > 1) v.x = dpp_add<0x4E>(v.x), v.y = dpp_add<0x4E>(v.y);
+  if (lt > 2) v.x = dpp_add<0x141>(v.x), v.y = dpp_add<0x141>(v.y);
+  if (lt > 3) v.x = dpp_add<0x140>(v.x), v.y = dpp_add<0x140>(v.y);
+  if (lt > 4) v.x += __shfl_xor(v.x, 16, 64), v.y += __shfl_xor(v.y, 16, 64);
+  if (lt > 5) v.x += __shfl_xor(v.x, 32, 64), v.y += __shfl_xor(v.y, 32, 64);
+}
+
+// 2^LE elements per lane of 2^LT K terms each, or (LOOP) one element of 2^t >= 2^LT terms,
+// 2^LT at a time.  `prefetch` runs once the first terms' loads are issued: loads return in
+// order, so one issued ahead of them would hold them up.
+template <typename T, int LE, int LT, bool LOOP, typename Prefetch>
+__device__ __forceinline__ void small_terms(int32_t d0, int32_t d1, uint64_t A, uint64_t B, uint64_t C, uint32_t oa,
+                                            uint32_t ob, uint32_t oc, int32_t pack, bool store, Prefetch &&prefetch) {
+  using G = SmallGlobal<T>;
+  using V = typename G::V;
+  constexpr int LU = LE + LT, U = 1 << LU;
+  const uint32_t sign_a = (uint32_t)((pack >> 20) & 1) << 31, sign_b = (uint32_t)((pack >> 21) & 1) << 31;
   auto word = [&](int i) { return __builtin_amdgcn_readlane(i < 64 ? d0 : d1, i & 63); };
-  // offsets of the U terms of a trip from the first of its increments
-  int32_t ua[U], ub[U];
+  auto flip = [](T x, uint32_t s) -> T {
+    if constexpr (sizeof(T) == 8)
+      return __hiloint2double((int)((uint32_t)__double2hiint(x) ^ s), __double2loint(x));
+    else
+      return __uint_as_float(__float_as_uint(x) ^ s);
+  };
+  // byte offsets of the U terms from the first, of its increments
+  int64_t ua[U], ub[U];
   {
-    int32_t wa[3] = {0, 0, 0}, wb[3] = {0, 0, 0}, sa = 0, sb = 0;
+    int64_t wa[3] = {0, 0, 0}, wb[3] = {0, 0, 0}, sa = 0, sb = 0;
 #pragma unroll
     for (int b = 0; b < LU; ++b) {
-      wa[b] = word(26 + b) + sa, wb[b] = word(45 + b) + sb;
+      wa[b] = ((int64_t)word(26 + b) << G::shift) + sa, wb[b] = ((int64_t)word(45 + b) << G::shift) + sb;
       sa += wa[b], sb += wb[b];
     }
 #pragma unroll
@@ -2542,42 +2593,63 @@ __device__ __forceinline__ void small_terms(int32_t d0, int32_t d1, const typena
       ub[u] = (u & 1 ? wb[0] : 0) + (u & 2 ? wb[1] : 0) + (u & 4 ? wb[2] : 0);
     }
   }
-  V acc{0, 0};
-  int e = 0;
-  for (int f0 = 0; f0 < nf; f0 += U) {
+  const int trips = LOOP ? 1 << (((pack >> 12) & 31) - LT) : 1;
+  V acc[1 << LE];
+#pragma unroll
+  for (int e = 0; e < (1 << LE); ++e) acc[e] = V{0, 0};
+  for (int f = 0; f < trips; ++f) {
     V av[U], bv[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) av[u] = A[oa + ua[u]], bv[u] = B[ob + ub[u]];
-    if (f0 == 0) prefetch();
-    if (f0 + U < nf) {   // the next trip's first term: one increment, plus what this trip's low bits hold
-      const int z = __ffs(f0 + U) - 1;
-      oa += __builtin_amdgcn_readlane(d0, 26 + z) + ua[U - 1];
-      ob += __builtin_amdgcn_readlane(d0, 45 + z) + ub[U - 1];
+    for (int u = 0; u < U; ++u) {
+      av[u] = small_load<V>(A + (uint64_t)ua[u], oa);
+      bv[u] = small_load<V>(B + (uint64_t)ub[u], ob);
+    }
+    if (!LOOP || f == 0) prefetch();
+    if (LOOP && f + 1 < trips) {   // the next trip's first term: one increment, plus what this trip's low bits hold
+      const int z = __ffs(f + 1) - 1 + LT;
+      A += (uint64_t)(((int64_t)__builtin_amdgcn_readlane(d0, 26 + z) << G::shift) + ua[U - 1]);
+      B += (uint64_t)(((int64_t)__builtin_amdgcn_readlane(d0, 45 + z) << G::shift) + ub[U - 1]);
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      cmac<T>(acc, av[u], bv[u], conj_a, conj_b);
-      if (((f0 + u + 1) & (nt - 1)) == 0) {   // element e is complete
-        for (int k = 1; k < (1 << lt); k <<= 1) {
-          acc.x += __shfl_xor(acc.x, k, 64);
-          acc.y += __shfl_xor(acc.y, k, 64);
-        }
-        const int32_t o = oc + (e & 1 ? word(64) : 0) + (e & 2 ? word(65) : 0) + (e & 4 ? word(66) : 0);
-        if (store) {
-          if (!((pack >> 22) & 1)) {
-            ((V *)C)[o] = acc;
-          } else if ((pack >> 23) & 1) {   // add into an FP64 gradient
-            double2 *dst = (double2 *)C + o;
-            dst->x += (double)acc.x;
-            dst->y += (double)acc.y;
-          } else {                         // add into a cotangent buffer
-            V *dst = (V *)C + o;
-            dst->x += acc.x;
-            dst->y += acc.y;
-          }
-        }
-        acc = V{0, 0};
-        ++e;
+      const T ax = av[u].x, ay = flip(av[u].y, sign_a), bx = bv[u].x, by = flip(bv[u].y, sign_b);
+      V &c = acc[u >> LT];
+      c.x = fma(ax, bx, c.x);
+      c.x = fma(-ay, by, c.x);
+      c.y = fma(ax, by, c.y);
+      c.y = fma(ay, bx, c.y);
+    }
+  }
+  if (LE == 0) small_lane_sum(acc[0], pack & 15);   // (K lanes only with one element per lane)
+  auto element = [&](int e) {
+    return (int64_t)((e & 1 ? word(64) : 0) + (e & 2 ? word(65) : 0) + (e & 4 ? word(66) : 0));
+  };
+  if (!((pack >> 22) & 1)) {
+    if (store) {
+#pragma unroll
+      for (int e = 0; e < (1 << LE); ++e) small_store<V>(C + (uint64_t)(element(e) << G::shift), oc, acc[e]);
+    }
+  } else if ((pack >> 23) & 1) {   // add into an FP64 gradient
+    typedef double D __attribute__((ext_vector_type(2)));
+    if (store) {
+      D d[1 << LE];
+#pragma unroll
+      for (int e = 0; e < (1 << LE); ++e) d[e] = small_load<D>(C + (uint64_t)(element(e) << 4), oc);
+#pragma unroll
+      for (int e = 0; e < (1 << LE); ++e) {
+        d[e].x += (double)acc[e].x, d[e].y += (double)acc[e].y;
+        small_store<D>(C + (uint64_t)(element(e) << 4), oc, d[e]);
+      }
+    }
+  } else {                         // add into a cotangent buffer
+    if (store) {
+      V d[1 << LE];
+#pragma unroll
+      for (int e = 0; e < (1 << LE); ++e) d[e] = small_load<V>(C + (uint64_t)(element(e) << G::shift), oc);
+#pragma unroll
+      for (int e = 0; e < (1 << LE); ++e) {
+        d[e].x += acc[e].x, d[e].y += acc[e].y;
+        small_store<V>(C + (uint64_t)(element(e) << G::shift), oc, d[e]);
       }
     }
   }
@@ -2585,32 +2657,51 @@ __device__ __forceinline__ void small_terms(int32_t d0, int32_t d1, const typena
 
 template <typename T, typename Prefetch>
 __device__ __forceinline__ void small_item(int32_t d0, int32_t d1, const SmallVars &vars, Prefetch &&prefetch) {
-  using V = typename Vec<T>::type;
+  constexpr int shift = SmallGlobal<T>::shift;
   const int lane = threadIdx.x & 63;
   auto word = [&](int i) { return __builtin_amdgcn_readlane(i < 64 ? d0 : d1, i & 63); };
   auto pointer = [&](int i) { return (uint64_t)(uint32_t)word(i) | (uint64_t)(uint32_t)word(i + 1) << 32; };
   const int32_t pack = word(6);
-  const V *A = (const V *)pointer(0);
-  const V *B = (const V *)pointer(2);
+  uint64_t A = pointer(0), B = pointer(2);
+  const uint64_t C = pointer(4);
   for (int q = 0; q < ((pack >> 24) & 15); ++q)
-    A += (int64_t)vars.v[(word(67) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 5 + q);
+    A += (uint64_t)((int64_t)vars.v[(word(67) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 5 + q) << shift);
   for (int q = 0; q < ((pack >> 28) & 15); ++q)
-    B += (int64_t)vars.v[(word(68) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 9 + q);
-  int32_t oa = 0, ob = 0, oc = 0;
+    B += (uint64_t)((int64_t)vars.v[(word(68) >> (8 * q)) & 31] * __builtin_amdgcn_readlane(d1, 9 + q) << shift);
+  const int lt = pack & 15;
+  int32_t oa = 0, ob = 0, oc = lane >> lt;   // a stored result is dense
 #pragma unroll
   for (int b = 0; b < kSmallLaneBits; ++b) {
     const int32_t on = -((lane >> b) & 1);
-    oa += on & word(8 + b), ob += on & word(14 + b), oc += on & word(20 + b);
+    oa += on & word(8 + b), ob += on & word(14 + b);
   }
-  const int lt = pack & 15;
+  uint32_t cb = (uint32_t)oc << shift;
+  if ((pack >> 22) & 1) {                    // an added one goes through its C offsets
+    oc = 0;
+#pragma unroll
+    for (int b = 0; b < kSmallLaneBits; ++b) oc += -((lane >> b) & 1) & word(20 + b);
+    cb = (uint32_t)oc << ((pack >> 23) & 1 ? 4 : shift);
+  }
+  const uint32_t ab = (uint32_t)oa << shift, bb = (uint32_t)ob << shift;
   const bool store = lane < (1 << ((pack >> 4) & 15)) && (lane & ((1 << lt) - 1)) == 0;
-  void *C = (void *)pointer(4);
-  switch (((pack >> 8) & 15) + ((pack >> 12) & 31)) {
-    case 0: small_terms<T, 1>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
-    case 1: small_terms<T, 2>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
-    case 2: small_terms<T, 4>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
-    default: small_terms<T, 8>(d0, d1, A, B, C, oa, ob, oc, pack, store, prefetch); break;
+  const int e = (pack >> 8) & 15, t = (pack >> 12) & 31;
+#define QX_SMALL(LE, LT, LOOP) small_terms<T, LE, LT, LOOP>(d0, d1, A, B, C, ab, bb, cb, pack, store, prefetch)
+  if (e == 0) {
+    if (t == 0) QX_SMALL(0, 0, false);
+    else if (t == 1) QX_SMALL(0, 1, false);
+    else if (t == 2) QX_SMALL(0, 2, false);
+    else QX_SMALL(0, 3, true);
+  } else if (e == 1) {
+    if (t == 0) QX_SMALL(1, 0, false);
+    else if (t == 1) QX_SMALL(1, 1, false);
+    else QX_SMALL(1, 2, false);
+  } else if (e == 2) {
+    if (t == 0) QX_SMALL(2, 0, false);
+    else QX_SMALL(2, 1, false);
+  } else {
+    QX_SMALL(3, 0, false);
   }
+#undef QX_SMALL
 }
 
 // Levels [0, nlevels) of items in order, the waves of the grid taking a level's items in

@@ -1560,8 +1560,8 @@ void chain_swizzle(ChainArgs &a, int elem_bytes) {
 namespace {
 
 // Whether a step may run inside a small-step batch: power-of-two legs with at most
-// kSmallMaxBits C and K bits each, at most 2^18 MACs, and operand offsets that fit 32 bits.  C and K are each at most 4096,
-// except with `wide` (the pullback, whose gradient steps sum long bitstring-batch
+// kSmallMaxBits C and K bits each, at most 2^18 MACs, and operand offsets of at most 32
+// bits in bytes of 16 per value.  C and K are each at most 4096, except with `wide` (the pullback, whose gradient steps sum long bitstring-batch
 // ranges into a few elements): then up to 2^16 MACs with any split.  (The forward
 // keeps the limit: its larger steps run faster as multi-workgroup launches.)
 bool small_step(const Step &st, bool wide = false) {
@@ -1581,7 +1581,7 @@ bool small_step(const Step &st, bool wide = false) {
     nbk += ilog2(g.dim);
     wa += g.sa * (g.dim - 1), wb += g.sb * (g.dim - 1);
   }
-  return nbc <= kSmallMaxBits && nbk <= kSmallMaxBits && std::max(wa, wb) < (int64_t(1) << 30);
+  return nbc <= kSmallMaxBits && nbk <= kSmallMaxBits && std::max(wa, wb) < (int64_t(1) << 28);
 }
 
 // Items of a small step (waves that work on it).
@@ -2257,7 +2257,9 @@ VjpLowered lower_vjp(const Program &p, int64_t batch, int precision, uint64_t fu
       BwdStep b = std::move(bv[i]);
       // adds of one level go out in one launch: each destination at most once (a key's
       // gradient has one adding step; a cotangent buffer one per level)
-      bool ok = small_step(b.step, true) && no_slice_terms(b) &&
+      int64_t add_reach = 0;   // in 32 bits of bytes, as the operands'
+      for (size_t j = 0; j < b.add_dims.size(); ++j) add_reach += b.add_strides[j] * (b.add_dims[j] - 1);
+      bool ok = small_step(b.step, true) && no_slice_terms(b) && add_reach < (int64_t(1) << 28) &&
                 (b.direct || (b.add_dims.size() <= (size_t)kSmallMaxBits &&
                               ((b.dest == Buf::Grad && key_uses[b.dest_key] == 1) ||
                                (b.dest == Buf::Cot && !level_cot.count({level_base + lev[i], b.dest_root})))));
