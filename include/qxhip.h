@@ -91,6 +91,10 @@ qx_status qx_plan_set_tensor(qx_plan *plan, const char *key, const double *z, in
  * re-tuning the plan.  Returns after the copy has reached the device. */
 qx_status qx_plan_update_tensor(qx_plan *plan, const char *key, const double *z, int64_t nelem);
 
+/* The same for n data keys in one copy: `keys` are indices of qx_plan_key, `z` their
+ * values one key after the other, `nelem` complex values in all. */
+qx_status qx_plan_update_tensors(qx_plan *plan, const int64_t *keys, int64_t n, const double *z, int64_t nelem);
+
 /* Plan options, set before qx_plan_finalize ("profile", "graph", "fuse_slices" and
  * "autotune" may also be set later, "small_walk" too; setting "profile" clears the accumulated step
  * times):

@@ -109,7 +109,11 @@ struct qx_plan {
                                             // swizzled tiles (bit 2), barriers (bit 3); tests
   bool finalized = false;
 
-  std::vector<DevBuf> data;                 // per key
+  // every key's tensor in one device allocation (256-byte aligned, as in `image`, the
+  // host's copy of it), so any number of new tensors is one copy
+  DevBuf data;
+  std::vector<size_t> data_off;             // per key: byte offset
+  std::vector<char> image;
   std::map<std::pair<int64_t, uint64_t>, qx::Lowered> lowered;   // per (batch size, fused slice vars)
   std::map<std::pair<int64_t, uint64_t>, qx::VjpLowered> vjp_lowered;
   std::map<std::pair<int64_t, int>, uint64_t> fuse_choice;          // (batch, vjp) -> fused vars
@@ -163,7 +167,7 @@ struct qx_plan {
   size_t esize() const { return prec == QX_C128 ? 16 : 8; }
 
   ~qx_plan() {
-    for (auto &d : data) d.release();
+    data.release();
     arena.release();
     out_off.release();
     out_q.release();
@@ -235,6 +239,39 @@ struct Bases {
   char *arena = nullptr, *cot = nullptr, *temp = nullptr;
 };
 
+// Key i's values (interleaved complex128, n doubles) into the host image, in the plan's type.
+void put_data(qx_plan *P, size_t i, const double *z, size_t n) {
+  char *dst = P->image.data() + P->data_off[i];
+  if (P->prec == QX_C128) {
+    if (n) std::memcpy(dst, z, n * 8);
+  } else {
+    for (size_t j = 0; j < n; ++j) {
+      const float f = (float)z[j];
+      std::memcpy(dst + 4 * j, &f, 4);
+    }
+  }
+}
+
+// New values of n keys, packed in z: into the image, then one copy of the bytes they
+// span.  Lowered steps, descriptor tables and captured graphs address the buffer, not its
+// values, so all of them stay valid.  The copy is stream-ordered after earlier calls'
+// work and synchronous towards the caller.
+void update_data(qx_plan *P, const int64_t *keys, int64_t n, const double *z) {
+  size_t lo = P->image.size(), hi = 0;
+  for (int64_t j = 0; j < n; ++j) {
+    const size_t i = (size_t)keys[j], values = 2 * (size_t)P->prog.key_elems.at(P->prog.keys[i]);
+    put_data(P, i, z, values);
+    z += values;
+    lo = std::min(lo, P->data_off[i]);
+    hi = std::max(hi, P->data_off[i] + values / 2 * P->esize());
+  }
+  if (lo >= hi) return;
+  hip_check(hipSetDevice(P->ctx->device), "hipSetDevice");
+  hipStream_t s = P->ctx->stream;
+  hip_check(hipMemcpyAsync((char *)P->data.p + lo, P->image.data() + lo, hi - lo, hipMemcpyHostToDevice, s), "upload");
+  hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
+}
+
 int64_t value_offset(const qx::Value &v, const std::vector<int64_t> &varval) {
   int64_t off = v.static_off;
   for (auto &t : v.var_terms) off += varval[t.first] * t.second;
@@ -246,7 +283,7 @@ void *value_ptr(qx_plan *P, const qx::Value &v, const std::vector<int64_t> &varv
   const int64_t es = (int64_t)P->esize();
   char *base = nullptr;
   switch (v.buf) {
-    case qx::Buf::Data: base = (char *)P->data[v.data_key].p; break;
+    case qx::Buf::Data: base = (char *)P->data.p + P->data_off[v.data_key]; break;
     case qx::Buf::Arena: base = b.arena + v.slot * es; break;
     case qx::Buf::Cot: base = b.cot + v.slot * es; break;
     case qx::Buf::Temp: base = b.temp + v.slot * es; break;
@@ -1810,20 +1847,24 @@ qx_status qx_plan_update_tensor(qx_plan *plan, const char *key, const double *z,
       throw qx::Error(QX_ERR_DATA, std::string("data key '") + key + "' needs " + std::to_string(it->second) +
                                        " elements, got " + std::to_string(nelem));
     const auto &keys = plan->prog.keys;
-    const size_t i = (size_t)(std::find(keys.begin(), keys.end(), std::string(key)) - keys.begin());
-    hip_check(hipSetDevice(plan->ctx->device), "hipSetDevice");
-    // same buffer, new contents: lowered steps, descriptor tables and captured graphs
-    // address the buffer, not its values, so all of them stay valid.  The copy is
-    // stream-ordered after earlier calls' work and synchronous towards the caller.
-    hipStream_t s = plan->ctx->stream;
-    if (plan->prec == QX_C128) {
-      hip_check(hipMemcpyAsync(plan->data[i].p, z, (size_t)nelem * 16, hipMemcpyHostToDevice, s), "upload");
-    } else {
-      std::vector<float> f(z, z + 2 * nelem);
-      hip_check(hipMemcpyAsync(plan->data[i].p, f.data(), (size_t)nelem * 8, hipMemcpyHostToDevice, s), "upload");
+    const int64_t i = std::find(keys.begin(), keys.end(), std::string(key)) - keys.begin();
+    update_data(plan, &i, 1, z);
+  });
+}
+
+qx_status qx_plan_update_tensors(qx_plan *plan, const int64_t *keys, int64_t n, const double *z, int64_t nelem) {
+  return guard([&] {
+    if (!plan || n < 0 || (!keys && n > 0) || (!z && nelem > 0)) throw qx::Error(QX_ERR_ARGUMENT, "null argument");
+    if (!plan->finalized) throw qx::Error(QX_ERR_STATE, "plan is not finalized (use qx_plan_set_tensor)");
+    int64_t need = 0;
+    for (int64_t i = 0; i < n; ++i) {
+      if (keys[i] < 0 || keys[i] >= (int64_t)plan->prog.keys.size())
+        throw qx::Error(QX_ERR_ARGUMENT, "key index out of range");
+      need += plan->prog.key_elems.at(plan->prog.keys[keys[i]]);
     }
-    hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
-    plan->host_data[key].assign(z, z + 2 * nelem);
+    if (need != nelem)
+      throw qx::Error(QX_ERR_DATA, "the data keys need " + std::to_string(need) + " elements, got " + std::to_string(nelem));
+    update_data(plan, keys, n, z);
   });
 }
 
@@ -1885,19 +1926,20 @@ qx_status qx_plan_finalize(qx_plan *plan) {
     }
     // lower once up front so label or memory errors surface here
     ensure_lowered(plan, plan->opt_batch);
-    plan->data.resize(plan->prog.keys.size());
-    const size_t es = plan->esize();
-    for (size_t i = 0; i < plan->prog.keys.size(); ++i) {
-      const auto &h = plan->host_data[plan->prog.keys[i]];
-      size_t n = h.size() / 2;
-      plan->data[i].reserve(std::max<size_t>(n * es, 16));
-      if (plan->prec == QX_C128) {
-        hip_check(hipMemcpy(plan->data[i].p, h.data(), n * 16, hipMemcpyHostToDevice), "upload");
-      } else {
-        std::vector<float> f(h.begin(), h.end());
-        hip_check(hipMemcpy(plan->data[i].p, f.data(), n * 8, hipMemcpyHostToDevice), "upload");
-      }
+    size_t bytes = 0;
+    plan->data_off.clear();
+    for (auto &k : plan->prog.keys) {
+      plan->data_off.push_back(bytes);
+      bytes += (plan->host_data.at(k).size() / 2 * plan->esize() + 255) / 256 * 256;
     }
+    plan->data.reserve(std::max<size_t>(bytes, 16));
+    plan->image.assign(bytes, 0);
+    for (size_t i = 0; i < plan->prog.keys.size(); ++i) {
+      const auto &h = plan->host_data.at(plan->prog.keys[i]);
+      put_data(plan, i, h.data(), h.size());
+    }
+    if (bytes) hip_check(hipMemcpy(plan->data.p, plan->image.data(), bytes, hipMemcpyHostToDevice), "upload");
+    plan->host_data.clear();
     plan->finalized = true;
   });
 }

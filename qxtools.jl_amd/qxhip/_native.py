@@ -23,7 +23,8 @@ SYMBOLS = [
     "qx_plan_set_option", "qx_plan_finalize", "qx_plan_info", "qx_plan_key",
     "qx_amplitudes", "qx_amplitudes_vjp", "qx_plan_stats", "qx_plan_destroy", "qx_last_error",
     "qx_dsl_inspect", "qx_dsl_inspect_ex", "qx_amplitudes_uniform", "qx_sample_rejection",
-    "qx_measure_mfma", "qx_norm_vjp", "qx_plan_update_tensor", "qx_amplitudes_noalloc",
+    "qx_measure_mfma", "qx_norm_vjp", "qx_plan_update_tensor", "qx_plan_update_tensors",
+    "qx_amplitudes_noalloc",
 ]
 
 
@@ -50,6 +51,7 @@ def lib() -> C.CDLL:
         L.qx_plan_from_dsl.argtypes = [p, C.c_char_p, sz, C.c_int, C.POINTER(p)]
         L.qx_plan_set_tensor.argtypes = [p, C.c_char_p, dp, i64]
         L.qx_plan_update_tensor.argtypes = [p, C.c_char_p, dp, i64]
+        L.qx_plan_update_tensors.argtypes = [p, C.POINTER(i64), i64, dp, i64]
         L.qx_plan_set_option.argtypes = [p, C.c_char_p, i64]
         L.qx_plan_finalize.argtypes = [p]
         L.qx_plan_info.argtypes = [p] + [C.POINTER(i64)] * 5
@@ -150,6 +152,15 @@ class Plan:
         (`qx_plan_update_tensor`): later calls, captured graphs included, see them."""
         arr = np.ascontiguousarray(np.asarray(value).reshape(-1, order="F"), dtype=np.complex128)
         _check(lib().qx_plan_update_tensor(self._h, key.encode(), _dptr(arr.view(np.float64)), arr.size))
+
+    def update_tensors(self, keys: np.ndarray, values: np.ndarray) -> None:
+        """New values of several data keys in one copy (`qx_plan_update_tensors`): int64
+        indices into `keys_needed()` and the keys' values, column-major, one after the
+        other."""
+        keys = np.ascontiguousarray(keys, dtype=np.int64)
+        arr = np.ascontiguousarray(values, dtype=np.complex128)
+        _check(lib().qx_plan_update_tensors(self._h, keys.ctypes.data_as(C.POINTER(C.c_int64)), keys.size,
+                                            _dptr(arr.view(np.float64)), arr.size))
 
     def keys_needed(self) -> list:
         n = C.c_int64()

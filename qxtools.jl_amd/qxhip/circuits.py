@@ -67,6 +67,23 @@ def dry(theta: float) -> np.ndarray:
     return 0.5 * np.array([[-s, -c], [c, -s]], dtype=np.complex128)
 
 
+def param_gate_tensors(name: str, angles, deriv: bool = False) -> np.ndarray:
+    """The network tensors of one parameterised gate at many angles (or their derivatives
+    in the angle), a row each, column-major: Rz as its diagonal, Ry as its matrix."""
+    if name == "rz":
+        a = np.asarray(angles, dtype=np.float64)
+        out = np.stack([np.exp(-0.5j * a), np.exp(0.5j * a)], axis=1)
+        if deriv:
+            out = out * np.array([-0.5j, 0.5j])
+        return out
+    c = [math.cos(a / 2) for a in angles]
+    s = [math.sin(a / 2) for a in angles]
+    if deriv:
+        c, s = [-0.5 * x for x in s], [0.5 * x for x in c]
+    c, s = np.array(c), np.array(s)
+    return np.stack([c, s, -s, c], axis=1).astype(np.complex128)
+
+
 GATES = {
     "x": X, "y": Y, "z": Z, "h": H, "sx": SQRT_X, "sy": SQRT_Y, "sw": SQRT_W,
     "cz": CZ, "cx": CX,

@@ -37,6 +37,7 @@ class TensorCache:
         self.key_dim_map: "OrderedDict[str, tuple]" = OrderedDict()
         self.id_val = 1
         self.label = label
+        self._exact: dict = {}   # (shape, bytes) of each finite tensor -> key: equal ones need no comparison
 
     def next_symbol(self) -> str:
         s = f"{self.label}{self.id_val}"
@@ -47,6 +48,9 @@ class TensorCache:
         data = np.asarray(data)
         dim = tuple(int(d) for d in data.shape)
         flat = data.reshape(-1, order="F").astype(np.complex128)
+        same = (dim, flat.tobytes())
+        if same in self._exact:   # (no earlier key is within eps of it: it would have that key)
+            return self._exact[same]
         eps = np.finfo(np.float64).eps
         if dim in self.tensors:
             for sym, stored in self.tensors[dim]:
@@ -55,6 +59,8 @@ class TensorCache:
         sym = self.next_symbol()
         self.tensors.setdefault(dim, []).append((sym, flat))
         self.key_dim_map[sym] = dim
+        if np.isfinite(flat).all():
+            self._exact[same] = sym
         return sym
 
     def __getitem__(self, sym: str) -> np.ndarray:

@@ -15,11 +15,11 @@ from __future__ import annotations
 import numpy as np
 
 from . import _native
-from .circuits import Circuit, gate_matrix, gate_matrix_derivative, gate_qubits
+from .circuits import Circuit, param_gate_tensors
 from .compute_graph import build_compute_graph
 from .planning import contraction_scheme, sweep_contraction_plan
 from .simulation import Executor
-from .tn import TensorNetworkCircuit, gate_tensor_map
+from .tn import gate_tensor_map
 
 
 class ParamCircuit:
@@ -27,7 +27,7 @@ class ParamCircuit:
 
     def __init__(self, circ: Circuit, planner: str = "sweep", nslice: int = 0, precision: str = "c128",
                  batch: int | None = None, device: int = 0, graph: int = 1, **plan_kwargs):
-        self.circ = circ
+        self._circ, self._angles = circ, None
         tnc, names = gate_tensor_map(circ)
         tnc.add_input()
         tnc.add_output()
@@ -44,58 +44,82 @@ class ParamCircuit:
             if len(tn_names) != 1:
                 raise ValueError("parameterised gates must convert to one tensor")
             self._pgates.append((gi, key_of[tn_names[0]]))
-        self._set_terms()
+        self._index_gates()
+        self._set_terms([circ.ops[gi].theta for gi, _ in self._pgates])
         self.dsl = self.graph.to_dsl()
         self.executor = Executor(self.dsl, self.graph.data, precision=precision, device=device, batch=batch,
                                  graph=graph)
+        at = {k: i for i, k in enumerate(self.executor.plan.keys_needed())}
+        self._pkeys = np.array([at[k] for k in self._tkeys], dtype=np.int64)
         self.num_params = circ.num_params
 
-    def _gate_tensor(self, g, deriv: bool) -> np.ndarray:
-        """The gate's tensor (or dT/dtheta) through the same conversion as the network."""
-        scratch = TensorNetworkCircuit(self.circ.num_qubits)
-        m = gate_matrix_derivative(g) if deriv else gate_matrix(g)
-        (name,) = scratch.push(gate_qubits(g), m)
-        return scratch.tn[name].data
+    @property
+    def circ(self) -> Circuit:
+        """The circuit at the current angles."""
+        if self._angles is not None:
+            self._circ, self._angles = self._circ.with_params(self._angles), None
+        return self._circ
 
-    def _set_terms(self) -> None:
-        """Chain-rule terms (param index, key, dT/dtheta in the key's array layout) at
-        the current angles, as one segmented reduction over all parameters."""
-        self.terms = []
-        for gi, key in self._pgates:
-            g = self.circ.ops[gi]
-            d = self._gate_tensor(g, True)
-            if d.shape != self.graph.data[key].shape:
-                raise ValueError(f"derivative of gate {g.name} has a different tensor structure")
-            self.terms.append((g.param, key, d))
-        self._tp = np.array([p for p, _, _ in self.terms], dtype=np.int64)
-        self._tkeys = [k for _, k, _ in self.terms]
-        self._td = np.concatenate([d.reshape(-1, order="F") for _, _, d in self.terms]) if self.terms else np.zeros(0)
-        self._tstart = np.cumsum([0] + [d.size for _, _, d in self.terms[:-1]]).astype(np.int64)
+    @property
+    def terms(self) -> list:
+        """Chain-rule terms (param index, key, dT/dtheta in the key's array layout)."""
+        return [(int(p), k, d) for p, k, d in zip(self._tp, self._tkeys, self._arrays(self._td))]
+
+    def _index_gates(self) -> None:
+        """Where each parameterised gate's tensor lies in the flat arrays of all of them,
+        gates of a kind together, so that a new set of angles is a few array operations."""
+        ops = self._circ.ops
+        self._tkeys = [k for _, k in self._pgates]
+        self._tp = np.array([ops[gi].param for gi, _ in self._pgates], dtype=np.int64)
+        self._shapes = [self.graph.data[k].shape for k in self._tkeys]
+        sizes = np.array([int(np.prod(s)) for s in self._shapes], dtype=np.int64)
+        self._tstart = np.cumsum(sizes) - sizes
+        self._tsize = int(sizes.sum())
+        self._kinds = []   # (gate name, its positions among the gates, flat index of every value)
+        for name in sorted({ops[gi].name for gi, _ in self._pgates}):
+            at = np.array([i for i, (gi, _) in enumerate(self._pgates) if ops[gi].name == name], dtype=np.int64)
+            shape = {"rz": (2,), "ry": (2, 2)}[name]
+            if any(self._shapes[i] != shape for i in at):
+                raise ValueError(f"derivative of gate {name} has a different tensor structure")
+            self._kinds.append((name, at, (self._tstart[at][:, None] + np.arange(int(np.prod(shape)))).reshape(-1)))
+
+    def _tensors(self, angles, deriv: bool) -> np.ndarray:
+        """Every parameterised gate's tensor (or dT/dtheta), flat, one after the other.  A
+        rotation whose tensor has no off-diagonal value has another structure there."""
+        out = np.zeros(self._tsize, dtype=np.complex128)
+        for name, at, index in self._kinds:
+            t = param_gate_tensors(name, [angles[i] for i in at], deriv)
+            if t.shape[1] == 4 and np.any((t[:, 1] == 0) & (t[:, 2] == 0)):
+                raise ValueError(f"derivative of gate {name} has a different tensor structure" if deriv else
+                                 f"gate {name} at the new angle has a different tensor structure")
+            out[index] = t.reshape(-1)
+        return out
+
+    def _arrays(self, flat: np.ndarray) -> list:
+        return [flat[a:a + int(np.prod(s))].reshape(s, order="F") for a, s in zip(self._tstart.tolist(), self._shapes)]
+
+    def _set_terms(self, angles) -> None:
+        """dT/dtheta of every gate at the given angles, for one segmented reduction."""
+        self._td = self._tensors(angles, True)
 
     def params(self) -> np.ndarray:
         return self.circ.params()
 
     def set_params(self, theta) -> None:
-        """Move the plan to new angles: every parameterised gate's tensor is rebuilt
-        and re-uploaded into its device buffer (`qx_plan_update_tensor`), so the
-        lowering, tuning and captured graphs are kept; the chain-rule terms follow."""
+        """Move the plan to new angles: every parameterised gate's tensor is rebuilt and
+        all of them re-uploaded in one copy (`qx_plan_update_tensors`), so the lowering,
+        tuning and captured graphs are kept; the chain-rule terms follow."""
         theta = np.asarray(theta, dtype=np.float64)
         if theta.shape != (self.num_params,):
             raise ValueError(f"need {self.num_params} angles, got shape {theta.shape}")
-        new = self.circ.with_params(theta)
-        tensors = []
-        for gi, key in self._pgates:
-            t = TensorNetworkCircuit(new.num_qubits)
-            (name,) = t.push(gate_qubits(new.ops[gi]), gate_matrix(new.ops[gi]))
-            arr = t.tn[name].data
-            if arr.shape != self.graph.data[key].shape:
-                raise ValueError(f"gate {new.ops[gi].name} at the new angle has a different tensor structure")
-            tensors.append((key, arr))
-        for key, arr in tensors:
-            self.executor.plan.update_tensor(key, arr)
+        angles = theta[self._tp].tolist()
+        flat = self._tensors(angles, False)
+        if self._tkeys:
+            self.executor.plan.update_tensors(self._pkeys, flat)
+        for key, arr in zip(self._tkeys, self._arrays(flat)):
             self.graph.data[key] = arr
-        self.circ = new
-        self._set_terms()
+        self._angles = theta.copy()
+        self._set_terms(angles)
 
     def amplitudes(self, bits) -> np.ndarray:
         return self.executor.amplitudes(bits)
@@ -104,7 +128,7 @@ class ParamCircuit:
         """dL/dtheta_p = sum over the gate tensors T of parameter p of
         Re <dL/dT, dT/dtheta_p> (the cotangent is conj-linear)."""
         out = np.zeros(self.num_params)
-        if not self.terms:
+        if not self._tkeys:
             return out
         g = np.concatenate([key_grad[k] for k in self._tkeys])
         per_term = np.add.reduceat(np.real(np.conj(g) * self._td), self._tstart)
@@ -115,7 +139,7 @@ class ParamCircuit:
         """`param_grad` from the pullback's flat gradient (layout of the plan's
         `key_offsets`): the terms' entries gathered by one precomputed index."""
         out = np.zeros(self.num_params)
-        if not self.terms:
+        if not self._tkeys:
             return out
         if getattr(self, "_tidx", None) is None:
             offs = self.executor.plan.key_offsets()

@@ -111,22 +111,23 @@ class TensorNetwork:
         return copy.deepcopy(self)
 
 
+def _at(t: np.ndarray, ax: int, i: int, ax2: int, j: int) -> np.ndarray:
+    """t with axis `ax` at i and axis `ax2` at j."""
+    idx = [slice(None)] * t.ndim
+    idx[ax], idx[ax2] = i, j
+    return t[tuple(idx)]
+
+
 def _diagonal_in(t: np.ndarray, ax_out: int, ax_in: int) -> bool:
     """True if t vanishes whenever the two axes take different values."""
     d = t.shape[ax_out]
-    for a in range(d):
-        for b in range(d):
-            if a != b and np.any(np.take(np.take(t, [a], axis=ax_out), [b], axis=ax_in)):
-                return False
-    return True
+    return not any(a != b and _at(t, ax_out, a, ax_in, b).any() for a in range(d) for b in range(d))
 
 
 def _take_diagonal(t: np.ndarray, ax_keep: int, ax_drop: int) -> np.ndarray:
     """Collapse two equal-dim axes to their diagonal, keeping it at ax_keep."""
-    d = t.shape[ax_keep]
-    parts = [np.take(np.take(t, [a], axis=ax_keep), [a], axis=ax_drop) for a in range(d)]
-    out = np.concatenate(parts, axis=ax_keep)
-    return np.squeeze(out, axis=ax_drop)
+    parts = [_at(t, ax_keep, a, ax_drop, a) for a in range(t.shape[ax_keep])]
+    return np.stack(parts, axis=ax_keep - (ax_keep > ax_drop))
 
 
 class TensorNetworkCircuit:
@@ -142,6 +143,7 @@ class TensorNetworkCircuit:
         self.output_tensors: list = []
         self.output_qubits: list = []  # qubit of each output tensor
         self.gate_tensors: list = []   # per pushed gate: (tensor names, qubits), time order
+        self._forms: dict = {}         # gate matrices seen (bytes): diagonal qubits and tensor
 
     def qubits(self) -> int:
         return self.num_qubits
@@ -180,12 +182,19 @@ class TensorNetworkCircuit:
         if decompose and k == 2:
             return self._push_decomposed(qubits, t)
         legs_out, legs_in, keep = [], [], []
-        diag = [_diagonal_in(t, j, k + j) for j in range(k)]
-        data = t
-        # collapse diagonal qubits (highest axes first so positions stay valid)
-        for j in reversed(range(k)):
-            if diag[j]:
-                data = _take_diagonal(data, j, k + j)
+        form = (k, t.tobytes())
+        if form in self._forms:
+            diag, data = self._forms[form]
+            data = data.copy()
+        else:
+            diag = [_diagonal_in(t, j, k + j) for j in range(k)]
+            data = t
+            # collapse diagonal qubits (highest axes first so positions stay valid)
+            for j in reversed(range(k)):
+                if diag[j]:
+                    data = _take_diagonal(data, j, k + j)
+            if len(self._forms) < 256:
+                self._forms[form] = (diag, data.copy())
         for j, q in enumerate(qubits):
             w = self.output_indices[q - 1]
             if diag[j]:
