@@ -463,9 +463,8 @@ void launch_fill_outputs(int prec, void *arena, const int64_t *d_out_off, int n_
                          const int *d_out_q, const char *d_bits, int64_t nvalid, int64_t batch,
                          int64_t num_chars, void *stream);
 void launch_accumulate(int prec, const void *root, int64_t root_bstride, int64_t batch, int64_t nvalid,
-                       int64_t relems, const int64_t *d_relem_off, double *acc, int64_t row0,
-                       void *stream);
-void launch_finalize(const double *acc, double *out, int64_t n, void *stream);
+                       int64_t relems, const int64_t *d_relem_off, double *acc, double *out, int64_t row0,
+                       bool first, bool last, void *stream);
 // dst[map(e)] += src[e] for src dense over dims (first fastest), map = sum digit*stride
 void launch_add_mapped(int prec, int dst_double, void *dst, const void *src, int64_t n,
                        const std::vector<int64_t> &dims, const std::vector<int64_t> &strides,

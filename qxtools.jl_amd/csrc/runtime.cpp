@@ -16,6 +16,7 @@
 #include <cmath>
 #include <cstring>
 #include <memory>
+#include <mutex>
 #include <set>
 #include <sstream>
 #include <tuple>
@@ -28,6 +29,9 @@ struct qx_ctx {
   rocblas_handle blas = nullptr;   // created by the first plan that runs a vendor BLAS step
   void *blas_ws = nullptr;         // its workspace (the handle allocates nothing itself)
   void *scratch = nullptr;         // device address of the library's fixed scratch area
+  // pinned host blocks of plans that are gone, at most kPinKept, for the next ones
+  std::mutex pin_mutex;
+  std::vector<void *> pins;
 };
 
 namespace {
@@ -54,6 +58,41 @@ qx_status guard(F &&f) {
     g_last_error = e.what();
     return QX_ERR_ARGUMENT;
   }
+}
+
+// One block of pinned host memory per plan carries what a small call hands over: the
+// kernels read its bitstrings and write its results there, in place of a copy launch on
+// each side (one 3x3 amplitude: 10 us before the first kernel, 13 after the last).
+constexpr size_t kPinBytes = size_t(256) << 10;   // a block
+constexpr size_t kPinBits = 4096;                 // bitstrings; larger calls copy theirs
+constexpr size_t kPinState = 256;                 // rejection state and counters after them
+constexpr size_t kPinOut = kPinBytes - kPinBits - kPinState;   // results; larger ones are copied
+constexpr size_t kPinKept = 8;
+
+void *pin_acquire(qx_ctx *c) {
+  {
+    std::lock_guard<std::mutex> lk(c->pin_mutex);
+    if (!c->pins.empty()) {
+      void *p = c->pins.back();
+      c->pins.pop_back();
+      return p;
+    }
+  }
+  void *p = nullptr;
+  hip_check(hipHostMalloc(&p, kPinBytes, hipHostMallocDefault), "hipHostMalloc");
+  return p;
+}
+
+void pin_release(qx_ctx *c, void *p) {
+  if (!p) return;
+  {
+    std::lock_guard<std::mutex> lk(c->pin_mutex);
+    if (c->pins.size() < kPinKept) {
+      c->pins.push_back(p);
+      return;
+    }
+  }
+  (void)hipHostFree(p);
 }
 
 struct DevBuf {
@@ -83,8 +122,8 @@ struct DevBuf {
   // exactly them from the previous upload (small per-call tables).
   void upload(const void *src, size_t n, hipStream_t s) {
     if (held.size() == n && n > 0 && std::memcmp(held.data(), src, n) == 0) return;
-    hip_check(hipMemcpyAsync(p, src, n, hipMemcpyHostToDevice, s), "copy");
-    held.assign((const char *)src, (const char *)src + n);
+    held.assign((const char *)src, (const char *)src + n);   // (the copy's source: it outlives the call)
+    hip_check(hipMemcpyAsync(p, held.data(), n, hipMemcpyHostToDevice, s), "copy");
   }
 };
 
@@ -164,9 +203,17 @@ struct qx_plan {
   }
   std::vector<int> event_step;              // step of each recorded pair this call
 
+  char *pin = nullptr;                      // its block of pinned host memory, from the first call on
+
   size_t esize() const { return prec == QX_C128 ? 16 : 8; }
+  char *pinned() {
+    if (!pin) pin = (char *)pin_acquire(ctx);
+    return pin;
+  }
 
   ~qx_plan() {
+    if (pin) (void)hipStreamSynchronize(ctx->stream);   // (a call that failed may have left work that uses it)
+    pin_release(ctx, pin);
     data.release();
     arena.release();
     out_off.release();
@@ -901,7 +948,7 @@ void check_bits(qx_plan *P, const char *bits, int64_t nb) {
 
 // Device buffers of one amplitudes call (besides the plan's arena, workspace and data).
 struct CallBufs {
-  void *acc = nullptr;        // nb * R FP64 Neumaier (sum, compensation) pairs, complex
+  void *acc = nullptr;        // nb * R FP64 Neumaier (sum, compensation) pairs, complex (several slices)
   void *outbuf = nullptr;     // nb * R complex128 results
   void *out_off = nullptr;    // per output tensor: its arena slot (int64)
   void *out_q = nullptr;      // per output tensor: its qubit (int32)
@@ -909,8 +956,8 @@ struct CallBufs {
   void *bits = nullptr;       // nb * num_chars bitstring characters
 };
 
-// The device work of one amplitudes call, from zeroing the accumulators to the final
-// sum: steps of section 0 once, per looped slice those of section 1, per batch of
+// The device work of one amplitudes call, from the first step to the final sum: steps of
+// section 0 once, per looped slice those of section 1, per batch of
 // bitstrings the output fill, section 2 and the accumulation into FP64 pairs.
 // `timed`: record per-launch events when the plan's "profile" option is on.
 void enqueue_amplitudes(qx_plan *P, const qx::Lowered &L, uint64_t fused, int64_t s0, int64_t s1, int64_t nb,
@@ -920,7 +967,6 @@ void enqueue_amplitudes(qx_plan *P, const qx::Lowered &L, uint64_t fused, int64_
   const int64_t R = L.result_elems;
   const int nout = (int)P->prog.outputs.size();
   const qx::Value &rv = L.values[P->prog.save];
-  qx::launch_zero(cb.acc, nb * R * 32, stream);
   const size_t nv = P->prog.vars.size();
   std::vector<int64_t> varval(nv, 0);
   const qx_plan::SmallTable &ST = P->small.at(&L);
@@ -954,10 +1000,10 @@ void enqueue_amplitudes(qx_plan *P, const qx::Lowered &L, uint64_t fused, int64_
                               (const char *)cb.bits + row0 * nch, nvalid, batch, nch, stream);
       run_section(2);
       qx::launch_accumulate(P->prec, value_ptr(P, rv, varval), rv.dep ? rv.beta_stride : 0, batch, nvalid, R,
-                            (const int64_t *)cb.relem_off, (double *)cb.acc, row0, stream);
+                            (const int64_t *)cb.relem_off, (double *)cb.acc, (double *)cb.outbuf, row0, sl == s0,
+                            sl + 1 == s1, stream);
     }
   }
-  qx::launch_finalize((const double *)cb.acc, (double *)cb.outbuf, nb * R, stream);
 }
 
 // Amplitudes of nb bitstrings summed over slices [s0, s1).  `bits` null: the
@@ -1032,15 +1078,18 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   }
   moved |= P->relem_off.reserve(std::max<size_t>(R * 8, 16));
   P->relem_off.upload(roff.data(), R * 8, stream);
-  size_t nbits = (size_t)nb * nch;
-  if (bits) {
+  const size_t nbits = (size_t)nb * nch, nout_bytes = (size_t)nb * R * 16;
+  const bool pin_bits = bits && nbits <= kPinBits, pin_out = out && nout_bytes <= kPinOut;
+  if (pin_bits) {
+    std::memcpy(P->pinned(), bits, nbits);
+  } else if (bits) {
     moved |= P->bits.reserve(std::max<size_t>(nbits, 16));
-    if (nbits) hip_check(hipMemcpyAsync(P->bits.p, bits, nbits, hipMemcpyHostToDevice, stream), "copy");
+    hip_check(hipMemcpyAsync(P->bits.p, bits, nbits, hipMemcpyHostToDevice, stream), "copy");
   } else if (P->bits.bytes < nbits) {
     throw qx::Error(QX_ERR_STATE, "internal: device bitstrings not staged");
   }
-  moved |= P->acc.reserve((size_t)nb * R * 32);
-  moved |= P->outbuf.reserve((size_t)nb * R * 16);
+  if (s1 - s0 > 1) moved |= P->acc.reserve((size_t)nb * R * 32);
+  if (!pin_out) moved |= P->outbuf.reserve(nout_bytes);
   if (moved) P->drop_graphs();
   {
     Bases bs;
@@ -1051,15 +1100,19 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   P->event_step.clear();
 
   CallBufs cb;
-  cb.acc = P->acc.p, cb.outbuf = P->outbuf.p, cb.out_off = P->out_off.p, cb.out_q = P->out_q.p;
-  cb.relem_off = P->relem_off.p, cb.bits = P->bits.p;
+  char *const pin_results = pin_out ? P->pinned() + kPinBits + kPinState : nullptr;
+  cb.acc = P->acc.p, cb.out_off = P->out_off.p, cb.out_q = P->out_q.p, cb.relem_off = P->relem_off.p;
+  cb.outbuf = pin_out ? pin_results : P->outbuf.p;
+  cb.bits = pin_bits ? P->pin : P->bits.p;
   auto enqueue = [&]() { enqueue_amplitudes(P, L, fused, s0, s1, nb, batch, cb, tuner.get(), true); };
   const int64_t nrows = (nb + batch - 1) / batch;
   const int64_t launches = 2 + section_launches(L, 0) +
                            (s1 - s0) * (section_launches(L, 1) + nrows * (section_launches(L, 2) + 2));
   P->last_launches = launches;
   if (P->opt_graph && !P->opt_profile && !tuner && launches <= kMaxGraphLaunches) {
-    auto key = std::make_tuple(batch, nb, s0, s1 + (fused ? (int64_t(1) << 40) : 0));
+    auto key = std::make_tuple(batch, nb, s0,
+                               s1 + (fused ? int64_t(1) << 40 : 0) + (out ? int64_t(1) << 41 : 0) +
+                                   (bits ? int64_t(1) << 42 : 0));
     auto it = P->graphs.find(key);
     if (it == P->graphs.end()) {
       hipGraph_t g = nullptr;
@@ -1083,8 +1136,10 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   } else {
     enqueue();
   }
-  if (out) hip_check(hipMemcpyAsync(out, P->outbuf.p, (size_t)nb * R * 16, hipMemcpyDeviceToHost, stream), "copy out");
-  hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  if (out && !pin_out) hip_check(hipMemcpyAsync(out, P->outbuf.p, nout_bytes, hipMemcpyDeviceToHost, stream), "copy out");
+  // (results that stay on the device: the caller's next launches are ordered after these)
+  if (out || tuner || P->opt_profile) hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  if (pin_out) std::memcpy(out, pin_results, nout_bytes);
   if (tuner) finish_tuning(P, L, *tuner);
   collect_profile(P, L);
 }
@@ -1205,14 +1260,19 @@ void sample_rejection(qx_plan *P, int64_t num_samples, uint64_t seed, double M, 
   hipStream_t stream = P->ctx->stream;
   int64_t nslices = 1;
   for (int64_t d : P->prog.var_dims) nslices *= d;
-  DevBuf obits, oamps, st;
-  obits.reserve(std::max<size_t>((size_t)num_samples * nch, 16));
-  oamps.reserve(std::max<size_t>((size_t)num_samples * 16, 16));
-  st.reserve(32);
-  int64_t cnt[2] = {0, 0};
-  double state[2] = {M, 0.0};
-  hip_check(hipMemcpyAsync(st.p, state, 8, hipMemcpyHostToDevice, stream), "copy");
-  hip_check(hipMemcpyAsync((char *)st.p + 16, cnt, 16, hipMemcpyHostToDevice, stream), "copy");
+  // M and the counters (accepted, used) in pinned memory, where the test's kernel updates
+  // them; the accepted samples too where they fit
+  char *const pin = P->pinned();
+  double *const state = (double *)(pin + kPinBits);
+  int64_t *const cnt = (int64_t *)(pin + kPinBits + 16);
+  state[0] = M;
+  cnt[0] = cnt[1] = 0;
+  const size_t bytes_amps = (size_t)num_samples * 16, bytes_bits = (size_t)num_samples * nch;
+  const bool fits = bytes_amps + bytes_bits <= kPinOut;
+  DevBuf far;
+  if (!fits) far.reserve(bytes_amps + bytes_bits);
+  char *const oamps = fits ? pin + kPinBits + kPinState : (char *)far.p;
+  char *const obits = oamps + bytes_amps;
   const double scale = std::ldexp(1.0, nch);
   try {
     while (cnt[0] < num_samples && cnt[1] < max_candidates) {
@@ -1220,25 +1280,21 @@ void sample_rejection(qx_plan *P, int64_t num_samples, uint64_t seed, double M, 
       stage_bits(P, nb, seed, cnt[1]);
       amplitudes(P, nullptr, nb, 0, nslices, nullptr, true);
       qx::launch_reject((const double *)P->outbuf.p, (const char *)P->bits.p, nb, nch, seed, cnt[1], scale, fix_m,
-                        num_samples, (double *)st.p, (int64_t *)((char *)st.p + 16), (char *)obits.p,
-                        (double *)oamps.p, stream);
-      hip_check(hipMemcpyAsync(cnt, (char *)st.p + 16, 16, hipMemcpyDeviceToHost, stream), "copy");
-      hip_check(hipMemcpyAsync(state, st.p, 8, hipMemcpyDeviceToHost, stream), "copy");
+                        num_samples, state, cnt, obits, (double *)oamps, stream);
       hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
     }
-    if (cnt[0] > 0) {
-      hip_check(hipMemcpy(bits_out, obits.p, (size_t)cnt[0] * nch, hipMemcpyDeviceToHost), "copy out");
-      hip_check(hipMemcpy(amps_out, oamps.p, (size_t)cnt[0] * 16, hipMemcpyDeviceToHost), "copy out");
+    if (cnt[0] > 0 && fits) {
+      std::memcpy(bits_out, obits, (size_t)cnt[0] * nch);
+      std::memcpy(amps_out, oamps, (size_t)cnt[0] * 16);
+    } else if (cnt[0] > 0) {
+      hip_check(hipMemcpy(bits_out, obits, (size_t)cnt[0] * nch, hipMemcpyDeviceToHost), "copy out");
+      hip_check(hipMemcpy(amps_out, oamps, (size_t)cnt[0] * 16, hipMemcpyDeviceToHost), "copy out");
     }
   } catch (...) {
-    obits.release();
-    oamps.release();
-    st.release();
+    far.release();
     throw;
   }
-  obits.release();
-  oamps.release();
-  st.release();
+  far.release();
   if (m_out) *m_out = state[0];
   if (cand_out) *cand_out = cnt[1];
   if (cnt[0] < num_samples)
@@ -1437,9 +1493,18 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   moved |= P->ampcot.reserve((size_t)nb * R * 16);
   if (!norm)
     hip_check(hipMemcpyAsync(P->ampcot.p, amp_cot, (size_t)nb * R * 16, hipMemcpyHostToDevice, stream), "copy");
-  size_t nbits = (size_t)nb * nch;
-  moved |= P->bits.reserve(std::max<size_t>(nbits, 16));
-  if (nbits) hip_check(hipMemcpyAsync(P->bits.p, bits, nbits, hipMemcpyHostToDevice, stream), "copy");
+  // bitstrings, amplitudes and gradient through the plan's pinned block where they fit
+  const size_t nbits = (size_t)nb * nch, amp_bytes = (size_t)nb * R * 16, grad_bytes = (size_t)ke * 16;
+  const bool pin_bits = nbits <= kPinBits, pin_amps = norm && amp_bytes <= kPinOut / 2, pin_grad = grad_bytes <= kPinOut / 2;
+  char *const pin_out = P->pinned() + kPinBits + kPinState;
+  if (pin_bits) {
+    std::memcpy(P->pin, bits, nbits);
+  } else {
+    moved |= P->bits.reserve(nbits);
+    hip_check(hipMemcpyAsync(P->bits.p, bits, nbits, hipMemcpyHostToDevice, stream), "copy");
+  }
+  const char *const d_bits = pin_bits ? P->pin : (const char *)P->bits.p;
+  double *const d_amps = pin_amps ? (double *)(pin_out + kPinOut / 2) : (double *)P->ampcot.p;
   std::vector<int64_t> ooff;
   std::vector<int> oq;
   for (int o : P->prog.outputs) {
@@ -1640,12 +1705,11 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
       int64_t nvalid = std::min<int64_t>(batch, nb - row0);
       zero_cots(2);
       qx::launch_fill_outputs(P->prec, bs.arena, (const int64_t *)P->out_off.p, nout, (const int *)P->out_q.p,
-                              (const char *)P->bits.p + row0 * nch, nvalid, batch, nch, stream);
+                              d_bits + row0 * nch, nvalid, batch, nch, stream);
       run_fwd(2);
       if (norm)
         qx::launch_root_cot_norm(P->prec, value_ptr(P, rc, varval, bs), value_ptr(P, rv, varval, bs), rc.beta_stride,
-                                 batch, nvalid, R, (const int64_t *)P->relem_off.p, (double *)P->ampcot.p, row0,
-                                 stream);
+                                 batch, nvalid, R, (const int64_t *)P->relem_off.p, d_amps, row0, stream);
       else
         qx::launch_root_cot(P->prec, value_ptr(P, rc, varval, bs), rc.dep ? rc.beta_stride : 0, batch, nvalid, R,
                             (const int64_t *)P->relem_off.p, (const double *)P->ampcot.p, row0, stream);
@@ -1688,10 +1752,13 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   } else {
     enqueue();
   }
-  hip_check(hipMemcpyAsync(grad, P->grad.p, (size_t)ke * 16, hipMemcpyDeviceToHost, stream), "copy out");
-  if (norm)
-    hip_check(hipMemcpyAsync(amps_out, P->ampcot.p, (size_t)nb * R * 16, hipMemcpyDeviceToHost, stream), "copy out");
+  hip_check(hipMemcpyAsync(pin_grad ? (void *)pin_out : grad, P->grad.p, grad_bytes, hipMemcpyDeviceToHost, stream),
+            "copy out");
+  if (norm && !pin_amps)
+    hip_check(hipMemcpyAsync(amps_out, P->ampcot.p, amp_bytes, hipMemcpyDeviceToHost, stream), "copy out");
   hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  if (pin_grad) std::memcpy(grad, pin_out, grad_bytes);
+  if (pin_amps) std::memcpy(amps_out, d_amps, amp_bytes);
 }
 
 std::string stats_json(const qx_plan *P) {
@@ -1806,6 +1873,7 @@ void qx_ctx_destroy(qx_ctx *ctx) {
   if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
   if (ctx->blas_ws) (void)hipFree(ctx->blas_ws);
   if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+  for (void *p : ctx->pins) (void)hipHostFree(p);
   delete ctx;
 }
 

@@ -30,6 +30,9 @@ hipError_t hipGetDeviceCount(int *count);
 const char *hipGetErrorString(hipError_t e);
 hipError_t hipMalloc(void **p, size_t bytes);
 hipError_t hipFree(void *p);
+#define hipHostMallocDefault 0u
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned flags);
+hipError_t hipHostFree(void *p);
 hipError_t hipMemGetInfo(size_t *free_bytes, size_t *total_bytes);
 hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind kind);
 hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind kind, hipStream_t s);

@@ -50,6 +50,7 @@ namespace {
 
 std::recursive_mutex g_mu;
 std::map<uintptr_t, size_t> g_allocs;   // base -> bytes of every live device allocation
+std::map<uintptr_t, size_t> g_pinned;   // those of them that are pinned host memory
 double g_clock = 0;                     // simulated time of recorded events
 int64_t g_launches = 0;                 // kernel launches checked (eager or replayed)
 
@@ -155,6 +156,26 @@ hipError_t hipFree(void *p) {
   return hipSuccess;
 }
 
+// pinned host memory: the device reaches it like an allocation of its own
+hipError_t hipHostMalloc(void **p, size_t bytes, unsigned) {
+  const hipError_t e = hipMalloc(p, bytes);
+  std::lock_guard<std::recursive_mutex> lk(g_mu);
+  if (e == hipSuccess) g_pinned[(uintptr_t)*p] = bytes;
+  return e;
+}
+hipError_t hipHostFree(void *p) {
+  {
+    std::lock_guard<std::recursive_mutex> lk(g_mu);
+    g_pinned.erase((uintptr_t)p);
+  }
+  return hipFree(p);
+}
+static bool is_pinned(const void *p) {
+  std::lock_guard<std::recursive_mutex> lk(g_mu);
+  auto it = g_pinned.upper_bound((uintptr_t)p);
+  return it != g_pinned.begin() && (uintptr_t)p < (--it)->first + it->second;
+}
+
 hipError_t hipMemGetInfo(size_t *free_bytes, size_t *total_bytes) {
   *total_bytes = size_t(288) << 30;
   *free_bytes = size_t(280) << 30;
@@ -165,8 +186,8 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
   submit(s, [=]() {
     if (kind == hipMemcpyHostToDevice || kind == hipMemcpyDeviceToDevice) need(dst, bytes, "copy destination");
     if (kind == hipMemcpyDeviceToHost || kind == hipMemcpyDeviceToDevice) need(src, bytes, "copy source");
-    if (kind == hipMemcpyHostToDevice && is_device(src)) violation("host-to-device copy from device memory");
-    if (kind == hipMemcpyDeviceToHost && is_device(dst)) violation("device-to-host copy into device memory");
+    if (kind == hipMemcpyHostToDevice && is_device(src) && !is_pinned(src)) violation("host-to-device copy from device memory");
+    if (kind == hipMemcpyDeviceToHost && is_device(dst) && !is_pinned(dst)) violation("device-to-host copy into device memory");
     if (bytes) std::memmove(dst, src, bytes);
   });
   return hipSuccess;
@@ -468,19 +489,14 @@ long double root_reach(const int64_t *d_relem_off, int64_t relems, int64_t bstri
 }  // namespace
 
 void launch_accumulate(int prec, const void *root, int64_t root_bstride, int64_t batch, int64_t nvalid,
-                       int64_t relems, const int64_t *d_relem_off, double *acc, int64_t row0, void *stream) {
+                       int64_t relems, const int64_t *d_relem_off, double *acc, double *out, int64_t row0, bool first,
+                       bool last, void *stream) {
   const size_t es = esize(prec);
   if (nvalid > batch) violation("accumulate: more valid rows than the batch");
   launch(stream, [=]() {
     need(root, root_reach(d_relem_off, relems, root_bstride, nvalid) * es, "saved tensor");
-    need(acc, (long double)(row0 + nvalid) * relems * 32, "accumulators");
-  });
-}
-
-void launch_finalize(const double *acc, double *out, int64_t n, void *stream) {
-  launch(stream, [=]() {
-    need(acc, (long double)n * 32, "accumulators");
-    need(out, (long double)n * 16, "results");
+    if (!first || !last) need(acc, (long double)(row0 + nvalid) * relems * 32, "accumulators");
+    if (last) need(out, (long double)(row0 + nvalid) * relems * 16, "results");
   });
 }
 
