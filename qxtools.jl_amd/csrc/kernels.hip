@@ -1507,24 +1507,29 @@ __global__ void k_plain_sum(typename Vec<T>::type *__restrict__ C, const typenam
 // (re hi, re lo, im hi, im lo) laid out [m][k] / [n][k], a row's 16-byte chunks
 // XOR-permuted by the row, so a lane's fragment (8 consecutive k values of one row) is
 // one 16-byte LDS read.
-// Tiles of 64 x 64 of C per workgroup (2 x 2 waves of 2 x 2 blocks), K stages of 32,
-// the next stage fetched into registers during the products; K split and unit order as
+// Tiles of 32 BI x 64 of C per workgroup (2 x 2 waves of BI x 2 blocks), K stages of 32,
+// the next stage fetched into registers during the products; 7x7 open batch's largest step
+// (4.4 TF complex): rounding value by value on 64 x 64 tiles 16.5 ms, bound by the vector
+// unit and by LDS reads (six fragments per four blocks' products), packed conversions on
+// 128 x 64 12.4 ms (1.06 PFLOP/s); 16-byte loads of pairs along k changed nothing; K split and unit order as
 // in k_plain_gemm.  A lane's k slot is the same in both operands, so the products pair
 // equal k whatever order the matrix core sums them in; the result layout is that of
 // the 16x16x4 FP32 product (Mfma16<float>).
-template <int OPX, int OPY>
+template <int OPX, int OPY, int BI>
 __global__ __launch_bounds__(256) void k_plain_gemm_bf16x3(const float2 *__restrict__ X, const float2 *__restrict__ Y,
                                                            float2 *__restrict__ C, float2 *__restrict__ ws,
                                                            BlasArgs b) {
   typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
+  typedef __bf16 bf2 __attribute__((ext_vector_type(2)));
   typedef float f4 __attribute__((ext_vector_type(4)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
   // a row of a plane: 16 dwords (32 bf16 values of k) in four 16-byte chunks, chunk c
   // of row r stored at chunk c ^ ((r >> 2) & 3): the 16 rows a fragment read spans
   // (one chunk each) and the 4 rows x 16 dwords a wave stores with lanes along k both
   // fall on distinct banks
-  constexpr int TM = 64, TN = 64, TK = 32, RW = TK / 2;
+  constexpr int TM = 32 * BI, TN = 64, TK = 32, RW = TK / 2, PA = 2 * BI, PB = 4;   // k pairs per thread
   auto slot = [](int row, int dw) { return dw ^ (((row >> 2) & 3) << 2); };
-  constexpr int BI = 2, BJ = 2, NP = 4;                           // planes: rh, rl, ih, il
+  constexpr int BJ = 2, NP = 4;                                   // planes: rh, rl, ih, il
   __shared__ uint32_t sA[NP][TM][RW];
   __shared__ uint32_t sB[NP][TN][RW];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1547,75 +1552,65 @@ __global__ __launch_bounds__(256) void k_plain_gemm_bf16x3(const float2 *__restr
   const int64_t m0 = rt * TM, n0 = st * TN;
   const int64_t stages = b.k / TK / b.ksplit;
   const int64_t k0 = ks * stages * TK;
-  // four k pairs per thread and operand: (row, pair) of each, and the two elements'
-  // offsets inside a stage
-  int ra_row[4], ra_pair[4], rb_row[4], rb_pair[4];
-  int64_t oa0[4], oa1[4], ob0[4], ob1[4];
-  bool oka[4], okb[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    int m, p;
-    if (OPX) p = tid % 16, m = tid / 16 + 16 * j;   // k contiguous in X: lanes along k
-    else m = tid % 64, p = tid / 64 + 4 * j;        // m contiguous in X: lanes along m
-    ra_row[j] = m, ra_pair[j] = p;
-    oka[j] = m0 + m < b.r;
-    const int64_t kk = 2 * p;
-    oa0[j] = OPX ? kk + (m0 + m) * b.ldx : (m0 + m) + kk * b.ldx;
-    oa1[j] = OPX ? oa0[j] + 1 : oa0[j] + b.ldx;
-    int n, q;
-    if (OPY) n = tid % 64, q = tid / 64 + 4 * j;    // Y stored n x k: lanes along n
-    else q = tid % 16, n = tid / 16 + 16 * j;       // Y stored k x n: lanes along k
-    rb_row[j] = n, rb_pair[j] = q;
-    okb[j] = n0 + n < b.s;
-    const int64_t kq = 2 * q;
-    ob0[j] = OPY ? (n0 + n) + kq * b.ldy : kq + (n0 + n) * b.ldy;
-    ob1[j] = OPY ? ob0[j] + b.ldy : ob0[j] + 1;
-  }
-  const float2 *Xb = X + bat * b.sx + (OPX ? k0 : k0 * b.ldx);
-  const float2 *Yb = Y + bat * b.sy + (OPY ? k0 * b.ldy : k0);
+  // a thread's first k pair of X and of Y (row, pair) and its element offset inside a
+  // stage; the next ones and a pair's second value lie at wave-uniform distances
+  const int ma = OPX ? tid / 16 : tid % TM, pa = OPX ? tid % 16 : tid / TM;   // lanes along X's contiguous index
+  const int nb0 = OPY ? tid % TN : tid / 16, qb = OPY ? tid / TN : tid % 16;
+  constexpr int pa_step = OPX ? 0 : 256 / TM, ma_step = OPX ? 16 : 0, qb_step = OPY ? 256 / TN : 0, nb_step = OPY ? 0 : 16;
+  const float2 *xa = X + bat * b.sx + (OPX ? k0 : k0 * b.ldx) + (OPX ? 2 * pa + (m0 + ma) * b.ldx : (m0 + ma) + 2 * pa * b.ldx);
+  const float2 *yb = Y + bat * b.sy + (OPY ? k0 * b.ldy : k0) + (OPY ? (n0 + nb0) + 2 * qb * b.ldy : 2 * qb + (n0 + nb0) * b.ldy);
+  const int64_t xj = OPX ? 16 * b.ldx : 2 * pa_step * b.ldx, x1 = OPX ? 1 : b.ldx;
+  const int64_t yj = OPY ? 2 * qb_step * b.ldy : 16 * b.ldy, y1 = OPY ? b.ldy : 1;
   const int64_t xstep = OPX ? TK : TK * b.ldx, ystep = OPY ? TK * b.ldy : TK;
-  float2 xa0[4], xa1[4], yb0[4], yb1[4];
-  auto fetch = [&](int64_t sg) {
-    const float2 *xa = Xb + sg * xstep;
-    const float2 *yb = Yb + sg * ystep;
+  float2 xa0[PA], xa1[PA], yb0[PB], yb1[PB];
+  auto fetch = [&]() {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      xa0[j] = oka[j] ? xa[oa0[j]] : float2{0, 0};
-      xa1[j] = oka[j] ? xa[oa1[j]] : float2{0, 0};
-      yb0[j] = okb[j] ? yb[ob0[j]] : float2{0, 0};
-      yb1[j] = okb[j] ? yb[ob1[j]] : float2{0, 0};
+    for (int j = 0; j < PA; ++j) {
+      const bool ok = m0 + ma + ma_step * j < b.r;
+      xa0[j] = ok ? xa[j * xj] : float2{0, 0};
+      xa1[j] = ok ? xa[j * xj + x1] : float2{0, 0};
     }
+#pragma unroll
+    for (int j = 0; j < PB; ++j) {
+      const bool ok = n0 + nb0 + nb_step * j < b.s;
+      yb0[j] = ok ? yb[j * yj] : float2{0, 0};
+      yb1[j] = ok ? yb[j * yj + y1] : float2{0, 0};
+    }
+    xa += xstep, yb += ystep;
   };
-  // (hi, lo) planes of a pair of values adjacent in k, packed two per dword
-  auto split_store = [&](uint32_t (*pl)[TM][RW], int row, int pair, float2 v0, float2 v1) {
-    const uint16_t rh0 = bf16_bits(v0.x), rh1 = bf16_bits(v1.x), ih0 = bf16_bits(v0.y), ih1 = bf16_bits(v1.y);
+  // (hi, lo) planes of a pair of values adjacent in k, packed two per dword by the packed
+  // conversion (nearest, ties to even)
+  auto pack = [](float v0, float v1) { return __builtin_bit_cast(uint32_t, __builtin_convertvector((f2{v0, v1}), bf2)); };
+  auto split_store = [&](auto pl, int row, int pair, float2 v0, float2 v1) {
+    const uint32_t rh = pack(v0.x, v1.x), ih = pack(v0.y, v1.y);
     const int d = slot(row, pair);
-    pl[0][row][d] = (uint32_t)rh0 | ((uint32_t)rh1 << 16);
-    pl[1][row][d] = (uint32_t)bf16_bits(v0.x - bf16_value(rh0)) | ((uint32_t)bf16_bits(v1.x - bf16_value(rh1)) << 16);
-    pl[2][row][d] = (uint32_t)ih0 | ((uint32_t)ih1 << 16);
-    pl[3][row][d] = (uint32_t)bf16_bits(v0.y - bf16_value(ih0)) | ((uint32_t)bf16_bits(v1.y - bf16_value(ih1)) << 16);
+    auto low = [](uint32_t h) { return __uint_as_float(h << 16); };
+    auto high = [](uint32_t h) { return __uint_as_float(h & 0xFFFF0000u); };
+    pl[0][row][d] = rh;
+    pl[1][row][d] = pack(v0.x - low(rh), v1.x - high(rh));
+    pl[2][row][d] = ih;
+    pl[3][row][d] = pack(v0.y - low(ih), v1.y - high(ih));
   };
   f4 accr[BI][BJ], acci[BI][BJ];
 #pragma unroll
   for (int i = 0; i < BI; ++i)
 #pragma unroll
     for (int j = 0; j < BJ; ++j) accr[i][j] = f4{0, 0, 0, 0}, acci[i][j] = f4{0, 0, 0, 0};
-  auto frag = [&](const uint32_t (*pl)[TM][RW], int plane, int row) {
+  auto frag = [&](auto pl, int plane, int row) {
     const uint4 v = *reinterpret_cast<const uint4 *>(&pl[plane][row][slot(row, 4 * lq)]);
     return v;
   };
   auto as_bf8 = [](uint4 v) { return __builtin_bit_cast(bf8, v); };
   auto neg = [](uint4 v) { return uint4{v.x ^ 0x80008000u, v.y ^ 0x80008000u, v.z ^ 0x80008000u, v.w ^ 0x80008000u}; };
-  fetch(0);
+  fetch();
   for (int64_t sg = 0; sg < stages; ++sg) {
     __syncthreads();
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      split_store(sA, ra_row[j], ra_pair[j], xa0[j], xa1[j]);
-      split_store(sB, rb_row[j], rb_pair[j], yb0[j], yb1[j]);
-    }
+    for (int j = 0; j < PA; ++j) split_store(sA, ma + ma_step * j, pa + pa_step * j, xa0[j], xa1[j]);
+#pragma unroll
+    for (int j = 0; j < PB; ++j) split_store(sB, nb0 + nb_step * j, qb + qb_step * j, yb0[j], yb1[j]);
     __syncthreads();
-    if (sg + 1 < stages) fetch(sg + 1);
+    if (sg + 1 < stages) fetch();
     bf8 yrh[BJ], yrl[BJ], yih[BJ], yil[BJ];
 #pragma unroll
     for (int j = 0; j < BJ; ++j) {
@@ -1627,7 +1622,7 @@ __global__ __launch_bounds__(256) void k_plain_gemm_bf16x3(const float2 *__restr
     }
 #pragma unroll
     for (int i = 0; i < BI; ++i) {
-      const int row = 32 * wm + 16 * i + li;
+      const int row = 16 * BI * wm + 16 * i + li;
       const uint4 ih = frag(sA, 2, row), il = frag(sA, 3, row);
       const bf8 xrh = as_bf8(frag(sA, 0, row)), xrl = as_bf8(frag(sA, 1, row));
       const bf8 xih = as_bf8(ih), xil = as_bf8(il), nxih = as_bf8(neg(ih)), nxil = as_bf8(neg(il));
@@ -1660,7 +1655,7 @@ __global__ __launch_bounds__(256) void k_plain_gemm_bf16x3(const float2 *__restr
       const int64_t n = n0 + 32 * wn + 16 * j + li;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        const int64_t m = m0 + 32 * wm + 16 * i + Mfma16<float>::row(lq, e);
+        const int64_t m = m0 + 16 * BI * wm + 16 * i + Mfma16<float>::row(lq, e);
         if (m < b.r && n < b.s) dst[m + n * ld] = float2{accr[i][j][e], acci[i][j][e]};
       }
     }
@@ -3131,12 +3126,24 @@ void launch_plain_gemm(int prec, const void *X, const void *Y, void *C, void *ws
   }
   if (b.split) {
     if (prec == QX_C128) throw Error(QX_ERR_STATE, "internal: split bf16 product of complex128 operands");
-    switch (sel) {
-      case 0: hipLaunchKernelGGL((k_plain_gemm_bf16x3<0, 0>), g, dim3(256), 0, s, (const float2 *)X, (const float2 *)Y, (float2 *)C, (float2 *)ws, b); break;
-      case 1: hipLaunchKernelGGL((k_plain_gemm_bf16x3<0, 1>), g, dim3(256), 0, s, (const float2 *)X, (const float2 *)Y, (float2 *)C, (float2 *)ws, b); break;
-      case 2: hipLaunchKernelGGL((k_plain_gemm_bf16x3<1, 0>), g, dim3(256), 0, s, (const float2 *)X, (const float2 *)Y, (float2 *)C, (float2 *)ws, b); break;
-      default: hipLaunchKernelGGL((k_plain_gemm_bf16x3<1, 1>), g, dim3(256), 0, s, (const float2 *)X, (const float2 *)Y, (float2 *)C, (float2 *)ws, b); break;
+    const int64_t wide = b.batch * ((b.r + 127) / 128) * ((b.s + 63) / 64) * b.ksplit;
+#define QX_SPLIT(OX, OY, BI_, G)                                                                                  \
+  hipLaunchKernelGGL((k_plain_gemm_bf16x3<OX, OY, BI_>), dim3((unsigned)(G)), dim3(256), 0, s, (const float2 *)X, \
+                     (const float2 *)Y, (float2 *)C, (float2 *)ws, b)
+#define QX_SPLIT_OPS(BI_, G)                    \
+  switch (sel) {                                \
+    case 0: QX_SPLIT(0, 0, BI_, G); break;      \
+    case 1: QX_SPLIT(0, 1, BI_, G); break;      \
+    case 2: QX_SPLIT(1, 0, BI_, G); break;      \
+    default: QX_SPLIT(1, 1, BI_, G); break;     \
+  }
+    if (wide >= 512) {   // 128 rows where that leaves two workgroups per CU (what its registers hold)
+      QX_SPLIT_OPS(4, wide)
+    } else {
+      QX_SPLIT_OPS(2, units)
     }
+#undef QX_SPLIT_OPS
+#undef QX_SPLIT
   } else if (prec == QX_C128) {
     if (b.gauss) {
       QX_PLAIN_OPS(double, double2, true)
