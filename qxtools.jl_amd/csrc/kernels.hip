@@ -614,6 +614,35 @@ __global__ void k_sum_splits(typename Vec<T>::type *__restrict__ C, const typena
   }
 }
 
+// The same for few elements: 16 lanes per element, each summing every sixteenth partial,
+// then over the 16 through LDS.  With one lane per element and n <= 256 one workgroup waited
+// for ksplit dependent rounds of loads (8 slices of the 6x6 plan, complex128: 31.2 us, 4.6 so).
+constexpr int kSumLanes = 16;
+template <typename T>
+__global__ __launch_bounds__(256) void k_sum_splits_few(typename Vec<T>::type *__restrict__ C,
+                                                        const typename Vec<T>::type *__restrict__ ws, int64_t n,
+                                                        int ksplit) {
+  using V = typename Vec<T>::type;
+  constexpr int E = 256 / kSumLanes;   // elements per workgroup
+  __shared__ V part[kSumLanes][E];
+  const int el = threadIdx.x % E, p = threadIdx.x / E;
+  const int64_t i = (int64_t)blockIdx.x * E + el;
+  V acc{0, 0};
+  if (i < n) {
+#pragma unroll 4
+    for (int s = p; s < ksplit; s += kSumLanes) {
+      const V v = ws[(int64_t)s * n + i];
+      acc.x += v.x;
+      acc.y += v.y;
+    }
+  }
+  part[p][el] = acc;
+  __syncthreads();
+  if (p != 0 || i >= n) return;
+  for (int q = 1; q < kSumLanes; ++q) acc.x += part[q][el].x, acc.y += part[q][el].y;
+  C[i] = acc;
+}
+
 // One wave per C element and K range, lanes along K (the larger operand's smallest
 // strides first), shuffle reduction.  Bound by HBM reads: four terms per lane are loaded
 // before they are used, and the offsets of the next four come from one table entry per
@@ -1063,6 +1092,22 @@ void check_launch(const char *what) {
   if (e != hipSuccess) throw Error(QX_ERR_DEVICE, std::string(what) + ": " + hipGetErrorString(e));
 }
 
+// Few: at least 8 partials of up to 2^14 elements, whose lanes would not give each CU a
+// workgroup.
+void launch_sum_splits(int prec, void *C, const void *ws, int64_t n, int ksplit, hipStream_t s) {
+  const bool few = ksplit >= 8 && n <= (int64_t(1) << 14);
+  const int g = grid_for(n, few ? 256 / kSumLanes : 256);
+  if (prec == QX_C128) {
+    if (few) hipLaunchKernelGGL(k_sum_splits_few<double>, dim3(g), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, n, ksplit);
+    else hipLaunchKernelGGL(k_sum_splits<double>, dim3(g), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, n, ksplit);
+  } else {
+    if (few) hipLaunchKernelGGL(k_sum_splits_few<float>, dim3(g), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, n, ksplit);
+    else hipLaunchKernelGGL(k_sum_splits<float>, dim3(g), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, n, ksplit);
+  }
+  check_launch("sum_splits");
+}
+
+
 
 template <int TM, int TN, int TK>
 void gemm_launch(int prec, const void *A, const void *B, void *C, const GemmArgs &a, hipStream_t s) {
@@ -1281,14 +1326,7 @@ void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void 
   else mfma_launch<float, false>(X, Y, dst, b, g, s);
   check_launch("contract_gemm_mfma");
   if (a.ksplit > 1) {
-    const int gs = grid_for(a.c_elems, 256);
-    if (prec == QX_C128)
-      hipLaunchKernelGGL(k_sum_splits<double>, dim3(gs), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, a.c_elems,
-                         a.ksplit);
-    else
-      hipLaunchKernelGGL(k_sum_splits<float>, dim3(gs), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, a.c_elems,
-                         a.ksplit);
-    check_launch("sum_splits");
+    launch_sum_splits(prec, C, ws, a.c_elems, a.ksplit, s);
   }
 }
 
@@ -1303,14 +1341,7 @@ void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void 
   }
   check_launch("contract_gemm");
   if (args.ksplit > 1) {
-    int g = grid_for(args.c_elems, 256);
-    if (prec == QX_C128)
-      hipLaunchKernelGGL(k_sum_splits<double>, dim3(g), dim3(256), 0, s, (double2 *)C, (const double2 *)ws,
-                         args.c_elems, args.ksplit);
-    else
-      hipLaunchKernelGGL(k_sum_splits<float>, dim3(g), dim3(256), 0, s, (float2 *)C, (const float2 *)ws,
-                         args.c_elems, args.ksplit);
-    check_launch("sum_splits");
+    launch_sum_splits(prec, C, ws, args.c_elems, args.ksplit, s);
   }
 }
 
@@ -1791,14 +1822,7 @@ void launch_contract_reduce(int prec, const void *A, const void *B, void *C, voi
   }
   check_launch("contract_reduce");
   if (args.ksplit > 1) {
-    int gs = grid_for(c_elems, 256);
-    if (prec == QX_C128)
-      hipLaunchKernelGGL(k_sum_splits<double>, dim3(gs), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, c_elems,
-                         args.ksplit);
-    else
-      hipLaunchKernelGGL(k_sum_splits<float>, dim3(gs), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, c_elems,
-                         args.ksplit);
-    check_launch("sum_splits");
+    launch_sum_splits(prec, C, ws, c_elems, args.ksplit, s);
   }
 }
 
@@ -1816,14 +1840,7 @@ void launch_contract_bits(int prec, const void *A, const void *B, void *C, void 
                        (float2 *)dst, c_elems, args);
   check_launch("contract_bits");
   if (args.ksplit > 1) {
-    int gs = grid_for(c_elems, 256);
-    if (prec == QX_C128)
-      hipLaunchKernelGGL(k_sum_splits<double>, dim3(gs), dim3(256), 0, s, (double2 *)C, (const double2 *)ws, c_elems,
-                         args.ksplit);
-    else
-      hipLaunchKernelGGL(k_sum_splits<float>, dim3(gs), dim3(256), 0, s, (float2 *)C, (const float2 *)ws, c_elems,
-                         args.ksplit);
-    check_launch("sum_splits");
+    launch_sum_splits(prec, C, ws, c_elems, args.ksplit, s);
   }
 }
 
