@@ -1290,6 +1290,19 @@ void mfma_launch(const void *X, const void *Y, void *C, const MfmaArgs &a, int g
     case 2: QX_MFMA(2, 2, 1); break;
     case 3: QX_MFMA(1, 1, 2); break;
     case 4: QX_MFMA(4, 2, 1); break;
+    case 5:
+    case 6:   // complex64 in four products, stages of 16 (mfma_args)
+      if constexpr (std::is_same_v<T, float> && !GAUSS) {
+        if (a.kk != 16) throw Error(QX_ERR_STATE, "internal: matrix-core tile");
+        if (a.cfg == 5)
+          hipLaunchKernelGGL((k_contract_gemm_mfma<T, GAUSS, 2, 4, 2, 16>), dim3(g), dim3(256), pad, s, (const V *)X,
+                             (const V *)Y, (V *)C, a);
+        else
+          hipLaunchKernelGGL((k_contract_gemm_mfma<T, GAUSS, 2, 2, 4, 16>), dim3(g), dim3(256), pad, s, (const V *)X,
+                             (const V *)Y, (V *)C, a);
+        break;
+      }
+      [[fallthrough]];
     default: throw Error(QX_ERR_STATE, "internal: matrix-core tile");
   }
 #undef QX_MFMA

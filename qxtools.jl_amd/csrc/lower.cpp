@@ -294,7 +294,7 @@ bool plain_gemm(const Step &st, BlasArgs &b) {
 }
 // Arguments of the matrix-core GEMM on operands of any layout.  The operand that holds
 // the lowest of C's M and N bits becomes Y (C's columns, which the result lanes walk;
-// `other`: the other one), the tile is 64 x 64 or, where a side has fewer values, the
+// `other`: the other one), the tile is 64 x 64 (128 on a side: below) or, where a side has fewer values, the
 // narrower shape that wastes least.  Tile bits: first those below a 128-byte line of X, Y
 // and C (lowest first, so each line is read and written by one workgroup), then each
 // operand's next smallest strides.
@@ -320,7 +320,12 @@ bool mfma_args(const StepBits &sb, int precision, bool other, int64_t c_elems, M
   auto count = [&](char cls) { return (int)std::count_if(bits.begin(), bits.end(), [&](const Bit &b) { return b.cls == cls; }); };
   const int nm = count('M'), nn = count('N'), nk = count('K');
   // tile shape
-  if (nm >= 6 && nn >= 6) g.cfg = 0;
+  // complex64 in four products with K >= 64 and at least 1024 such tiles: a side of 128
+  // (three products' accumulators do not fit the registers).  A 64 x 64 tile's operands
+  // take 4.8 TB/s from the caches at the FP32 rate, two thirds or half of that so: 512
+  // strings of the 6x6 plan 12.34 -> 12.09 ms, 7x7 split bf16 35.16 -> 34.61
+  const bool big = (precision == QX_C64_4M || precision == QX_C64_BF16X3) && nk >= 6 && count('H') + nm + nn >= 23;
+  if (nm >= 6 && nn >= 6) g.cfg = big && nm >= 7 ? 5 : big && nn >= 7 ? 6 : 0;
   else if (nm <= 4 && nm <= nn) g.cfg = 3;
   else if (nn <= 4) g.cfg = 4;
   else g.cfg = nm <= nn ? 1 : 2;

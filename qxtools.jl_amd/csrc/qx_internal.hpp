@@ -244,7 +244,8 @@ struct GemmArgs {
 // order -- the low 8 the lane, the rest its registers -- each with its stride and its LDS
 // slot increment.  Unit bits (tiles, batch elements, K splits) in C order, stage bits in X
 // order.  cm / cn: C strides of the tile's row and column index bits.
-constexpr int kMfmaTiles[5][2] = {{64, 64}, {32, 64}, {64, 32}, {16, 128}, {128, 16}};   // rows, columns
+constexpr int kMfmaTileCount = 7;
+constexpr int kMfmaTiles[kMfmaTileCount][2] = {{64, 64}, {32, 64}, {64, 32}, {16, 128}, {128, 16}, {128, 64}, {64, 128}};   // rows, columns
 constexpr int kMfmaStageBits = 4;   // log2 of a stage's k values
 constexpr int kMfmaTileBits = 11;   // bits of a 128 x 16 stage
 // Elements between consecutive k of a tile in LDS: complex64 rows 136 bytes apart modulo

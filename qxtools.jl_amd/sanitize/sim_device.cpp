@@ -398,7 +398,7 @@ void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void 
 
 void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &g, void *stream) {
   const size_t es = esize(prec);
-  if (g.cfg < 0 || g.cfg >= 5 || g.nxb > kMfmaTileBits || g.nyb > kMfmaTileBits || g.nsb > kMaxBits || g.nub > kMaxBits)
+  if (g.cfg < 0 || g.cfg >= kMfmaTileCount || g.nxb > kMfmaTileBits || g.nyb > kMfmaTileBits || g.nsb > kMaxBits || g.nub > kMaxBits)
     violation("matrix-core GEMM arguments out of range");
   // LDS slots of the tile's elements, rows and columns of its results
   const int tm = kMfmaTiles[g.cfg][0], tn = kMfmaTiles[g.cfg][1], tk = g.kk;
