@@ -123,7 +123,9 @@ struct DevBuf {
   void upload(const void *src, size_t n, hipStream_t s) {
     if (held.size() == n && n > 0 && std::memcmp(held.data(), src, n) == 0) return;
     held.assign((const char *)src, (const char *)src + n);   // (the copy's source: it outlives the call)
-    hip_check(hipMemcpyAsync(p, held.data(), n, hipMemcpyHostToDevice, s), "copy");
+    const hipError_t e = hipMemcpyAsync(p, held.data(), n, hipMemcpyHostToDevice, s);
+    if (e != hipSuccess) held.clear();
+    hip_check(e, "copy");
   }
 };
 
