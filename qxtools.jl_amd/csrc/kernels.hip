@@ -1310,17 +1310,11 @@ void mfma_launch(const void *X, const void *Y, void *C, const MfmaArgs &a, int g
 
 }  // namespace
 
-// One unit per workgroup (units then start in C order as others end); K = 64 (four
-// stages) takes two, whose second first loads run during the first's products (7x7,
-// M 64, N 2048, 1024-fold, complex128: 1.30 -> 1.21 ms; longer K hides its first loads by
-// itself, shorter K lost 3-25% with two or more).
 void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &a, void *stream) {
   hipStream_t s = (hipStream_t)stream;
   const void *X = a.swap ? B : A, *Y = a.swap ? A : B;
   void *dst = a.ksplit > 1 ? ws : C;
-  const int q = a.nsb == 2 && a.nub > 12 ? 1 : 0;
-  if (a.nub - q > 30) throw Error(QX_ERR_STATE, "internal: matrix-core GEMM grid");
-  const int g = 1 << (a.nub - q);
+  const int q = mfma_trip_bits(a), g = 1 << (a.nub - q);
   MfmaArgs b = a;   // strides -> increments: of the stages, and of the unit bits a trip counter walks
   auto increments = [](int64_t *w, int n) {
     int64_t below = 0;

@@ -270,6 +270,17 @@ struct MfmaArgs {
   int64_t c_elems = 0;                  // dense C size: stride between K-split partials
 };
 static_assert(sizeof(MfmaArgs) <= 4000, "matrix-core GEMM arguments must fit the kernel argument segment");
+// A launch takes fewer than 2^32 lanes in a dimension of its grid: of 256 per workgroup, at
+// most 2^23 workgroups.
+constexpr int kMfmaGridBits = 23;
+// log2 of the units a workgroup walks.  One (units then start in C order as others end);
+// K = 64 (four stages) takes two, whose second first loads run during the first's products
+// (7x7, M 64, N 2048, 1024-fold, complex128: 1.30 -> 1.21 ms; longer K hides its first loads
+// by itself, shorter K lost 3-25% with two or more); more only where the grid has no room.
+inline int mfma_trip_bits(const MfmaArgs &a) {
+  const int q = a.nsb == 2 && a.nub > 12 ? 1 : 0;
+  return a.nub - q > kMfmaGridBits ? a.nub - kMfmaGridBits : q;
+}
 
 // One leg of a step in canonical form: dims and element strides in A, B and C.
 struct Leg {

@@ -1395,6 +1395,14 @@ std::string kern_variant(const qx::Step &st) {
   }
 }
 
+// The matrix-core GEMM's tile (rows, columns, k values of a stage), workgroups and units of each.
+void mfma_json(std::ostringstream &os, const qx::Step &st) {
+  if (st.kern != qx::Kern::Gemm || st.gemm.tile != 3) return;
+  const int q = qx::mfma_trip_bits(*st.mfma), *t = qx::kMfmaTiles[st.mfma->cfg];
+  os << ",\"tile\":[" << t[0] << "," << t[1] << "," << st.mfma->kk << "],\"workgroups\":"
+     << (int64_t(1) << (st.mfma->nub - q)) << ",\"units_per_workgroup\":" << (int64_t(1) << q);
+}
+
 void lowered_json(std::ostringstream &os, const qx::Program &prog, const qx::Lowered &L, int prec,
                   bool with_slots) {
   const size_t es = prec == QX_C128 ? 16 : 8;
@@ -1422,6 +1430,7 @@ void lowered_json(std::ostringstream &os, const qx::Program &prog, const qx::Low
        << ",\"M\":" << st.M << ",\"N\":" << st.N << ",\"K\":" << st.K << ",\"flops\":" << flops
        << ",\"bytes\":" << bytes << ",\"kernel\":\"" << kern_name(st) << "\",\"variant\":\""
        << kern_variant(st) << "\",\"config\":\"" << cand_label(st) << "\",\"ws_elems\":" << st.ws_elems;
+    mfma_json(os, st);
     if (with_slots) {   // arena values read (views resolved), and the small-step level
       auto root_name = [&](int n) {
         while (prog.nodes[n].op == qx::Op::View || prog.nodes[n].op == qx::Op::Save) n = prog.nodes[n].ia;
@@ -1839,6 +1848,7 @@ std::string stats_json(const qx_plan *P) {
          << ",\"flops\":" << flops << ",\"bytes\":" << bytes << ",\"kernel\":\""
          << kern_name(st) << "\",\"variant\":\"" << variant << "\",\"config\":\"" << cand_label(st)
          << "\"";
+      mfma_json(os, st);
       if (P->opt_profile && &L == P->last_lowered && s < P->step_ms.size())
         os << ",\"ms\":" << P->step_ms[s] << ",\"calls\":" << P->step_calls[s];
       if (s < L.tune_log.size() && !L.tune_log[s].empty()) os << ",\"tuning_ms\":{" << L.tune_log[s] << "}";

@@ -413,6 +413,7 @@ void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void 
   const long double ry = (sum_n(g.yw, g.nyb) + sum_n(g.sy, g.nsb) + sum_n(g.uy, g.nub) + 1) * es;
   const void *X = g.swap ? B : A, *Y = g.swap ? A : B;
   if (cu > (long double)g.c_elems * g.ksplit) violation("matrix-core GEMM results outside C");
+  if (g.nub - mfma_trip_bits(g) > kMfmaGridBits) violation("matrix-core GEMM grid of 2^32 lanes or more");
   launch(stream, [=]() {
     need(X, rx, "matrix-core GEMM X");
     need(Y, ry, "matrix-core GEMM Y");
