@@ -62,6 +62,8 @@ typedef struct qx_plan qx_plan; /* lowered, device-resident plan */
 /* Create a context on HIP device `device`.  No reference counterpart: the
  * reference selects the GPU inside QXContexts (bin/qxrun.jl:47-49, --gpu). */
 qx_status qx_ctx_create(int device, qx_ctx **out);
+/* Gives the handle back.  Plans may outlive it: the stream and the context's memory go
+ * with the last plan, and calls on those plans stay valid until then. */
 void qx_ctx_destroy(qx_ctx *ctx);
 
 /* Measured matrix-core rate of the context's device in TFLOP/s: a register-only loop

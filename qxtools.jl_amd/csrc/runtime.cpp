@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cmath>
 #include <cstring>
 #include <memory>
@@ -32,6 +33,7 @@ struct qx_ctx {
   // pinned host blocks of plans that are gone, at most kPinKept, for the next ones
   std::mutex pin_mutex;
   std::vector<void *> pins;
+  std::atomic<int> users{1};       // its handle and its live plans; freed by the last of them
 };
 
 namespace {
@@ -93,6 +95,16 @@ void pin_release(qx_ctx *c, void *p) {
     }
   }
   (void)hipHostFree(p);
+}
+
+void ctx_release(qx_ctx *c) {
+  if (!c || c->users.fetch_sub(1) != 1) return;
+  (void)hipSetDevice(c->device);
+  if (c->blas) (void)rocblas_destroy_handle(c->blas);
+  if (c->blas_ws) (void)hipFree(c->blas_ws);
+  if (c->stream) (void)hipStreamDestroy(c->stream);
+  for (void *p : c->pins) (void)hipHostFree(p);
+  delete c;
 }
 
 struct DevBuf {
@@ -213,6 +225,8 @@ struct qx_plan {
     return pin;
   }
 
+  qx_plan() = default;
+  qx_plan(const qx_plan &) = delete;
   ~qx_plan() {
     if (pin) (void)hipStreamSynchronize(ctx->stream);   // (a call that failed may have left work that uses it)
     pin_release(ctx, pin);
@@ -235,6 +249,7 @@ struct qx_plan {
     for (auto e : events) (void)hipEventDestroy(e);
     for (auto e : tune_events) (void)hipEventDestroy(e);
     drop_graphs();
+    ctx_release(ctx);
   }
 };
 
@@ -1924,15 +1939,7 @@ qx_status qx_measure_mfma(qx_ctx *ctx, int precision, double *tflops) {
   });
 }
 
-void qx_ctx_destroy(qx_ctx *ctx) {
-  if (!ctx) return;
-  (void)hipSetDevice(ctx->device);
-  if (ctx->blas) (void)rocblas_destroy_handle(ctx->blas);
-  if (ctx->blas_ws) (void)hipFree(ctx->blas_ws);
-  if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
-  for (void *p : ctx->pins) (void)hipHostFree(p);
-  delete ctx;
-}
+void qx_ctx_destroy(qx_ctx *ctx) { ctx_release(ctx); }
 
 qx_status qx_plan_from_dsl(qx_ctx *ctx, const char *dsl, size_t len, int precision, qx_plan **out) {
   return guard([&] {
@@ -1940,6 +1947,7 @@ qx_status qx_plan_from_dsl(qx_ctx *ctx, const char *dsl, size_t len, int precisi
     *out = nullptr;
     if (precision < QX_C128 || precision > QX_C64_BF16X3) throw qx::Error(QX_ERR_ARGUMENT, "unknown precision");
     auto P = std::make_unique<qx_plan>();
+    ++ctx->users;
     P->ctx = ctx;
     P->prec = precision;
     P->prog = qx::parse_program(dsl, len);

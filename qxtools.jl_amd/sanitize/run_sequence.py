@@ -63,6 +63,7 @@ def main() -> int:
     ap.add_argument("--precision", default=None)
     ap.add_argument("--vjp", action="store_true")
     ap.add_argument("--noalloc", action="store_true")
+    ap.add_argument("--close-context-first", action="store_true", help="destroy the context before the last calls")
     ap.add_argument("--kernel", type=int, default=None, help="force a kernel choice (plan option)")
     a = ap.parse_args()
     if a.workload.startswith("plain:"):   # plain:nh,nm,nn,nk,layout
@@ -90,6 +91,9 @@ def main() -> int:
         print(f"call {i + 1}: {len(bits)} bitstrings in {time.time() - t0:.1f} s, "
               f"{lib.qx_sim_launches()} launches checked, last call {ex.stats()['last_call_launches']} launches",
               flush=True)
+    if a.close_context_first:
+        ex.plan.ctx.close()
+        ex.amplitudes(bits)
     if a.vjp:
         import numpy as np
 
