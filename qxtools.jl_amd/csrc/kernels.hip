@@ -1329,7 +1329,7 @@ void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void 
   increments(b.sx, b.nsb), increments(b.sy, b.nsb);
   for (int64_t *w : {b.ux, b.uy, b.uc}) increments(w + b.trip_at, q);
   if (prec == QX_C128) mfma_launch<double, false>(X, Y, dst, b, g, s);
-  else if (prec == QX_C64_3M) mfma_launch<float, true>(X, Y, dst, b, g, s);
+  else if (a.gauss) mfma_launch<float, true>(X, Y, dst, b, g, s);
   else mfma_launch<float, false>(X, Y, dst, b, g, s);
   check_launch("contract_gemm_mfma");
   if (a.ksplit > 1) {

@@ -329,6 +329,10 @@ bool mfma_args(const StepBits &sb, int precision, bool other, int64_t c_elems, M
   else if (nm <= 4 && nm <= nn) g.cfg = 3;
   else if (nn <= 4) g.cfg = 4;
   else g.cfg = nm <= nn ? 1 : 2;
+  // QX_C64_3M: three products where the FP32 products bind, both sides >= 64 and K >= 32 (below,
+  // 64 K / 8 flops per byte of C are under the 30 at which products and memory balance).
+  // Their error is about 1.5 times that of four, which every other step keeps
+  g.gauss = precision == QX_C64_3M && nm >= 6 && nn >= 6 && nk >= 5;
   int cap[3] = {ilog2(kMfmaTiles[g.cfg][0]), ilog2(kMfmaTiles[g.cfg][1]), kMfmaStageBits};
   int used[3] = {0, 0, 0};
   auto slot = [](char cls) { return cls == 'M' ? 0 : cls == 'N' ? 1 : cls == 'K' ? 2 : -1; };

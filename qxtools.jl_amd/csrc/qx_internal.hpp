@@ -257,6 +257,7 @@ constexpr int mfma_pitch(int width, int elem_bytes) {
 struct MfmaArgs {
   int cfg = 0, swap = 0, other = 0;   // other: result lanes not along C's fastest leg
   int partial = 0;                      // the tile has fewer rows, columns or k values
+  int gauss = 0;                        // three real products per complex product (QX_C64_3M)
   int conj_x = 0, conj_y = 0;
   int nxb = 0, nyb = 0, kk = 0;         // tile bits of X and Y; k values of a stage
   int nsb = 0, nub = 0, ksplit = 1;     // stage bits, unit bits (K splits the highest)

@@ -1410,11 +1410,13 @@ std::string kern_variant(const qx::Step &st) {
   }
 }
 
-// The matrix-core GEMM's tile (rows, columns, k values of a stage), workgroups and units of each.
+// The matrix-core GEMM's tile (rows, columns, k values of a stage), real products per complex
+// product, workgroups and units of each.
 void mfma_json(std::ostringstream &os, const qx::Step &st) {
   if (st.kern != qx::Kern::Gemm || st.gemm.tile != 3) return;
   const int q = qx::mfma_trip_bits(*st.mfma), *t = qx::kMfmaTiles[st.mfma->cfg];
-  os << ",\"tile\":[" << t[0] << "," << t[1] << "," << st.mfma->kk << "],\"workgroups\":"
+  os << ",\"tile\":[" << t[0] << "," << t[1] << "," << st.mfma->kk << "],\"products\":"
+     << (st.mfma->gauss ? 3 : 4) << ",\"workgroups\":"
      << (int64_t(1) << (st.mfma->nub - q)) << ",\"units_per_workgroup\":" << (int64_t(1) << q);
 }
 
