@@ -941,6 +941,40 @@ static void fused_shapes(const Program &p, uint64_t fused, std::vector<std::vect
   }
 }
 
+uint64_t inline_vars(const Program &p) {
+  uint64_t mask = 0;
+  auto in = [](const std::vector<int> &labels, int l) { return std::find(labels.begin(), labels.end(), l) != labels.end(); };
+  for (size_t j = 0; j < p.vars.size() && j < 63; ++j) {
+    std::vector<int> leg(p.nodes.size(), -1);   // each node's leg of this variable
+    int sums = 0;
+    bool ok = true;
+    for (size_t i = 0; i < p.nodes.size() && ok; ++i) {
+      const Node &n = p.nodes[i];
+      if (n.op == Op::View) {
+        leg[i] = leg[n.ia];
+        if (n.var_id == (int)j) {
+          ok = leg[i] < 0;
+          leg[i] = n.pos;
+        } else {
+          ok = leg[i] != n.pos;
+        }
+      } else if (n.op == Op::Ncon) {
+        const int a = leg[n.ia] < 0 ? -1 : n.alab[leg[n.ia]], b = leg[n.ib] < 0 ? -1 : n.blab[leg[n.ib]];
+        if (leg[n.ia] < 0 && leg[n.ib] < 0) continue;
+        if (leg[n.ia] >= 0 && leg[n.ib] >= 0) ok = a == b;
+        else ok = leg[n.ia] >= 0 ? !in(n.blab, a) : !in(n.alab, b);
+        const int l = leg[n.ia] >= 0 ? a : b;
+        if (in(n.clab, l)) leg[i] = (int)(std::find(n.clab.begin(), n.clab.end(), l) - n.clab.begin());
+        else ++sums;
+      } else if (n.op == Op::Save) {
+        ok = leg[n.ia] < 0;
+      }
+    }
+    if (ok && sums == 1) mask |= uint64_t(1) << j;
+  }
+  return mask;
+}
+
 namespace {
 
 // One step seen as X' = S . X with X the large operand: its legs by X stride.

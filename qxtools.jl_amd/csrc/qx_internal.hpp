@@ -62,6 +62,11 @@ struct Program {
 
 Program parse_program(const char *text, size_t len);
 
+// Slice variables (bit j = variable j) whose sum over values is a contraction of the
+// program with their legs whole: all their views meet as one label, which one ncon sums.
+// Others are looped: a variable that cuts two bonds, or a leg of the saved tensor.
+uint64_t inline_vars(const Program &p);
+
 // ----------------------------------------------------------------------------
 // Lowered form for one batch size.
 enum class Buf : int8_t { None, Data, Arena, Cot, Temp, Grad };

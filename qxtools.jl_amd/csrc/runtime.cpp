@@ -171,6 +171,7 @@ struct qx_plan {
   std::map<std::pair<int64_t, uint64_t>, qx::VjpLowered> vjp_lowered;
   std::map<std::pair<int64_t, int>, uint64_t> fuse_choice;          // (batch, vjp) -> fused vars
   int64_t opt_fuse = 1;
+  uint64_t inline_ok = 0;                   // slice variables that may be contracted inline
   const qx::Lowered *last_lowered = nullptr;   // lowering used by the last qx_amplitudes
   DevBuf varena, cot, temp, grad, ampcot, ws;
   DevBuf arena, out_off, out_q, bits, acc, outbuf, relem_off;
@@ -883,7 +884,8 @@ void collect_profile(qx_plan *P, const qx::Lowered &L) {
 // for the largest j whose lowered program (arena + workspace, or for the vjp the
 // kept forward values + cotangents) fits half the memory cap.  Slicing bounds
 // memory; when memory does not bind, fewer and larger launches are faster and the
-// sum over the fused variables happens inside the contractions (by linearity).
+// sum over the fused variables happens inside the contractions (by linearity, where
+// inline_vars says that this is the same sum).
 uint64_t choose_fused(qx_plan *P, int64_t batch, bool for_vjp) {
   const int nv = (int)P->prog.vars.size();
   if (!P->opt_fuse || nv == 0) return 0;
@@ -895,6 +897,7 @@ uint64_t choose_fused(qx_plan *P, int64_t batch, bool for_vjp) {
   uint64_t pick = 0;
   for (int j = std::min(nv, 63); j > 0; --j) {
     uint64_t mask = (uint64_t(1) << j) - 1;
+    if (mask & ~P->inline_ok) continue;
     try {
       int64_t need;
       if (for_vjp) {
@@ -931,7 +934,7 @@ uint64_t choose_fused_range(qx_plan *P, int64_t batch, int64_t s0, int64_t s1, i
   int64_t block = 1;
   for (size_t j = 0; j < P->prog.var_dims.size() && j < 63; ++j) {
     block *= P->prog.var_dims[j];
-    if (s0 % block || s1 % block) break;
+    if (s0 % block || s1 % block || !((P->inline_ok >> j) & 1)) break;
     mask |= uint64_t(1) << j;
   }
   if (!mask) return 0;
@@ -1953,6 +1956,7 @@ qx_status qx_plan_from_dsl(qx_ctx *ctx, const char *dsl, size_t len, int precisi
     P->ctx = ctx;
     P->prec = precision;
     P->prog = qx::parse_program(dsl, len);
+    P->inline_ok = qx::inline_vars(P->prog);
     *out = P.release();
   });
 }
@@ -2200,6 +2204,7 @@ qx_status qx_dsl_inspect_ex(const char *dsl, size_t len, int precision, int64_t 
     os.precision(17);
     lowered_json(os, prog, L, precision, true);
     std::string s = os.str();
+    s.insert(s.size() - 1, ",\"inline_vars\":" + std::to_string(qx::inline_vars(prog)));
     // reverse-mode lowering (its own host-side bounds proof runs here too)
     std::string v;
     try {
