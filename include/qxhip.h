@@ -237,8 +237,9 @@ qx_status qx_dsl_inspect(const char *dsl, size_t len, int precision, int64_t bat
                          char *json, size_t cap);
 
 /* qx_dsl_inspect with lowering flags: bit 0 = the "batch_last" plan option (batched
- * bitstring leg slowest in bitstring-dependent intermediates).  No reference
- * counterpart. */
+ * bitstring leg slowest in bitstring-dependent intermediates), bit 1 = the slices of the
+ * variables in `fused` stay apart, side by side in the saved tensor, instead of being
+ * summed (as qx_amplitudes contracts a part of the slices).  No reference counterpart. */
 qx_status qx_dsl_inspect_ex(const char *dsl, size_t len, int precision, int64_t batch, uint64_t fused,
                             int64_t flags, char *json, size_t cap);
 

@@ -934,20 +934,23 @@ __device__ __forceinline__ void neumaier(double &s, double &c, double x) {
 
 template <typename T>
 __global__ void k_accumulate(const typename Vec<T>::type *__restrict__ root, int64_t root_bstride, int64_t batch,
-                             int64_t nvalid, int64_t relems, const int64_t *__restrict__ relem_off,
+                             int64_t nvalid, int64_t relems, int64_t slices, const int64_t *__restrict__ relem_off,
                              double *__restrict__ acc, double2 *__restrict__ out, int64_t row0, int first, int last) {
   int64_t total = nvalid * relems;
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < total;
        t += (int64_t)gridDim.x * blockDim.x) {
     int64_t beta = t % nvalid;
     int64_t e = t / nvalid;
-    auto v = root[relem_off[e] + beta * root_bstride];
     const int64_t i = (row0 + beta) * relems + e;
     double *a = acc + i * 4;
     double s0 = 0, s1 = 0, c0 = 0, c1 = 0;
     if (!first) s0 = a[0], s1 = a[1], c0 = a[2], c1 = a[3];
-    neumaier(s0, c0, (double)v.x);
-    neumaier(s1, c1, (double)v.y);
+#pragma unroll 4
+    for (int64_t sl = 0; sl < slices; ++sl) {
+      const auto v = root[relem_off[sl * relems + e] + beta * root_bstride];
+      neumaier(s0, c0, (double)v.x);
+      neumaier(s1, c1, (double)v.y);
+    }
     if (last) {
       out[i] = double2{s0 + c0, s1 + c1};
     } else {
@@ -2903,16 +2906,16 @@ void launch_fill_outputs(int prec, void *arena, const int64_t *d_out_off, int n_
 }
 
 void launch_accumulate(int prec, const void *root, int64_t root_bstride, int64_t batch, int64_t nvalid, int64_t relems,
-                       const int64_t *d_relem_off, double *acc, double *out, int64_t row0, bool first, bool last,
-                       void *stream) {
+                       int64_t slices, const int64_t *d_relem_off, double *acc, double *out, int64_t row0, bool first,
+                       bool last, void *stream) {
   int g = grid_for(nvalid * relems, 256);
   hipStream_t s = (hipStream_t)stream;
   if (prec == QX_C128)
     hipLaunchKernelGGL(k_accumulate<double>, dim3(g), dim3(256), 0, s, (const double2 *)root, root_bstride, batch,
-                       nvalid, relems, d_relem_off, acc, (double2 *)out, row0, (int)first, (int)last);
+                       nvalid, relems, slices, d_relem_off, acc, (double2 *)out, row0, (int)first, (int)last);
   else
     hipLaunchKernelGGL(k_accumulate<float>, dim3(g), dim3(256), 0, s, (const float2 *)root, root_bstride, batch,
-                       nvalid, relems, d_relem_off, acc, (double2 *)out, row0, (int)first, (int)last);
+                       nvalid, relems, slices, d_relem_off, acc, (double2 *)out, row0, (int)first, (int)last);
   check_launch("accumulate");
 }
 

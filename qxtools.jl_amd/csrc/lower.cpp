@@ -975,6 +975,51 @@ uint64_t inline_vars(const Program &p) {
   return mask;
 }
 
+bool keep_slices(Program &p, uint64_t vars) {
+  p.kept.clear();
+  for (size_t j = 0; j < p.vars.size() && j < 63; ++j) {
+    if (!((vars >> j) & 1)) continue;
+    std::vector<int> leg(p.nodes.size(), -1);   // each node's leg of this variable
+    for (size_t i = 0; i < p.nodes.size(); ++i) {
+      Node &n = p.nodes[i];
+      if (n.op == Op::View) {
+        leg[i] = leg[n.ia];
+        if (n.var_id == (int)j) {
+          if (leg[i] >= 0) return false;
+          leg[i] = n.pos;
+        } else if (leg[i] == n.pos) {
+          return false;
+        }
+      } else if (n.op == Op::Ncon) {
+        const int a = leg[n.ia], b = leg[n.ib];
+        if (a < 0 && b < 0) continue;
+        int fresh = 0;   // a leg that an operand keeps beyond the program's own takes a new label
+        for (const std::vector<int> *v : {&n.alab, &n.blab})
+          for (int l : *v) fresh = std::max(fresh, l + 1);
+        if (a == (int)n.alab.size()) n.alab.push_back(fresh);
+        if (b == (int)n.blab.size()) n.blab.push_back(fresh);
+        auto count = [](const std::vector<int> &v, int l) { return (int)std::count(v.begin(), v.end(), l); };
+        int l = a >= 0 ? n.alab[a] : n.blab[b];
+        if (a >= 0 && b >= 0 && n.blab[b] != l) {   // both hold it: one label
+          const int lb = n.blab[b];
+          if (count(n.blab, l) || count(n.alab, lb) || (count(n.clab, l) && count(n.clab, lb))) return false;
+          n.blab[b] = l;
+          std::replace(n.clab.begin(), n.clab.end(), lb, l);
+        } else if ((a < 0 && count(n.alab, l)) || (b < 0 && count(n.blab, l))) {
+          return false;
+        }
+        leg[i] = (int)(std::find(n.clab.begin(), n.clab.end(), l) - n.clab.begin());
+        if (leg[i] == (int)n.clab.size()) n.clab.push_back(l);
+      } else if (n.op == Op::Save) {
+        leg[i] = leg[n.ia];
+      }
+    }
+    if (leg[p.save] < 0) return false;
+    p.kept.push_back(leg[p.save]);
+  }
+  return true;
+}
+
 namespace {
 
 // One step seen as X' = S . X with X the large operand: its legs by X stride.
@@ -2036,7 +2081,9 @@ Lowered lower(const Program &p, int64_t batch, bool keep_all, int precision, uin
 
   // result elements per bitstring
   L.result_elems = 1;
-  for (int64_t d : shape[p.save]) L.result_elems *= d;
+  L.kept = p.kept;
+  for (size_t j = 0; j < shape[p.save].size(); ++j)
+    (std::count(p.kept.begin(), p.kept.end(), (int)j) ? L.kept_values : L.result_elems) *= shape[p.save][j];
 
   // liveness: schedule positions = sections 0, 1, then output fill, then section 2
   std::vector<int> order;

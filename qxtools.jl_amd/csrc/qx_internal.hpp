@@ -58,6 +58,7 @@ struct Program {
   std::map<std::string, int64_t> key_elems;
   int num_chars = 0;                      // largest output qubit
   std::vector<int> outputs;               // output node indices
+  std::vector<int> kept;                  // keep_slices: leg of the saved tensor of each kept variable
 };
 
 Program parse_program(const char *text, size_t len);
@@ -66,6 +67,13 @@ Program parse_program(const char *text, size_t len);
 // program with their legs whole: all their views meet as one label, which one ncon sums.
 // Others are looped: a variable that cuts two bonds, or a leg of the saved tensor.
 uint64_t inline_vars(const Program &p);
+
+// Rewrite a program so that the legs of the variables in `vars`, left whole (lower's
+// `fused`), are summed nowhere and end as legs of the saved tensor, one per variable: the
+// results of their slices side by side.  A contraction that summed such a leg, or that
+// combines two tensors of one variable, carries it as a leg of both operands and the
+// result.  False (p unusable) where a tensor would hold two legs of one variable.
+bool keep_slices(Program &p, uint64_t vars);
 
 // ----------------------------------------------------------------------------
 // Lowered form for one batch size.
@@ -390,6 +398,8 @@ struct Lowered {
   int64_t ws_elems = 0;             // largest K-split workspace of any step
   int64_t out_elems = 0;            // elements of one output tensor incl. batch
   int64_t result_elems = 1;         // complex values per bitstring
+  std::vector<int> kept;            // legs of the saved tensor that number slices (keep_slices)
+  int64_t kept_values = 1;          // slices side by side in it
   // per section: launches of a pass were every slice-dependent or lone step a launch of
   // its own (the size a call is held to for graph capture); -1: one per step
   int64_t est_launches[3] = {-1, -1, -1};
@@ -480,9 +490,10 @@ void launch_contract_radix(int prec, const void *A, const void *B, void *C, int6
 void launch_fill_outputs(int prec, void *arena, const int64_t *d_out_off, int n_out,
                          const int *d_out_q, const char *d_bits, int64_t nvalid, int64_t batch,
                          int64_t num_chars, void *stream);
+// (`slices` of them side by side in the root: d_relem_off holds relems offsets of each in turn)
 void launch_accumulate(int prec, const void *root, int64_t root_bstride, int64_t batch, int64_t nvalid,
-                       int64_t relems, const int64_t *d_relem_off, double *acc, double *out, int64_t row0,
-                       bool first, bool last, void *stream);
+                       int64_t relems, int64_t slices, const int64_t *d_relem_off, double *acc, double *out,
+                       int64_t row0, bool first, bool last, void *stream);
 // dst[map(e)] += src[e] for src dense over dims (first fastest), map = sum digit*stride
 void launch_add_mapped(int prec, int dst_double, void *dst, const void *src, int64_t n,
                        const std::vector<int64_t> &dims, const std::vector<int64_t> &strides,

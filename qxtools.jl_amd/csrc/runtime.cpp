@@ -279,11 +279,14 @@ void force_chain_variant(qx::Step &st, int64_t v) {
   if (v & 8) st.chain.wave_local = 0;
 }
 
-const qx::Lowered &ensure_lowered(qx_plan *P, int64_t batch, uint64_t fused = 0) {
-  auto key = std::make_pair(batch, fused);
+constexpr uint64_t kKept = uint64_t(1) << 63;   // in the key of a lowering of keep_slices
+
+// `kept`: a program of keep_slices over the variables in `fused`, in place of the plan's.
+const qx::Lowered &ensure_lowered(qx_plan *P, int64_t batch, uint64_t fused = 0, const qx::Program *kept = nullptr) {
+  auto key = std::make_pair(batch, kept ? fused | kKept : fused);
   auto it = P->lowered.find(key);
   if (it != P->lowered.end()) return it->second;
-  qx::Lowered L = qx::lower(P->prog, batch, false, P->prec, fused, P->opt_chains != 0, P->opt_batch_last != 0);
+  qx::Lowered L = qx::lower(kept ? *kept : P->prog, batch, false, P->prec, fused, P->opt_chains != 0, P->opt_batch_last != 0);
   if (P->opt_kernel >= 0)
     for (auto &st : L.steps) {
       if (st.lone) st.level = -1;   // a forced kernel runs every step of its own
@@ -919,22 +922,20 @@ uint64_t choose_fused(qx_plan *P, int64_t batch, bool for_vjp) {
   return pick;
 }
 
-// Slice variables a call over slices [s0, s1) contracts inline.  All slices: the choice
-// above.  A part of them (a worker's share of a sharded run): the first f variables, for
-// the largest f such that the range consists of whole blocks of their values -- the first
-// variable runs fastest, so both ends are multiples of the product of their dims -- and
-// the program fits as above; by linearity a block's sum is one slice of that program.
-// complex128 only: the looped sum of slices is held in FP64, which a complex64
-// contraction over the same values would not be.  8 slices of the 6x6 plan, 37 strings:
-// 3.99 ms looped, 0.97 inline (looped launches of 10 us leave most of the chip idle).
-uint64_t choose_fused_range(qx_plan *P, int64_t batch, int64_t s0, int64_t s1, int64_t nslices) {
-  if (s0 == 0 && s1 == nslices) return choose_fused(P, batch, false);
+// Slice variables whose slices a call over a part [s0, s1) of them (a worker's share of a
+// sharded run) contracts side by side: the first f, for the largest f such that the range
+// consists of whole blocks of their values -- the first variable runs fastest, so both ends
+// are multiples of the product of their dims -- and the program fits as above.  Each slice's
+// result stays apart and enters the compensated sum like a looped one (complex64 parts loop).
+// 8 slices of the 6x6 plan, 37 strings: looped 3.99 ms (launches of 10 us that leave most of
+// the chip idle), side by side 0.95; 256 strings: 7.0, 2.7.
+uint64_t choose_kept(qx_plan *P, int64_t batch, int64_t s0, int64_t s1) {
   if (!P->opt_fuse || P->prec != QX_C128) return 0;
   uint64_t mask = 0;
   int64_t block = 1;
-  for (size_t j = 0; j < P->prog.var_dims.size() && j < 63; ++j) {
+  for (size_t j = 0; j < P->prog.var_dims.size() && j < 62; ++j) {
     block *= P->prog.var_dims[j];
-    if (s0 % block || s1 % block || !((P->inline_ok >> j) & 1)) break;
+    if (s0 % block || s1 % block) break;
     mask |= uint64_t(1) << j;
   }
   if (!mask) return 0;
@@ -943,11 +944,13 @@ uint64_t choose_fused_range(qx_plan *P, int64_t batch, int64_t s0, int64_t s1, i
   if (it != P->fuse_choice.end()) return it->second;
   const int64_t budget = P->arena_cap_bytes / 2, es = (int64_t)P->esize();
   for (; mask; mask >>= 1) {
-    const bool known = P->lowered.count({batch, mask}) > 0;
+    const bool known = P->lowered.count({batch, mask | kKept}) > 0;
+    qx::Program kept = P->prog;
+    if (!known && !qx::keep_slices(kept, mask)) continue;
     try {
-      const qx::Lowered &L = ensure_lowered(P, batch, mask);
+      const qx::Lowered &L = ensure_lowered(P, batch, mask, &kept);
       if ((L.arena_elems + L.ws_elems) * es <= budget) break;
-      if (!known) P->lowered.erase({batch, mask});
+      if (!known) P->lowered.erase({batch, mask | kKept});
     } catch (const qx::Error &e) {
       if (e.code != QX_ERR_UNSUPPORTED && e.code != QX_ERR_MEMORY) throw;
     }
@@ -1013,6 +1016,32 @@ struct CallBufs {
   void *bits = nullptr;       // nb * num_chars bitstring characters
 };
 
+// Offsets in the saved tensor of a bitstring's results, in logical column-major order; where
+// slices lie side by side in it, those of each slice in turn (first variable fastest).
+std::vector<int64_t> result_offsets(const qx::Lowered &L, const qx::Value &rv) {
+  const int64_t R = L.result_elems;
+  std::vector<int64_t> roff(R * L.kept_values);
+  auto kept = [&](size_t j) { return std::count(L.kept.begin(), L.kept.end(), (int)j) > 0; };
+  for (int64_t e = 0; e < R; ++e) {
+    int64_t r = e, o = 0;
+    for (size_t j = 0; j < rv.dims.size(); ++j) {
+      if (kept(j)) continue;
+      o += r % rv.dims[j] * rv.strides[j];
+      r /= rv.dims[j];
+    }
+    roff[e] = o;
+  }
+  for (int64_t v = 1; v < L.kept_values; ++v) {
+    int64_t r = v, o = 0;
+    for (int j : L.kept) {
+      o += r % rv.dims[j] * rv.strides[j];
+      r /= rv.dims[j];
+    }
+    for (int64_t e = 0; e < R; ++e) roff[v * R + e] = roff[e] + o;
+  }
+  return roff;
+}
+
 // The device work of one amplitudes call, from the first step to the final sum: steps of
 // section 0 once, per looped slice those of section 1, per batch of
 // bitstrings the output fill, section 2 and the accumulation into FP64 pairs.
@@ -1057,8 +1086,8 @@ void enqueue_amplitudes(qx_plan *P, const qx::Lowered &L, uint64_t fused, int64_
                               (const char *)cb.bits + row0 * nch, nvalid, batch, nch, stream);
       run_section(2);
       qx::launch_accumulate(P->prec, value_ptr(P, rv, varval), rv.dep ? rv.beta_stride : 0, batch, nvalid, R,
-                            (const int64_t *)cb.relem_off, (double *)cb.acc, (double *)cb.outbuf, row0, sl == s0,
-                            sl + 1 == s1, stream);
+                            L.kept_values, (const int64_t *)cb.relem_off, (double *)cb.acc, (double *)cb.outbuf, row0,
+                            sl == s0, sl + 1 == s1, stream);
     }
   }
 }
@@ -1080,10 +1109,11 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   int64_t batch = 1;
   while (batch < nb && batch < P->opt_batch) batch <<= 1;
   const bool part = s0 != 0 || s1 != nslices;
-  const uint64_t fused = choose_fused_range(P, batch, s0, s1, nslices);
+  const uint64_t fused = part ? choose_kept(P, batch, s0, s1) : choose_fused(P, batch, false);
+  const bool kept = part && fused;
   const int64_t per = nslices / looped_slices(P, fused);   // slices of one pass
   s0 /= per, s1 /= per;
-  qx::Lowered &L = const_cast<qx::Lowered &>(ensure_lowered(P, batch, fused));
+  qx::Lowered &L = kept ? P->lowered.at({batch, fused | kKept}) : const_cast<qx::Lowered &>(ensure_lowered(P, batch, fused));
   if (P->last_lowered != &L) {
     P->step_ms.clear();
     P->step_calls.clear();
@@ -1102,10 +1132,9 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
     }
     tuner->seen.assign(L.steps.size(), 0);
   }
-  // a part of the slices contracted inline: the looped program stays ready as well, at the
-  // batch size of qx_amplitudes_noalloc, for parts that are not whole blocks
-  const qx::Lowered *plain = nullptr;
-  if (part && fused && batch == P->opt_batch) plain = &ensure_lowered(P, batch);
+  // the looped program stays ready as well, at the batch size of qx_amplitudes_noalloc, whose
+  // parts loop
+  const qx::Lowered *plain = kept && batch == P->opt_batch ? &ensure_lowered(P, batch) : nullptr;
   bool moved = P->arena.reserve(
       std::max<size_t>((size_t)std::max(L.arena_elems, plain ? plain->arena_elems : 0) * es, 256));
   moved |= P->ws.reserve(std::max<size_t>((size_t)std::max(ws_elems, plain ? plain->ws_elems : 0) * es, 256));
@@ -1124,21 +1153,11 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
     P->out_off.upload(ooff.data(), ooff.size() * 8, stream);
     P->out_q.upload(oq.data(), oq.size() * 4, stream);
   }
-  // root element offsets (logical column-major order of the saved tensor)
   const qx::Value &rv = L.values[P->prog.save];
   const int64_t R = L.result_elems;
-  std::vector<int64_t> roff(R);
-  for (int64_t e = 0; e < R; ++e) {
-    int64_t r = e, o = 0;
-    for (size_t j = 0; j < rv.dims.size(); ++j) {
-      int64_t d = r % rv.dims[j];
-      r /= rv.dims[j];
-      o += d * rv.strides[j];
-    }
-    roff[e] = o;
-  }
-  moved |= P->relem_off.reserve(std::max<size_t>(R * 8, 16));
-  P->relem_off.upload(roff.data(), R * 8, stream);
+  const std::vector<int64_t> roff = result_offsets(L, rv);
+  moved |= P->relem_off.reserve(std::max<size_t>(roff.size() * 8, 16));
+  P->relem_off.upload(roff.data(), roff.size() * 8, stream);
   const size_t nbits = (size_t)nb * nch, nout_bytes = (size_t)nb * R * 16;
   const bool pin_bits = bits && nbits <= kPinBits, pin_out = out && nout_bytes <= kPinOut;
   if (pin_bits) {
@@ -1156,7 +1175,10 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
     Bases bs;
     bs.arena = (char *)P->arena.p;
     prepare_small(P, L, bs);
-    if (plain) prepare_small(P, *plain, bs);
+    if (plain) {
+      prepare_small(P, *plain, bs);
+      blas_before_capture(P->ctx, plain->steps);
+    }
   }
 
   P->event_step.clear();
@@ -1173,8 +1195,8 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   P->last_launches = launches;
   if (P->opt_graph && !P->opt_profile && !tuner && launches <= kMaxGraphLaunches) {
     auto key = std::make_tuple(batch, nb, s0,
-                               s1 + (int64_t)__builtin_popcountll(fused) * (int64_t(1) << 43) + (out ? int64_t(1) << 41 : 0) +
-                                   (bits ? int64_t(1) << 42 : 0));
+                               s1 + (int64_t)__builtin_popcountll(fused) * (int64_t(1) << 44) + (out ? int64_t(1) << 41 : 0) +
+                                   (bits ? int64_t(1) << 42 : 0) + (kept ? int64_t(1) << 43 : 0));
     auto it = P->graphs.find(key);
     if (it == P->graphs.end()) {
       hipGraph_t g = nullptr;
@@ -1220,20 +1242,18 @@ void amplitudes_noalloc(qx_plan *P, const char *bits, int64_t nb, int64_t s0, in
   check_bits(P, bits, nb);
   const int64_t batch = P->opt_batch;
   const bool part = s0 != 0 || s1 != nslices;
-  auto tables = [&](const qx::Lowered &L) {
-    auto sm = P->small.find(&L);
-    return sm != P->small.end() && sm->second.arena == P->arena.p && sm->second.index.size() == L.steps.size();
-  };
-  uint64_t fused = choose_fused_range(P, batch, s0, s1, nslices);
-  if (part && fused && !tables(ensure_lowered(P, batch, fused))) fused = 0;   // as an earlier call left them
-  const int64_t per = nslices / looped_slices(P, fused);   // slices of one pass
-  s0 /= per, s1 /= per;
+  const uint64_t fused = part ? 0 : choose_fused(P, batch, false);   // (parts loop: no table depends on their range)
+  if (fused) {
+    s0 = 0;
+    s1 = looped_slices(P, fused);
+  }
   const qx::Lowered &L = ensure_lowered(P, batch, fused);
   const size_t es = P->esize();
   const char *warm = ": run one qx_amplitudes call of at least the plan's batch option in bitstrings first";
   if ((size_t)L.arena_elems * es > P->arena.bytes || (size_t)L.ws_elems * es > P->ws.bytes || !P->arena.p)
     throw qx::Error(QX_ERR_STATE, std::string("plan memory not sized for this call") + warm);
-  if (!tables(L))
+  auto sm = P->small.find(&L);
+  if (sm == P->small.end() || sm->second.arena != P->arena.p || sm->second.index.size() != L.steps.size())
     throw qx::Error(QX_ERR_STATE, std::string("small-step tables not built for this call") + warm);
   for (auto &st : L.steps)
     if (st.kern == qx::Kern::Blas && !st.blas.own && !P->ctx->blas)
@@ -1248,16 +1268,7 @@ void amplitudes_noalloc(qx_plan *P, const char *bits, int64_t nb, int64_t s0, in
     ooff.push_back(L.values[o].slot);
     oq.push_back(P->prog.nodes[o].qubit);
   }
-  const qx::Value &rv = L.values[P->prog.save];
-  std::vector<int64_t> roff(R);
-  for (int64_t e = 0; e < R; ++e) {
-    int64_t r = e, o = 0;
-    for (size_t j = 0; j < rv.dims.size(); ++j) {
-      o += (r % rv.dims[j]) * rv.strides[j];
-      r /= rv.dims[j];
-    }
-    roff[e] = o;
-  }
+  const std::vector<int64_t> roff = result_offsets(L, L.values[P->prog.save]);
   auto up = [](size_t b) { return (b + 255) / 256 * 256; };
   const size_t b_acc = up((size_t)nb * R * 32), b_out = up((size_t)nb * R * 16), b_roff = up((size_t)R * 8),
                b_ooff = up(ooff.size() * 8), b_oq = up(oq.size() * 4), b_bits = up((size_t)nb * nch);
@@ -1599,18 +1610,7 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   if (norm && (looped_slices(P, fused) != 1 || !rc.dep || rc.beta_stride != rv.beta_stride))
     throw qx::Error(QX_ERR_UNSUPPORTED, "the norm pullback needs every slice variable contracted inline and a "
                                         "bitstring-dependent root");
-  std::vector<int64_t> roff(R);
-  {
-    for (int64_t e = 0; e < R; ++e) {
-      int64_t r = e, o = 0;
-      for (size_t j = 0; j < rv.dims.size(); ++j) {
-        int64_t d = r % rv.dims[j];
-        r /= rv.dims[j];
-        o += d * rv.strides[j];
-      }
-      roff[e] = o;
-    }
-  }
+  const std::vector<int64_t> roff = result_offsets(L, rv);
   moved |= P->relem_off.reserve(std::max<size_t>(R * 8, 16));
   P->relem_off.upload(roff.data(), R * 8, stream);
   if (moved) P->drop_graphs();
@@ -1847,7 +1847,7 @@ std::string stats_json(const qx_plan *P) {
     const qx::Lowered &L = kv.second;
     if (!first) os << ",";
     first = false;
-    os << "{\"batch\":" << L.batch << ",\"fused\":" << L.fused << ",\"active\":" << (&L == P->last_lowered)
+    os << "{\"batch\":" << L.batch << ",\"fused\":" << L.fused << ",\"kept_slices\":" << L.kept_values << ",\"active\":" << (&L == P->last_lowered)
        << ",\"tuned\":" << L.tuned
        << ",\"arena_bytes\":" << L.arena_elems * (int64_t)P->esize() << ",\"result_elems\":" << L.result_elems
        << ",\"steps\":[";
@@ -2194,17 +2194,20 @@ qx_status qx_dsl_inspect(const char *dsl, size_t len, int precision, int64_t bat
 qx_status qx_dsl_inspect_ex(const char *dsl, size_t len, int precision, int64_t batch, uint64_t fused,
                             int64_t flags, char *json, size_t cap) {
   return guard([&] {
-    if (flags & ~int64_t(1)) throw qx::Error(QX_ERR_ARGUMENT, "unknown inspect flags");
+    if (flags & ~int64_t(3)) throw qx::Error(QX_ERR_ARGUMENT, "unknown inspect flags");
     const bool batch_last = flags & 1;
     if (!json || cap == 0) throw qx::Error(QX_ERR_ARGUMENT, "null output buffer");
     if (precision < QX_C128 || precision > QX_C64_BF16X3) throw qx::Error(QX_ERR_ARGUMENT, "unknown precision");
     qx::Program prog = qx::parse_program(dsl, len);
+    const uint64_t inline_ok = qx::inline_vars(prog);
+    if ((flags & 2) && !qx::keep_slices(prog, fused))
+      throw qx::Error(QX_ERR_UNSUPPORTED, "a tensor would hold two legs of one slice variable");
     qx::Lowered L = qx::lower(prog, batch, false, precision, fused, true, batch_last);
     std::ostringstream os;
     os.precision(17);
     lowered_json(os, prog, L, precision, true);
     std::string s = os.str();
-    s.insert(s.size() - 1, ",\"inline_vars\":" + std::to_string(qx::inline_vars(prog)));
+    s.insert(s.size() - 1, ",\"inline_vars\":" + std::to_string(inline_ok) + ",\"kept_slices\":" + std::to_string(L.kept_values));
     // reverse-mode lowering (its own host-side bounds proof runs here too)
     std::string v;
     try {

@@ -87,15 +87,18 @@ def _dptr(a: np.ndarray):
     return a.ctypes.data_as(C.POINTER(C.c_double))
 
 
-def inspect(dsl: str, precision: str = "c128", batch: int = 1, fused: int = 0, batch_last: bool = False) -> dict:
+def inspect(dsl: str, precision: str = "c128", batch: int = 1, fused: int = 0, batch_last: bool = False,
+            kept: bool = False) -> dict:
     """Lower a program on the host (no device): steps, kernels, arena schedule.
-    `fused`: bit mask of slice variables contracted inline; `batch_last`: the plan
-    option of that name."""
+    `fused`: bit mask of slice variables contracted inline (`kept`: their
+    slices stay apart, as for a part of the slices); `batch_last`: the plan option of that
+    name."""
     b = dsl.encode()
     cap = 1 << 16
     while True:
         buf = C.create_string_buffer(cap)
-        st = lib().qx_dsl_inspect_ex(b, len(b), PRECISIONS[precision], batch, fused, int(bool(batch_last)), buf, cap)
+        st = lib().qx_dsl_inspect_ex(b, len(b), PRECISIONS[precision], batch, fused, int(bool(batch_last)) + 2 * int(bool(kept)), buf,
+                                     cap)
         if st == 0:
             return json.loads(buf.value.decode())
         if st != -1 or cap > (1 << 28):

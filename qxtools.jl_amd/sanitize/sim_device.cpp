@@ -490,12 +490,12 @@ long double root_reach(const int64_t *d_relem_off, int64_t relems, int64_t bstri
 }  // namespace
 
 void launch_accumulate(int prec, const void *root, int64_t root_bstride, int64_t batch, int64_t nvalid,
-                       int64_t relems, const int64_t *d_relem_off, double *acc, double *out, int64_t row0, bool first,
-                       bool last, void *stream) {
+                       int64_t relems, int64_t slices, const int64_t *d_relem_off, double *acc, double *out,
+                       int64_t row0, bool first, bool last, void *stream) {
   const size_t es = esize(prec);
   if (nvalid > batch) violation("accumulate: more valid rows than the batch");
   launch(stream, [=]() {
-    need(root, root_reach(d_relem_off, relems, root_bstride, nvalid) * es, "saved tensor");
+    need(root, root_reach(d_relem_off, relems * slices, root_bstride, nvalid) * es, "saved tensor");
     if (!first || !last) need(acc, (long double)(row0 + nvalid) * relems * 32, "accumulators");
     if (last) need(out, (long double)(row0 + nvalid) * relems * 16, "results");
   });
