@@ -1763,19 +1763,6 @@ void level_small_steps(const Program &p, Lowered &L) {
     }
     return level;
   };
-  {   // the launches of a pass were slice-dependent steps launched one by one
-    const std::vector<int> level = levels([&](size_t s) {
-      const Step &st = L.steps[s];
-      return small[s] && st.section != 1 && L.values[st.in_a].var_terms.empty() && L.values[st.in_b].var_terms.empty();
-    });
-    for (int sec = 0; sec < 3; ++sec) {
-      std::set<int> seen;
-      int64_t n = 0;
-      for (size_t s = 0; s < L.steps.size(); ++s)
-        if (L.steps[s].section == sec && (level[s] < 0 || seen.insert(level[s]).second)) ++n;
-      L.est_launches[sec] = n;
-    }
-  }
   const std::vector<int> level = levels([&](size_t s) { return small[s] != 0; });
   int key = 0;
   std::vector<Step> out;

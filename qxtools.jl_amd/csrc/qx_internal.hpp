@@ -400,9 +400,6 @@ struct Lowered {
   int64_t result_elems = 1;         // complex values per bitstring
   std::vector<int> kept;            // legs of the saved tensor that number slices (keep_slices)
   int64_t kept_values = 1;          // slices side by side in it
-  // per section: launches of a pass were every slice-dependent or lone step a launch of
-  // its own (the size a call is held to for graph capture); -1: one per step
-  int64_t est_launches[3] = {-1, -1, -1};
 };
 
 // batch_last: lay the batched bitstring leg out slowest in bitstring-dependent

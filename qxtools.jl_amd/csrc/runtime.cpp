@@ -151,7 +151,7 @@ struct qx_plan {
   int64_t opt_batch = 256;
   int64_t opt_arena_mb = -1;
   int64_t opt_graph = 0;
-  int64_t last_launches = 0;   // launches of the last amplitudes / vjp call (estimate)
+  int64_t last_launches = 0;   // kernel launches of the last amplitudes / vjp call
   int64_t opt_profile = 0;
   int64_t opt_autotune = 0;
   int64_t opt_kernel = -1;                  // >= 0: force that kernel wherever it can run
@@ -978,24 +978,42 @@ void slice_values(const qx_plan *P, uint64_t fused, int64_t sl, std::vector<int6
   }
 }
 
-// Launches of one section of a lowered program per pass, at most (Lowered::est_launches:
-// runs of levels and slice-dependent small steps take fewer).
-int64_t section_launches(const qx::Lowered &L, int sec) {
-  if (L.est_launches[sec] >= 0) return L.est_launches[sec];
-  int64_t n = 0;
-  std::set<int> levels;
-  for (auto &st : L.steps)
-    if (st.section == sec) {
-      if (st.level >= 0) levels.insert(st.level);
-      else ++n;
+// Kernels that launch_step launches for a step.
+int step_launches(const qx::Step &st) {
+  switch (st.kern) {
+    case qx::Kern::Blas: {
+      const qx::BlasArgs &b = st.blas;
+      return (b.ttgt ? 3 : 0) + (b.own ? 1 + (b.ksplit > 1) : b.split ? 15 : 1);
     }
-  return n + (int64_t)levels.size();
+    case qx::Kern::Chain: return 2 + !st.chain_merge.empty();
+    case qx::Kern::Gemm: return 1 + ((st.gemm.tile == 3 ? st.mfma->ksplit : st.gemm.ksplit) > 1);
+    case qx::Kern::Outer:
+    case qx::Kern::Radix:
+    case qx::Kern::Rows: return 1;
+    default: return 1 + (st.bits.ksplit > 1);
+  }
 }
 
-// A call of more launches than this runs without graph capture: capturing and
-// instantiating a graph of that many nodes costs host time and memory that its replay
-// cannot win back, since such a call runs for a long time anyway.
-constexpr int64_t kMaxGraphLaunches = int64_t(1) << 15;
+// Launches of one section of a lowered program per pass: its steps', one per level or run
+// of levels of small steps, or one for all of them (prepare_small has built the tables).
+int64_t section_launches(const qx_plan *P, const qx::Lowered &L, int sec) {
+  const qx_plan::SmallTable &T = P->small.at(&L);
+  const bool walk = walks(P, T, sec);
+  int64_t n = walk;
+  for (size_t s = 0; s < L.steps.size(); ++s) {
+    if (L.steps[s].section != sec) continue;
+    if (L.steps[s].level < 0) n += step_launches(L.steps[s]);
+    else n += !walk && T.count[s] > 0 && !T.inside[s];
+  }
+  return n;
+}
+
+// A call of more launches than this runs without graph capture.  A captured launch costs
+// about 2 us once and saves 0.2 us or less per replay (3x3 plan, 256 looped slices, 3329
+// launches: first call 15.1 ms eager, 22.3 captured, later ones 15.3 and 14.7; 6x6, 64
+// looped slices: 41.4 and 41.2), so that a graph of this size pays after ten calls of tens
+// of milliseconds, if at all, and one of 150K launches has ended in a host fault.
+constexpr int64_t kMaxGraphLaunches = int64_t(1) << 12;
 
 void check_bits(qx_plan *P, const char *bits, int64_t nb) {
   const int64_t nch = P->prog.num_chars;
@@ -1190,8 +1208,9 @@ void amplitudes(qx_plan *P, const char *bits, int64_t nb, int64_t s0, int64_t s1
   cb.bits = pin_bits ? P->pin : P->bits.p;
   auto enqueue = [&]() { enqueue_amplitudes(P, L, fused, s0, s1, nb, batch, cb, tuner.get(), true); };
   const int64_t nrows = (nb + batch - 1) / batch;
-  const int64_t launches = 2 + section_launches(L, 0) +
-                           (s1 - s0) * (section_launches(L, 1) + nrows * (section_launches(L, 2) + 2));
+  const int64_t launches =
+      section_launches(P, L, 0) +
+      (s1 - s0) * (section_launches(P, L, 1) + nrows * ((nout > 0) + section_launches(P, L, 2) + 1));
   P->last_launches = launches;
   if (P->opt_graph && !P->opt_profile && !tuner && launches <= kMaxGraphLaunches) {
     auto key = std::make_tuple(batch, nb, s0,
@@ -1795,13 +1814,19 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   }
   run_bwd(0);
   };
-  // forward launches plus at most two per backward step (a contraction and its add)
-  int64_t bwd[3] = {0, 0, 0};
-  for (int sec = 0; sec < 3; ++sec) bwd[sec] = 2 * (int64_t)V.bsteps[sec].size();
+  // launches of a pass over each section: its forward, zero fills and backward steps
+  int64_t pass[3];
+  for (int sec = 0; sec < 3; ++sec) {
+    pass[sec] = section_launches(P, L, sec) + (BT.nzero[sec] > 0);
+    for (size_t i = 0; i < V.bsteps[sec].size(); ++i) {
+      const qx::BwdStep &b = V.bsteps[sec][i];
+      const int gi = BT.first[sec][i];
+      if (b.level < 0) pass[sec] += step_launches(b.step) + !b.direct;
+      else pass[sec] += gi >= 0 && !BT.groups[gi].inside;
+    }
+  }
   const int64_t nrows = (nb + batch - 1) / batch;
-  const int64_t launches = 1 + section_launches(L, 0) + bwd[0] + 1 +
-                           nslices * (section_launches(L, 1) + bwd[1] + 1 +
-                                      nrows * (section_launches(L, 2) + bwd[2] + 3));
+  const int64_t launches = (ke > 0) + pass[0] + nslices * (pass[1] + nrows * ((nout > 0) + 1 + pass[2]));
   P->last_launches = launches;
   if (P->opt_graph && !P->opt_profile && launches <= kMaxGraphLaunches) {
     auto key = std::make_tuple(batch, nb, int64_t(norm ? -2 : -1), (int64_t)fused);

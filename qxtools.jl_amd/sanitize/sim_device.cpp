@@ -94,10 +94,11 @@ void submit(hipStream_t s, std::function<void()> f) {
   f();
 }
 
-void launch(void *stream, std::function<void()> check) {
-  submit((hipStream_t)stream, [check]() {
+// `kernels`: how many the launch function would launch
+void launch(void *stream, std::function<void()> check, int kernels = 1) {
+  submit((hipStream_t)stream, [check, kernels]() {
     check();
-    ++g_launches;
+    g_launches += kernels;
   });
 }
 
@@ -373,7 +374,7 @@ void launch_contract_bits(int prec, const void *A, const void *B, void *C, void 
     need(B, rb, "bits B");
     need(C, (long double)c_elems * es, "bits C");
     need(ws, rw, "bits K-split partials");
-  });
+  }, 1 + (a.ksplit > 1));
 }
 
 void launch_contract_reduce(int prec, const void *A, const void *B, void *C, void *ws, int64_t c_elems,
@@ -393,7 +394,7 @@ void launch_contract_gemm(int prec, const void *A, const void *B, void *C, void 
     need(B, rb, "gemm B");
     need(C, rc, "gemm C");
     need(ws, rw, "gemm K-split partials");
-  });
+  }, 1 + (g.ksplit > 1));
 }
 
 void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void *ws, const MfmaArgs &g, void *stream) {
@@ -419,7 +420,7 @@ void launch_contract_mfma(int prec, const void *A, const void *B, void *C, void 
     need(Y, ry, "matrix-core GEMM Y");
     need(C, (long double)g.c_elems * es, "matrix-core GEMM C");
     need(ws, g.ksplit > 1 ? (long double)g.c_elems * g.ksplit * es : 0, "matrix-core GEMM K-split partials");
-  });
+  }, 1 + (g.ksplit > 1));
 }
 
 void launch_contract_rows(int prec, const void *A, const void *B, void *C, const RowArgs &r, void *stream) {
@@ -479,7 +480,7 @@ void launch_fill_outputs(int prec, void *arena, const int64_t *d_out_off, int n_
       if (d_out_q[o] < 1 || d_out_q[o] > num_chars) violation("output qubit outside the bitstring");
       need((const char *)arena + d_out_off[o] * (int64_t)es, (long double)2 * batch * es, "output tensor");
     }
-  });
+  }, n_out > 0);
 }
 
 namespace {
@@ -622,7 +623,7 @@ void launch_zero_batch(void *base, const int64_t *d_ranges, int n, void *stream)
     need(d_ranges, (long double)n * 16, "zero ranges");
     for (int i = 0; i < n; ++i)
       need((char *)base + d_ranges[2 * i] * 16, (long double)d_ranges[2 * i + 1] * 16, "zero range");
-  });
+  }, n > 0);
 }
 
 void launch_contract_chain(int prec, const void *X0, void *Xm, void *ws, const ChainArgs &a,
@@ -678,7 +679,7 @@ void launch_contract_chain(int prec, const void *X0, void *Xm, void *ws, const C
     need(ws, packed * es, "chain packed gate blocks");
     need((const char *)ws + (size_t)a.tab_off * es, (long double)kChainTabInts * 4 * a.nsteps, "chain step tables");
     for (auto &p : s) need(p.first, p.second, "chain gate block");
-  });
+  }, 2 + (merge.ngroups > 0));
 }
 
 int64_t plain_gemm_units(int prec, const BlasArgs &b) {
@@ -700,7 +701,7 @@ void launch_plain_gemm(int prec, const void *X, const void *Y, void *C, void *ws
     need(Y, ry, "plain GEMM Y");
     need(C, rc, "plain GEMM C");
     need(ws, rw, "plain GEMM K-split partials");
-  });
+  }, 1 + (b.ksplit > 1));
 }
 
 void launch_gen_bits(char *bits, int64_t nb, int nch, uint64_t, int64_t, void *stream) {
@@ -726,7 +727,7 @@ void launch_reject(const double *amps, const char *cand, int64_t nb, int nch, ui
 
 void launch_zero(void *p, int64_t bytes, void *stream) {
   if (bytes % 16) throw Error(QX_ERR_ARGUMENT, "zero fill of a size not a multiple of 16 bytes");
-  launch(stream, [=]() { need(p, bytes, "zero fill"); });
+  launch(stream, [=]() { need(p, bytes, "zero fill"); }, bytes > 0);
 }
 
 }  // namespace qx
