@@ -93,7 +93,7 @@ qx_status qx_plan_set_tensor(qx_plan *plan, const char *key, const double *z, in
  * re-tuning the plan.  Returns after the copy has reached the device. */
 qx_status qx_plan_update_tensor(qx_plan *plan, const char *key, const double *z, int64_t nelem);
 
-/* The same for n data keys in one copy: `keys` are indices of qx_plan_key, `z` their
+/* The same for n data keys in one copy (several where keys between them are large): `keys` are indices of qx_plan_key, `z` their
  * values one key after the other, `nelem` complex values in all. */
 qx_status qx_plan_update_tensors(qx_plan *plan, const int64_t *keys, int64_t n, const double *z, int64_t nelem);
 

@@ -320,23 +320,30 @@ void put_data(qx_plan *P, size_t i, const double *z, size_t n) {
   }
 }
 
-// New values of n keys, packed in z: into the image, then one copy of the bytes they
-// span.  Lowered steps, descriptor tables and captured graphs address the buffer, not its
-// values, so all of them stay valid.  The copy is stream-ordered after earlier calls'
-// work and synchronous towards the caller.
+// New values of n keys, packed in z: into the image, then copies of the bytes they span,
+// keys at most kUpdateGap apart in one (a copy of its own takes as long as 64 KiB more).
+// Lowered steps, descriptor tables and captured graphs address the buffer, not its values,
+// so all of them stay valid.  The copies are stream-ordered after earlier calls' work and
+// synchronous towards the caller.
+constexpr size_t kUpdateGap = size_t(64) << 10;
 void update_data(qx_plan *P, const int64_t *keys, int64_t n, const double *z) {
-  size_t lo = P->image.size(), hi = 0;
+  std::vector<std::pair<size_t, size_t>> span;
   for (int64_t j = 0; j < n; ++j) {
     const size_t i = (size_t)keys[j], values = 2 * (size_t)P->prog.key_elems.at(P->prog.keys[i]);
     put_data(P, i, z, values);
     z += values;
-    lo = std::min(lo, P->data_off[i]);
-    hi = std::max(hi, P->data_off[i] + values / 2 * P->esize());
+    if (values) span.push_back({P->data_off[i], P->data_off[i] + values / 2 * P->esize()});
   }
-  if (lo >= hi) return;
+  if (span.empty()) return;
+  std::sort(span.begin(), span.end());
   hip_check(hipSetDevice(P->ctx->device), "hipSetDevice");
   hipStream_t s = P->ctx->stream;
-  hip_check(hipMemcpyAsync((char *)P->data.p + lo, P->image.data() + lo, hi - lo, hipMemcpyHostToDevice, s), "upload");
+  for (size_t j = 0; j < span.size();) {
+    const size_t lo = span[j].first;
+    size_t hi = span[j].second;
+    while (++j < span.size() && span[j].first <= hi + kUpdateGap) hi = std::max(hi, span[j].second);
+    hip_check(hipMemcpyAsync((char *)P->data.p + lo, P->image.data() + lo, hi - lo, hipMemcpyHostToDevice, s), "upload");
+  }
   hip_check(hipStreamSynchronize(s), "hipStreamSynchronize");
 }
 

@@ -53,6 +53,7 @@ std::map<uintptr_t, size_t> g_allocs;   // base -> bytes of every live device al
 std::map<uintptr_t, size_t> g_pinned;   // those of them that are pinned host memory
 double g_clock = 0;                     // simulated time of recorded events
 int64_t g_launches = 0;                 // kernel launches checked (eager or replayed)
+int64_t g_uploaded = 0;                 // bytes copied from host to device memory
 
 [[noreturn]] void violation(const std::string &msg) {
   std::fprintf(stderr, "SIM DEVICE VIOLATION: %s\n", msg.c_str());
@@ -189,6 +190,7 @@ hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKin
     if (kind == hipMemcpyDeviceToHost || kind == hipMemcpyDeviceToDevice) need(src, bytes, "copy source");
     if (kind == hipMemcpyHostToDevice && is_device(src) && !is_pinned(src)) violation("host-to-device copy from device memory");
     if (kind == hipMemcpyDeviceToHost && is_device(dst) && !is_pinned(dst)) violation("device-to-host copy into device memory");
+    if (kind == hipMemcpyHostToDevice) g_uploaded += (int64_t)bytes;
     if (bytes) std::memmove(dst, src, bytes);
   });
   return hipSuccess;
@@ -734,3 +736,5 @@ void launch_zero(void *p, int64_t bytes, void *stream) {
 
 // number of kernel launches checked so far (eager and graph replays)
 extern "C" int64_t qx_sim_launches(void) { return g_launches; }
+// bytes copied to device memory so far
+extern "C" int64_t qx_sim_uploaded(void) { return g_uploaded; }
