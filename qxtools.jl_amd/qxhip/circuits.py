@@ -76,6 +76,8 @@ def param_gate_tensors(name: str, angles, deriv: bool = False) -> np.ndarray:
         if deriv:
             out = out * np.array([-0.5j, 0.5j])
         return out
+    if name != "ry":
+        raise ValueError(f"gate {name} has no parameterised tensor")
     c = [math.cos(a / 2) for a in angles]
     s = [math.sin(a / 2) for a in angles]
     if deriv:

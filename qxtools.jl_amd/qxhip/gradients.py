@@ -60,6 +60,10 @@ class ParamCircuit:
             self._circ, self._angles = self._circ.with_params(self._angles), None
         return self._circ
 
+    @circ.setter
+    def circ(self, circ: Circuit) -> None:
+        self._circ, self._angles = circ, None
+
     @property
     def terms(self) -> list:
         """Chain-rule terms (param index, key, dT/dtheta in the key's array layout)."""
