@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 from qxhip import Executor, _native
+from test_gpu_kernels import plain_step
 
 
 def batched_gemm(nh, nm, nn, nk, seed=0):
@@ -75,3 +76,21 @@ def test_workgroups_of_several_units(nh, nm, nn, nk, units):
     ex.close()
     assert g["units_per_workgroup"] == units
     assert np.linalg.norm(got - ref) <= 2.4e-5 * np.linalg.norm(ref)
+
+
+# (H, M, N, K bits; operand orders) -> tile: a side of 128 for complex64 in four products, K >= 64,
+# from 1024 such tiles
+WIDE = [((10, 7, 6, 6), 0, [128, 64, 16]), ((10, 6, 7, 6), 3, [64, 128, 16]), ((9, 7, 7, 6), 5, [128, 64, 16]),
+        ((9, 7, 6, 6), 0, [64, 64, 16]), ((10, 7, 6, 5), 0, [64, 64, 16])]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,layout,tile", WIDE)
+def test_wide_tiles_are_the_ones_that_run(shape, layout, tile):
+    dsl, data, ref = plain_step(41 + layout, *shape, layout & 1, layout >> 1 & 1, layout >> 2)
+    ex = Executor(dsl, data, precision="c64_4m", batch=1, kernel=5)
+    got = np.asarray(ex.amplitudes([""])).reshape(-1)
+    (g,) = gemm_steps(ex.stats()["batches"][0]["steps"])
+    ex.close()
+    assert sorted(g["tile"]) == sorted(tile)          # (which operand gives the rows is the layout's)
+    assert np.linalg.norm(got - ref) <= 5e-6 * np.linalg.norm(ref)
