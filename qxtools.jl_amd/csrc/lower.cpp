@@ -2299,9 +2299,9 @@ VjpLowered lower_vjp(const Program &p, int64_t batch, int precision, uint64_t fu
 
   // Backward steps of sections 0 and 2 in dependency levels: a step reads the
   // cotangent written one level earlier.  Small ones whose operands have no
-  // slice-dependent offsets and that write a cotangent directly, or a temp added
-  // into a data key's gradient that no other step adds into, run batched per level
-  // (each with its own temp); the order is stable per level.
+  // slice-dependent offsets run batched per level and write their result themselves: a
+  // cotangent, or an add into a data key's gradient that no other step adds into or into a
+  // cotangent that no other of the level does.  The order is stable per level.
   std::vector<int> key_uses(p.keys.size(), 0);
   for (auto &sec : V.bsteps)
     for (auto &b : sec)
@@ -2309,14 +2309,15 @@ VjpLowered lower_vjp(const Program &p, int64_t batch, int precision, uint64_t fu
   int level_base = 0;
   for (int sec : {0, 2}) {
     auto &bv = V.bsteps[sec];
-    std::map<int, size_t> prod;   // node -> backward step writing its cotangent
-    for (size_t i = 0; i < bv.size(); ++i)
-      if (bv[i].direct) prod[bv[i].x] = i;
+    // level at which a node's cotangent is whole: after the step that writes it, or every
+    // step that adds into it through a view of the node
+    std::vector<int> whole(nn, 0);
     std::vector<int> lev(bv.size(), 0);
     int maxlev = 0;
     for (size_t i = 0; i < bv.size(); ++i) {
-      auto it = prod.find(bv[i].step.node);
-      lev[i] = it == prod.end() ? 0 : lev[it->second] + 1;
+      lev[i] = whole[bv[i].step.node];
+      const int to = bv[i].direct ? bv[i].x : bv[i].dest == Buf::Cot ? bv[i].dest_root : -1;
+      if (to >= 0) whole[to] = std::max(whole[to], lev[i] + 1);
       maxlev = std::max(maxlev, lev[i]);
     }
     auto no_slice_terms = [&](const BwdStep &b) {
