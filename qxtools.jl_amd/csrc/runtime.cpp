@@ -194,6 +194,7 @@ struct qx_plan {
     std::vector<char> inside;
     // a whole section's levels (plan option small_walk): table offset, levels (0: not)
     int walk_at[3] = {0, 0, 0}, walk_levels[3] = {0, 0, 0};
+    int64_t launches[2][3] = {{-1, -1, -1}, {-1, -1, -1}};   // section_launches, without and with the walk; -1: not counted
   };
   std::map<const qx::Lowered *, SmallTable> small;   // per lowering (forward or pullback)
   // batched slice-free backward levels of one pullback lowering
@@ -204,6 +205,7 @@ struct qx_plan {
     std::vector<int> first[3];              // per section and backward step: its level's group, or -1
     struct Group { int desc0, ndesc, run_at, run_levels, inside; };   // runs as in SmallTable
     std::vector<Group> groups;
+    int64_t launches[3] = {0, 0, 0};        // per section: of its zero fills and backward steps
   };
   std::map<const qx::VjpLowered *, BwdTable> bwd;
   // captured device work of qx_amplitudes per (batch, nb, slice_begin, slice_end)
@@ -871,6 +873,7 @@ void finish_tuning(qx_plan *P, qx::Lowered &L, Tuner &T) {
     L.ws_elems = std::max(L.ws_elems, L.steps[s].ws_elems);
   }
   L.tuned = true;
+  for (auto &of_walk : P->small.at(&L).launches) std::fill(of_walk, of_walk + 3, -1);
   P->drop_graphs();
 }
 
@@ -1003,10 +1006,12 @@ int step_launches(const qx::Step &st) {
 
 // Launches of one section of a lowered program per pass: its steps', one per level or run
 // of levels of small steps, or one for all of them (prepare_small has built the tables).
-int64_t section_launches(const qx_plan *P, const qx::Lowered &L, int sec) {
-  const qx_plan::SmallTable &T = P->small.at(&L);
+int64_t section_launches(qx_plan *P, const qx::Lowered &L, int sec) {
+  qx_plan::SmallTable &T = P->small.at(&L);
   const bool walk = walks(P, T, sec);
-  int64_t n = walk;
+  int64_t &n = T.launches[walk][sec];
+  if (n >= 0) return n;
+  n = walk;
   for (size_t s = 0; s < L.steps.size(); ++s) {
     if (L.steps[s].section != sec) continue;
     if (L.steps[s].level < 0) n += step_launches(L.steps[s]);
@@ -1754,6 +1759,15 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
         BT.zeros.reserve(zr.size() * 8);
         hip_check(hipMemcpy(BT.zeros.p, zr.data(), zr.size() * 8, hipMemcpyHostToDevice), "copy");
       }
+      for (int sec = 0; sec < 3; ++sec) {
+        int64_t &n = BT.launches[sec] = BT.nzero[sec] > 0;
+        for (size_t i = 0; i < V.bsteps[sec].size(); ++i) {
+          const qx::BwdStep &b = V.bsteps[sec][i];
+          const int gi = BT.first[sec][i];
+          if (b.level < 0) n += step_launches(b.step) + !b.direct;
+          else n += gi >= 0 && !BT.groups[gi].inside;
+        }
+      }
       BT.bases = bases;
       P->drop_graphs();
     }
@@ -1821,17 +1835,9 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
   }
   run_bwd(0);
   };
-  // launches of a pass over each section: its forward, zero fills and backward steps
+  // launches of a pass over each section
   int64_t pass[3];
-  for (int sec = 0; sec < 3; ++sec) {
-    pass[sec] = section_launches(P, L, sec) + (BT.nzero[sec] > 0);
-    for (size_t i = 0; i < V.bsteps[sec].size(); ++i) {
-      const qx::BwdStep &b = V.bsteps[sec][i];
-      const int gi = BT.first[sec][i];
-      if (b.level < 0) pass[sec] += step_launches(b.step) + !b.direct;
-      else pass[sec] += gi >= 0 && !BT.groups[gi].inside;
-    }
-  }
+  for (int sec = 0; sec < 3; ++sec) pass[sec] = section_launches(P, L, sec) + BT.launches[sec];
   const int64_t nrows = (nb + batch - 1) / batch;
   const int64_t launches = (ke > 0) + pass[0] + nslices * (pass[1] + nrows * ((nout > 0) + 1 + pass[2]));
   P->last_launches = launches;
