@@ -945,11 +945,12 @@ __global__ void k_accumulate(const typename Vec<T>::type *__restrict__ root, int
     double *a = acc + i * 4;
     double s0 = 0, s1 = 0, c0 = 0, c1 = 0;
     if (!first) s0 = a[0], s1 = a[1], c0 = a[2], c1 = a[3];
-#pragma unroll 4
-    for (int64_t sl = 0; sl < slices; ++sl) {
-      const auto v = root[relem_off[sl * relems + e] + beta * root_bstride];
+    auto v = root[relem_off[e] + beta * root_bstride];
+    for (int64_t sl = 1;; ++sl) {   // (most calls: one)
       neumaier(s0, c0, (double)v.x);
       neumaier(s1, c1, (double)v.y);
+      if (sl >= slices) break;
+      v = root[relem_off[sl * relems + e] + beta * root_bstride];
     }
     if (last) {
       out[i] = double2{s0 + c0, s1 + c1};
