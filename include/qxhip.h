@@ -106,9 +106,12 @@ qx_status qx_plan_update_tensors(qx_plan *plan, const int64_t *keys, int64_t n, 
  *                 and batches) once per (batch, nb, slice range) and replay it;
  *                 ignored while "profile" is on
  *   "profile"     1 = time every step with HIP events (qx_plan_stats)
- *   "fuse_slices" 1 (default) = when a call covers every slice, contract as many
- *                 slice variables inline as fit half the arena cap instead of
- *                 looping over them; 0 = always loop
+ *   "fuse_slices" 1 (default) = contract as many slice variables inline as fit half the
+ *                 arena cap instead of looping over them: summed in the contractions
+ *                 when a call covers every slice; for a part of the slices (complex128)
+ *                 those whose blocks of values the part consists of, each slice's result
+ *                 apart and added in the compensated sum as a looped one is; 0 = always
+ *                 loop.  Variables whose sum is not one contraction always loop
  *   "autotune"    1 = the next call of each lowering runs every candidate kernel of
  *                 every step (same results), times them with HIP events and keeps
  *                 the fastest per step for later calls; default 0
@@ -119,8 +122,9 @@ qx_status qx_plan_update_tensors(qx_plan *plan, const int64_t *keys, int64_t n, 
  *                 intermediates (default 0: fastest)
  *   "small_walk"  1 = a section whose batched small steps total at most 2^22
  *                 multiply-adds runs all their dependency levels in one launch of one
- *                 workgroup; 0 (default) = one launch per level (may be set at any time;
- *                 the walk is latency-bound and slower on the plans measured so far)
+ *                 workgroup; 0 (default) = one launch per level, or per run of levels of
+ *                 few items each (may be set at any time; a walk of wide levels leaves
+ *                 the other CUs idle and is slower on the plans measured so far)
  *   "kernel"      -1 (default) = heuristic kernel choice; 0 gather, 1 rows, 2-4
  *                 FP tile GEMMs, 5 / 7 matrix-core GEMM on any layout (result lanes along
  *                 C's fastest leg / along the other operand's), 6 reduce,
@@ -169,7 +173,7 @@ qx_status qx_amplitudes(qx_plan *plan, const char *bits, int64_t nb, int64_t sli
 /* qx_amplitudes that allocates no device memory, for callers that cannot allocate
  * (code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc).  No counterpart in the reference.  Same arguments, results and slice
- * handling as qx_amplitudes; it contracts in batches of the plan's "batch" option and
+ * handling as qx_amplitudes (a part of the slices always loops); it contracts in batches of the plan's "batch" option and
  * uses the plan's arena, workspace and tables as an earlier qx_amplitudes call of at
  * least that many bitstrings sized them (QX_ERR_STATE otherwise).  Its per-call device
  * buffers (FP64 accumulators, staged bitstrings, index tables and results: about

@@ -2773,14 +2773,6 @@ __global__ __launch_bounds__(kSmallRunThreads) void k_small_batch(const SmallDes
   small_levels<T>(d, off, n, nlevels, vars);
 }
 
-// Every level of a section in one workgroup (plan option small_walk).
-template <typename T>
-__global__ __launch_bounds__(kSmallRunThreads) void k_small_walk(const SmallDesc *__restrict__ d,
-                                                                 const int *__restrict__ off, int n, int nlevels,
-                                                                 SmallVars vars) {
-  small_levels<T>(d, off, n, nlevels, vars);
-}
-
 // ---------------------------------------------------------------------------
 // Output sampling on the device.  Counter-based Philox4x64-10 (Salmon, Moraes,
 // Dror, Shaw, "Parallel random numbers: as easy as 1, 2, 3", SC 2011): candidate j
@@ -3208,16 +3200,13 @@ void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVar
 }
 
 void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
-                      bool walk, void *stream) {
+                      void *stream) {
   if (nlevels <= 0) return;
   hipStream_t s = (hipStream_t)stream;
-#define QX_RUN(K) hipLaunchKernelGGL(K, dim3(1), dim3(kSmallRunThreads), 0, s, d_desc, d_level_off, 0, nlevels, vars)
-  if (prec == QX_C128) {
-    if (walk) QX_RUN(k_small_walk<double>); else QX_RUN(k_small_batch<double>);
-  } else {
-    if (walk) QX_RUN(k_small_walk<float>); else QX_RUN(k_small_batch<float>);
-  }
-#undef QX_RUN
+  if (prec == QX_C128)
+    hipLaunchKernelGGL(k_small_batch<double>, dim3(1), dim3(kSmallRunThreads), 0, s, d_desc, d_level_off, 0, nlevels, vars);
+  else
+    hipLaunchKernelGGL(k_small_batch<float>, dim3(1), dim3(kSmallRunThreads), 0, s, d_desc, d_level_off, 0, nlevels, vars);
   check_launch("small_run");
 }
 

@@ -504,10 +504,9 @@ void launch_root_cot_norm(int prec, void *dst, const void *val, int64_t dep, int
 // n independent items (one level), a wave each.
 void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVars &vars, void *stream);
 // Levels [0, nlevels) of items in one workgroup: level L is the descriptors
-// [d_level_off[L], d_level_off[L + 1]), run after every earlier level.  `walk`: the
-// instance named k_small_walk (a whole section, plan option small_walk).
+// [d_level_off[L], d_level_off[L + 1]), run after every earlier level.
 void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
-                      bool walk, void *stream);
+                      void *stream);
 // bf16 split of n complex64 values: out holds four planar n-element bf16 arrays
 // (re hi, re lo, im hi, im lo); hi = x rounded to bf16 (nearest, ties to even),
 // lo = (x - hi) rounded likewise.

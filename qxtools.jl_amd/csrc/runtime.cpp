@@ -157,7 +157,7 @@ struct qx_plan {
   int64_t opt_kernel = -1;                  // >= 0: force that kernel wherever it can run
   int64_t opt_chains = 1;                   // fold runs of gate-block steps into chain passes
   int64_t opt_batch_last = 0;               // batched leg slowest in bitstring-dependent values
-  int64_t opt_small_walk = 0;               // small sections' levels in one launch (k_small_walk)
+  int64_t opt_small_walk = 0;               // small sections' levels in one launch
   int64_t opt_chain_variant = -1;           // >= 0: chain passes' 16-value path (bits 0-1),
                                             // swizzled tiles (bit 2), barriers (bit 3); tests
   bool finalized = false;
@@ -747,7 +747,7 @@ void run_small_walk(qx_plan *P, const qx::Lowered &L, size_t s, int sec, const s
     hip_check(hipEventRecord(P->events[2 * ev], stream), "hipEventRecord");
   }
   qx::launch_small_run(P->prec, (const qx::SmallDesc *)T.desc.p, (const int *)T.walk.p + T.walk_at[sec],
-                       T.walk_levels[sec], small_vars(varval), true, stream);
+                       T.walk_levels[sec], small_vars(varval), stream);
   if (timed) hip_check(hipEventRecord(P->events[2 * ev + 1], stream), "hipEventRecord");
 }
 
@@ -770,7 +770,7 @@ void run_small_level(qx_plan *P, const qx::Lowered &L, size_t s, const std::vect
   }
   if (T.run_levels[s] > 0)
     qx::launch_small_run(P->prec, (const qx::SmallDesc *)T.desc.p, (const int *)T.walk.p + T.run_at[s],
-                         T.run_levels[s], small_vars(varval), false, stream);
+                         T.run_levels[s], small_vars(varval), stream);
   else
     qx::launch_small_batch(P->prec, (const qx::SmallDesc *)T.desc.p + T.index[s], T.count[s], small_vars(varval), stream);
   if (timed) hip_check(hipEventRecord(P->events[2 * ev + 1], stream), "hipEventRecord");
@@ -1784,8 +1784,7 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
         const auto &g = BT.groups[gi];
         const qx::SmallDesc *d = (const qx::SmallDesc *)BT.desc.p;
         if (g.run_levels > 0)
-          qx::launch_small_run(P->prec, d, (const int *)BT.walk.p + g.run_at, g.run_levels, qx::SmallVars(), false,
-                               stream);
+          qx::launch_small_run(P->prec, d, (const int *)BT.walk.p + g.run_at, g.run_levels, qx::SmallVars(), stream);
         else
           qx::launch_small_batch(P->prec, d + g.desc0, g.ndesc, qx::SmallVars(), stream);
         continue;
@@ -1896,7 +1895,7 @@ std::string stats_json(const qx_plan *P) {
       double bytes = (double)P->esize() * st.H * (st.M * st.K + st.K * st.N + st.M * st.N);
       if (st.kern == qx::Kern::Chain || st.kern == qx::Kern::Outer) flops = st.chain_flops, bytes = (double)P->esize() * st.chain_elems;
       std::string variant = kern_variant(st);
-      if (st.level >= 0 && P->opt_small_walk) {   // levels walked by one workgroup
+      if (st.level >= 0 && P->opt_small_walk) {   // k_small_batch over all levels, in one workgroup
         auto it = P->small.find(&L);
         if (it != P->small.end() && it->second.walk_levels[st.section] > 0) variant = "k_small_walk";
       }

@@ -585,7 +585,7 @@ void launch_small_batch(int prec, const SmallDesc *d_desc, int n, const SmallVar
 }
 
 void launch_small_run(int prec, const SmallDesc *d_desc, const int *d_level_off, int nlevels, const SmallVars &vars,
-                      bool, void *stream) {
+                      void *stream) {
   launch(stream, [=]() {
     need(d_level_off, (long double)(nlevels + 1) * 4, "level table");
     for (int L = 0; L < nlevels; ++L)
