@@ -943,6 +943,12 @@ static void fused_shapes(const Program &p, uint64_t fused, std::vector<std::vect
 
 uint64_t inline_vars(const Program &p) {
   uint64_t mask = 0;
+  std::vector<char> used(p.nodes.size(), 0);   // tensors that the saved one depends on
+  used[p.save] = 1;
+  for (size_t i = p.nodes.size(); i-- > 0;)
+    if (used[i])
+      for (int in : {p.nodes[i].ia, p.nodes[i].ib})
+        if (in >= 0) used[in] = 1;
   auto in = [](const std::vector<int> &labels, int l) { return std::find(labels.begin(), labels.end(), l) != labels.end(); };
   for (size_t j = 0; j < p.vars.size() && j < 63; ++j) {
     std::vector<int> leg(p.nodes.size(), -1);   // each node's leg of this variable
@@ -965,7 +971,7 @@ uint64_t inline_vars(const Program &p) {
         else ok = leg[n.ia] >= 0 ? !in(n.blab, a) : !in(n.alab, b);
         const int l = leg[n.ia] >= 0 ? a : b;
         if (in(n.clab, l)) leg[i] = (int)(std::find(n.clab.begin(), n.clab.end(), l) - n.clab.begin());
-        else ++sums;
+        else sums += used[i];
       } else if (n.op == Op::Save) {
         ok = leg[n.ia] < 0;
       }

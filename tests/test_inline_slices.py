@@ -67,8 +67,18 @@ ncon E 2,5,6 D 2,3 B 5,3,6
 ncon F 2,5,7 E 2,5,6 C 6,7
 save output F
 """,
+    "unused_sum": HEAD + """load G data_5 2,2
+load H data_6 2
+view G1 G v1 1 2
+view H1 H v1 1 2
+ncon I 2 G1 1,2 H1 1
+ncon D 2,3 O1 1 A 1,2,3
+ncon E 2,5,6 D 2,3 B 5,3,6
+ncon F 2,5,7 E 2,5,6 C 6,7
+save output F
+""",
 }
-INLINE = {"one_bond": 1, "two_bonds": 0, "two_apart": 0, "saved_leg": 2, "unsummed": 0}
+INLINE = {"one_bond": 1, "two_bonds": 0, "two_apart": 0, "saved_leg": 2, "unsummed": 0, "unused_sum": 0}
 
 
 def data(dsl, seed=3):
