@@ -1020,11 +1020,11 @@ int64_t section_launches(qx_plan *P, const qx::Lowered &L, int sec) {
   return n;
 }
 
-// A call of more launches than this runs without graph capture.  A captured launch costs
-// about 2 us once and saves 0.2 us or less per replay (3x3 plan, 256 looped slices, 3329
-// launches: first call 15.1 ms eager, 22.3 captured, later ones 15.3 and 14.7; 6x6, 64
-// looped slices: 41.4 and 41.2), so that a graph of this size pays after ten calls of tens
-// of milliseconds, if at all, and one of 150K launches has ended in a host fault.
+// A call of more launches than this runs without graph capture.  A captured launch costs 2
+// to 5 us once and saves 0.2 us or less per replay: first and later calls in ms, 3x3 plan,
+// 256 looped slices, 3329 launches: 15.1 and 15.3 eager, 22.3 and 14.7 captured; 6x6, 64
+// looped slices, 7940 launches: 132 and 126.5, 163 and 126.3; 21124: 323 and 322.4, 428 and
+// 321.7.  One of 150K launches has ended in a host fault.
 constexpr int64_t kMaxGraphLaunches = int64_t(1) << 12;
 
 void check_bits(qx_plan *P, const char *bits, int64_t nb) {
