@@ -30,7 +30,19 @@ def asan_runtime() -> str:
                           check=True).stdout.strip()
 
 
+def _inputs():
+    """Every file the library is built from, this one (the flags) among them."""
+    yield from SOURCES
+    yield os.path.abspath(__file__)
+    for top in (os.path.join(HERE, "include"), os.path.join(PKG, "csrc"), os.path.join(os.path.dirname(PKG), "include")):
+        for folder, _, names in os.walk(top):
+            yield from (os.path.join(folder, n) for n in names if n.endswith((".h", ".hpp")))
+
+
 def build() -> str:
+    """Compile, unless the library is newer than all it is built from."""
+    if os.path.exists(OUT) and os.path.getmtime(OUT) > max(map(os.path.getmtime, _inputs())):
+        return OUT
     os.makedirs(os.path.dirname(OUT), exist_ok=True)
     cmd = ["g++", *FLAGS, f"-I{os.path.join(HERE, 'include')}", *SOURCES, "-o", OUT + ".tmp"]
     r = subprocess.run(cmd, capture_output=True, text=True)
