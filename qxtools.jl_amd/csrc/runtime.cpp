@@ -822,18 +822,19 @@ struct Tuner {
 };
 
 void tune_step(qx_plan *P, const qx::Lowered &L, size_t s, const std::vector<int64_t> &varval, Tuner &T) {
-  const qx::Step &st = L.steps[s];
-  void *A = value_ptr(P, L.values[st.in_a], varval);
-  void *B = value_ptr(P, L.values[st.in_b], varval);
-  void *C = value_ptr(P, L.values[st.node], varval);
+  // (a candidate may exchange the operands, so each takes its own pointers)
+  auto run = [&](const qx::Step &c) {
+    launch_step(P, L, c, value_ptr(P, L.values[c.in_a], varval), value_ptr(P, L.values[c.in_b], varval),
+                value_ptr(P, L.values[c.node], varval), varval);
+  };
   const auto &cs = T.cands[s];
   if (cs.size() < 2 || T.seen[s] >= Tuner::kTimedLaunches) {
-    launch_step(P, L, st, A, B, C, varval);
+    run(L.steps[s]);
     return;
   }
   hipStream_t stream = P->ctx->stream;
   if (T.seen[s] == 0)   // first launch of every candidate untimed: code loading, cold caches
-    for (auto &c : cs) launch_step(P, L, c, A, B, C, varval);
+    for (auto &c : cs) run(c);
   ++T.seen[s];
   for (size_t c = 0; c < cs.size(); ++c) {
     size_t ev = T.rec.size();
@@ -844,7 +845,7 @@ void tune_step(qx_plan *P, const qx::Lowered &L, size_t s, const std::vector<int
     }
     T.rec.push_back({(int)s, (int)c, (int)ev});
     hip_check(hipEventRecord(P->tune_events[2 * ev], stream), "hipEventRecord");
-    launch_step(P, L, cs[c], A, B, C, varval);
+    run(cs[c]);
     hip_check(hipEventRecord(P->tune_events[2 * ev + 1], stream), "hipEventRecord");
   }
 }
