@@ -1683,6 +1683,7 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
     A = xa ? value_ptr(P, cv, varval, bs) : value_ptr(P, L.values[cn.ia], varval, bs);
     B = xa ? value_ptr(P, L.values[cn.ib], varval, bs) : value_ptr(P, cv, varval, bs);
     C = b.direct ? value_ptr(P, V.cot[b.x], varval, bs) : (void *)bs.temp;
+    if (b.step.swapped) std::swap(A, B);   // (a forced row kernel over the other side)
   };
   // descriptor tables of the batched backward levels (sections 0 and 2; their
   // operands have no slice-dependent offsets)
