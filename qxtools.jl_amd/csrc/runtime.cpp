@@ -194,7 +194,7 @@ struct qx_plan {
     std::vector<char> inside;
     // a whole section's levels (plan option small_walk): table offset, levels (0: not)
     int walk_at[3] = {0, 0, 0}, walk_levels[3] = {0, 0, 0};
-    int64_t launches[2][3] = {{-1, -1, -1}, {-1, -1, -1}};   // section_launches, without and with the walk; -1: not counted
+    int64_t launches[2][3] = {};            // kernels of a pass over each section, without and with the walk
   };
   std::map<const qx::Lowered *, SmallTable> small;   // per lowering (forward or pullback)
   // batched slice-free backward levels of one pullback lowering
@@ -642,6 +642,22 @@ qx::SmallVars small_vars(const std::vector<int64_t> &varval) {
   return v;
 }
 
+// Kernels that launch_step launches for a step.
+int step_launches(const qx::Step &st) {
+  switch (st.kern) {
+    case qx::Kern::Blas: {
+      const qx::BlasArgs &b = st.blas;
+      return (b.ttgt ? 3 : 0) + (b.own ? 1 + (b.ksplit > 1) : b.split ? 15 : 1);
+    }
+    case qx::Kern::Chain: return 2 + !st.chain_merge.empty();
+    case qx::Kern::Gemm: return 1 + ((st.gemm.tile == 3 ? st.mfma->ksplit : st.gemm.ksplit) > 1);
+    case qx::Kern::Outer:
+    case qx::Kern::Radix:
+    case qx::Kern::Rows: return 1;
+    default: return 1 + (st.bits.ksplit > 1);
+  }
+}
+
 // Build and upload the descriptor table of L's batched small steps (operand addresses at
 // the first slice; an item adds its slice's terms) and the level tables of its runs.
 void prepare_small(qx_plan *P, const qx::Lowered &L, const Bases &bs) {
@@ -657,10 +673,12 @@ void prepare_small(qx_plan *P, const qx::Lowered &L, const Bases &bs) {
   const std::vector<int64_t> zero(P->prog.vars.size(), 0);
   std::vector<std::array<int, 3>> lv;   // levels and other launches, in order
   std::vector<int> at;                  // their first steps
+  for (auto &of_walk : T.launches) std::fill(of_walk, of_walk + 3, 0);
   int first = -1;
   for (size_t s = 0; s < ns; ++s) {
     const qx::Step &st = L.steps[s];
     if (st.level < 0) {
+      for (auto &of_walk : T.launches) of_walk[st.section] += step_launches(st);
       lv.push_back({-1, 0, st.section});
       at.push_back((int)s);
       first = -1;
@@ -688,6 +706,7 @@ void prepare_small(qx_plan *P, const qx::Lowered &L, const Bases &bs) {
     T.run_at[at[g]] = runs[g].at;
     T.run_levels[at[g]] = runs[g].levels;
     T.inside[at[g]] = runs[g].inside;
+    T.launches[0][lv[g][2]] += lv[g][0] >= 0 && !runs[g].inside;
   }
   // whole sections (plan option small_walk): levels at its front of at most 2^22
   // multiply-adds and 2^14 items in all
@@ -715,6 +734,7 @@ void prepare_small(qx_plan *P, const qx::Lowered &L, const Bases &bs) {
     if (front && !later && offs.size() >= 2 && macs <= double(1 << 22)) {
       walk.insert(walk.end(), offs.begin(), offs.end());
       T.walk_levels[sec] = (int)offs.size() - 1;
+      T.launches[1][sec] += 1;
     }
   }
   if (!walk.empty()) {
@@ -870,11 +890,12 @@ void finish_tuning(qx_plan *P, qx::Lowered &L, Tuner &T) {
       os << (c ? "," : "") << "\"" << cand_label(T.cands[s][c]) << "\":" << T.ms[s][c] / T.seen[s];
     }
     L.tune_log[s] = os.str();
+    for (auto &of_walk : P->small.at(&L).launches)
+      of_walk[L.steps[s].section] += step_launches(T.cands[s][best]) - step_launches(L.steps[s]);
     L.steps[s] = T.cands[s][best];
     L.ws_elems = std::max(L.ws_elems, L.steps[s].ws_elems);
   }
   L.tuned = true;
-  for (auto &of_walk : P->small.at(&L).launches) std::fill(of_walk, of_walk + 3, -1);
   P->drop_graphs();
 }
 
@@ -989,36 +1010,10 @@ void slice_values(const qx_plan *P, uint64_t fused, int64_t sl, std::vector<int6
   }
 }
 
-// Kernels that launch_step launches for a step.
-int step_launches(const qx::Step &st) {
-  switch (st.kern) {
-    case qx::Kern::Blas: {
-      const qx::BlasArgs &b = st.blas;
-      return (b.ttgt ? 3 : 0) + (b.own ? 1 + (b.ksplit > 1) : b.split ? 15 : 1);
-    }
-    case qx::Kern::Chain: return 2 + !st.chain_merge.empty();
-    case qx::Kern::Gemm: return 1 + ((st.gemm.tile == 3 ? st.mfma->ksplit : st.gemm.ksplit) > 1);
-    case qx::Kern::Outer:
-    case qx::Kern::Radix:
-    case qx::Kern::Rows: return 1;
-    default: return 1 + (st.bits.ksplit > 1);
-  }
-}
-
-// Launches of one section of a lowered program per pass: its steps', one per level or run
-// of levels of small steps, or one for all of them (prepare_small has built the tables).
-int64_t section_launches(qx_plan *P, const qx::Lowered &L, int sec) {
-  qx_plan::SmallTable &T = P->small.at(&L);
-  const bool walk = walks(P, T, sec);
-  int64_t &n = T.launches[walk][sec];
-  if (n >= 0) return n;
-  n = walk;
-  for (size_t s = 0; s < L.steps.size(); ++s) {
-    if (L.steps[s].section != sec) continue;
-    if (L.steps[s].level < 0) n += step_launches(L.steps[s]);
-    else n += !walk && T.count[s] > 0 && !T.inside[s];
-  }
-  return n;
+// Launches of one section of a lowered program per pass (prepare_small has counted them).
+int64_t section_launches(const qx_plan *P, const qx::Lowered &L, int sec) {
+  const qx_plan::SmallTable &T = P->small.at(&L);
+  return T.launches[walks(P, T, sec)][sec];
 }
 
 // A call of more launches than this runs without graph capture.  A captured launch costs 2
@@ -1697,12 +1692,14 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
       for (int sec = 0; sec < 3; ++sec) {
         const auto &bv = V.bsteps[sec];
         BT.first[sec].assign(bv.size(), -1);
+        BT.launches[sec] = !V.zero_at[sec].empty();
         std::vector<std::array<int, 3>> lv;   // the section's levels and other launches
         std::vector<int> group;               // their groups (-1: another launch)
         int cur_level = -1;
         for (size_t i = 0; i < bv.size(); ++i) {
           const qx::BwdStep &b = bv[i];
           if (b.level < 0) {
+            BT.launches[sec] += step_launches(b.step) + !b.direct;
             lv.push_back({-1, 0, sec});
             group.push_back(-1);
             cur_level = -1;
@@ -1737,6 +1734,7 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
           if (group[k] >= 0) {
             auto &g = BT.groups[group[k]];
             g.run_at = runs[k].at, g.run_levels = runs[k].levels, g.inside = runs[k].inside;
+            BT.launches[sec] += !g.inside;
           }
       }
       if (!d.empty()) {
@@ -1760,15 +1758,6 @@ void vjp(qx_plan *P, const char *bits, int64_t nb, const double *amp_cot, double
       if (!zr.empty()) {
         BT.zeros.reserve(zr.size() * 8);
         hip_check(hipMemcpy(BT.zeros.p, zr.data(), zr.size() * 8, hipMemcpyHostToDevice), "copy");
-      }
-      for (int sec = 0; sec < 3; ++sec) {
-        int64_t &n = BT.launches[sec] = BT.nzero[sec] > 0;
-        for (size_t i = 0; i < V.bsteps[sec].size(); ++i) {
-          const qx::BwdStep &b = V.bsteps[sec][i];
-          const int gi = BT.first[sec][i];
-          if (b.level < 0) n += step_launches(b.step) + !b.direct;
-          else n += gi >= 0 && !BT.groups[gi].inside;
-        }
       }
       BT.bases = bases;
       P->drop_graphs();
